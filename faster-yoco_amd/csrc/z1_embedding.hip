@@ -12,10 +12,10 @@
 //      while the stream is being captured into a HIP graph, rocPRIM's merge sort, which clears nothing with
 //      memsets (the radix sort does; both are stable, so the order is the same: 0.136 vs 0.142 ms per call);
 //   3. row_lo[t] = start of id t's run in the sorted keys (one binary search per t, all in parallel);
-//   4. one wave per output row t writes the row's sums -- or zeros -- exactly once, 8 bf16 columns per lane, with
-//      nontemporal stores (aten zero-fills the whole table and then scatters into it; here every row of the table
-//      is written once), for ids with at most kHeavyRows occurrences; the others are listed, with a slot range
-//      for their runs, for
+//   4. one wave per output row t writes the row's sums -- or zeros -- exactly once, 8 bf16 columns per lane and
+//      group, with nontemporal stores (aten zero-fills the whole table and then scatters into it; here every row of
+//      the table is written once), for ids with at most kHeavyRows occurrences; the others are listed, with a slot
+//      range for their runs, for
 //   5. emb_heavy_parts_kernel, which forms every run partial of every heavy id in parallel over the whole chip
 //      into an fp32 workspace, and
 //   6. emb_heavy_chain_kernel, which adds each heavy id's partials in run order per column.  Token frequencies in
@@ -113,23 +113,119 @@ __device__ __forceinline__ uint16_t finish(float acc, float scale, int scale_mod
     return o;
 }
 
-__device__ __forceinline__ void nt_store(u4* p, u4 x) {
-    __builtin_nontemporal_store(x, (__attribute__((address_space(1))) u4*)p);
+// Rows start wherever t * D puts them: the wide accesses below assume 2-byte alignment only (gfx950 loads and stores 16
+// bytes at any address; an odd D costs the lines that straddle).
+typedef u4 u4_any __attribute__((aligned(2)));
+
+__device__ __forceinline__ u4 load8(const uint16_t* p) {
+    return *(const __attribute__((address_space(1))) u4_any*)p;
+}
+__device__ __forceinline__ void nt_store8(uint16_t* p, u4 x) {
+    __builtin_nontemporal_store((u4_any)x, (__attribute__((address_space(1))) u4_any*)p);
+}
+
+// Adds a finished partial to the row's sum: aten's sort path adds fp32 partials; its few-indices kernel rounds the
+// partial to bf16 and the row after the add.
+template <bool FEW>
+__device__ __forceinline__ float add_part(float acc, float part) {
+    return FEW ? bf16f(bf16r(acc + bf16f(bf16r(part)))) : acc + part;
+}
+
+// Whether occurrence j of a row whose occurrences start at lo begins another partial (j > lo): every 10th occurrence,
+// or, for few indices, where the next chunk of 16 indices begins.
+template <bool FEW>
+__device__ __forceinline__ bool new_part(const int32_t* __restrict__ spos, int64_t lo, int64_t j) {
+    return FEW ? spos[j] / kFewRowsChunk != spos[j - 1] / kFewRowsChunk : (j - lo) % kRowsPerPartial == 0;
+}
+
+// A row with one occurrence: all G of a lane's column groups (gi, gi + 64, ... below ng, 8 columns each) loaded at once
+// -- the gradient row comes from HBM, so the wave waits for memory once a row instead of once a group -- and rounded.
+// With this and sum_row below, 16,384 rows of 3072 into a 100,288-row table, gradients not in a cache: 163 us a call
+// against 205 us with each group loaded, summed and stored before the next (Zipf ids 205 against 231 us).
+template <int G>
+__device__ __forceinline__ void copy_row(const uint16_t* __restrict__ row, int64_t gi, int64_t ng, float scale,
+                                         int scale_mode, uint16_t* __restrict__ orow) {
+    u4 x[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+        x[g] = u4{0u, 0u, 0u, 0u};
+        if (gi + g * kEmbThreads < ng) x[g] = load8(row + (gi + g * kEmbThreads) * 8);
+    }
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+        u4 o;
+#pragma unroll
+        for (int k = 0; k < 4; ++k)       // 0 + x: the sum of one element (-0 gives +0)
+            o[k] = (uint32_t)finish(0.0f + grad_elem((uint16_t)x[g][k], scale, scale_mode), scale, scale_mode) |
+                   ((uint32_t)finish(0.0f + grad_elem((uint16_t)(x[g][k] >> 16), scale, scale_mode), scale, scale_mode)
+                    << 16);
+        if (gi + g * kEmbThreads < ng) nt_store8(orow + (gi + g * kEmbThreads) * 8, o);
+    }
+}
+
+// One row's sum over its occurrences [lo, hi) for G column groups of a lane, as in copy_row: all G loads of an
+// occurrence are in flight together, the next occurrence's as well.
+template <bool FEW, int G>
+__device__ __forceinline__ void sum_row(const uint16_t* __restrict__ grad, int64_t D, const int32_t* __restrict__ spos,
+                                        int64_t lo, int64_t hi, int64_t gi, int64_t ng, float scale, int scale_mode,
+                                        uint16_t* __restrict__ orow) {
+    u4 x[G], y[G];
+    float acc[G][8], part[G][8];
+    auto load = [&](u4* d, int64_t j) {
+        const uint16_t* row = grad + (int64_t)spos[j] * D;
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+            if (gi + g * kEmbThreads < ng) d[g] = load8(row + (gi + g * kEmbThreads) * 8);
+    };
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+        x[g] = y[g] = u4{0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int k = 0; k < 8; ++k) acc[g][k] = part[g][k] = 0.0f;
+    }
+    load(x, lo);
+    for (int64_t j = lo; j < hi; ++j) {
+        if (j + 1 < hi) load(y, j + 1);
+        if (j > lo && new_part<FEW>(spos, lo, j)) {
+#pragma unroll
+            for (int g = 0; g < G; ++g)
+#pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    acc[g][k] = add_part<FEW>(acc[g][k], part[g][k]);
+                    part[g][k] = 0.0f;
+                }
+        }
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+                part[g][k] = part[g][k] + grad_elem((uint16_t)(x[g][k >> 1] >> ((k & 1) * 16)), scale, scale_mode);
+            x[g] = y[g];
+        }
+    }
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+        u4 o;
+#pragma unroll
+        for (int k = 0; k < 8; k += 2)
+            o[k >> 1] = (uint32_t)finish(add_part<FEW>(acc[g][k], part[g][k]), scale, scale_mode) |
+                        ((uint32_t)finish(add_part<FEW>(acc[g][k + 1], part[g][k + 1]), scale, scale_mode) << 16);
+        if (gi + g * kEmbThreads < ng) nt_store8(orow + (gi + g * kEmbThreads) * 8, o);
+    }
 }
 
 // One wave per output row t (light tokens: at most kHeavyRows occurrences, and empty or padding rows): the row's
-// sums -- or zeros -- written once, 8 bf16 columns per lane when vec (D % 8 == 0, 16-byte aligned tables).  Each
-// run of up to kRowsPerPartial occurrences has its loads issued together, then is summed in order.  A token with
-// more occurrences is appended, with the first of its nrun run slots (from counts[1]), to the list of tokens of at
-// most kWaveChainRuns runs (heavy_list / heavy_base, count counts[0]) or to that of longer ones (long_list /
-// long_base, counts[2]); run_start[slot] = the sorted position of the run's first row.  Its row is left to the heavy
-// passes.  The atomics only decide where a token's partials are kept, not how they are summed.
-template <bool FEW>
+// sums -- or zeros -- written once, G groups of 8 bf16 columns per lane and step, the last D % 8 columns one per lane.
+// A token with more occurrences is appended, with the first of its nrun run slots (from counts[1]), to the list of
+// tokens of at most kWaveChainRuns runs (heavy_list / heavy_base, count counts[0]) or to that of longer ones
+// (long_list / long_base, counts[2]); run_start[slot] = the sorted position of the run's first row.  Its row is left to
+// the heavy passes.  The atomics only decide where a token's partials are kept, not how they are summed.
+template <bool FEW, int G>
 __global__ __launch_bounds__(kEmbThreads) void emb_rows_kernel(const uint16_t* __restrict__ grad, int64_t D,
                                                                const int32_t* __restrict__ spos,
                                                                const int32_t* __restrict__ row_lo,
                                                                int64_t padding_idx, float scale, int scale_mode,
-                                                               int vec, uint16_t* __restrict__ out,
+                                                               uint16_t* __restrict__ out,
                                                                int* __restrict__ counts,
                                                                int32_t* __restrict__ heavy_list,
                                                                int32_t* __restrict__ heavy_base,
@@ -148,7 +244,6 @@ __global__ __launch_bounds__(kEmbThreads) void emb_rows_kernel(const uint16_t* _
     uint16_t* orow = out + t * D;
     const int64_t lo = row_lo[t], hi = row_lo[t + 1];
     const bool empty = lo == hi || t == padding_idx;
-    constexpr int chunk = kFewRowsChunk;
     if (!FEW && !empty && hi - lo > kHeavyRows) {
         const int nrun = (int)((hi - lo + kRowsPerPartial - 1) / kRowsPerPartial);
         int base = 0;
@@ -163,107 +258,33 @@ __global__ __launch_bounds__(kEmbThreads) void emb_rows_kernel(const uint16_t* _
         for (int k = lane; k < nrun; k += kEmbThreads) run_start[base + k] = (int32_t)(lo + (int64_t)k * kRowsPerPartial);
         return;
     }
-    if (vec) {
-        const int64_t ng = D / 8;
-        for (int64_t gi = lane; gi < ng; gi += kEmbThreads) {
-            u4 o = u4{0u, 0u, 0u, 0u};
-            if constexpr (FEW) {
-              if (!empty) {
-                // aten's few-indices order: the id's occurrences grouped by index chunk (positions ascend), each
-                // group's fp32 sum rounded to bf16 and added to the bf16 row
-                float acc[8];
-#pragma unroll
-                for (int k = 0; k < 8; ++k) acc[k] = 0.0f;
-                for (int64_t j0 = lo; j0 < hi;) {
-                    const int32_t cid = spos[j0] / chunk;
-                    int cnt = 1;
-                    while (cnt < kFewRowsChunk && j0 + cnt < hi && spos[j0 + cnt] / chunk == cid) ++cnt;
-                    u4 x[kFewRowsChunk];
-#pragma unroll
-                    for (int u = 0; u < kFewRowsChunk; ++u)
-                        if (u < cnt) x[u] = reinterpret_cast<const u4*>(grad + (int64_t)spos[j0 + u] * D)[gi];
-                    float part[8];
-#pragma unroll
-                    for (int k = 0; k < 8; ++k) part[k] = 0.0f;
-#pragma unroll
-                    for (int u = 0; u < kFewRowsChunk; ++u) {
-                        if (u < cnt) {
-#pragma unroll
-                            for (int k = 0; k < 8; ++k)
-                                part[k] = part[k] + grad_elem((uint16_t)(x[u][k >> 1] >> ((k & 1) * 16)), scale,
-                                                              scale_mode);
-                        }
-                    }
-#pragma unroll
-                    for (int k = 0; k < 8; ++k) acc[k] = bf16f(bf16r(acc[k] + bf16f(bf16r(part[k]))));
-                    j0 += cnt;
-                }
-#pragma unroll
-                for (int k = 0; k < 8; k += 2)
-                    o[k >> 1] = (uint32_t)finish(acc[k], scale, scale_mode) |
-                                ((uint32_t)finish(acc[k + 1], scale, scale_mode) << 16);
-              }
-            } else if (!empty) {
-                float acc[8];
-#pragma unroll
-                for (int k = 0; k < 8; ++k) acc[k] = 0.0f;
-                for (int64_t j0 = lo; j0 < hi; j0 += kRowsPerPartial) {
-                    const int cnt = (int)(j0 + kRowsPerPartial < hi ? kRowsPerPartial : hi - j0);
-                    u4 x[kRowsPerPartial];
-#pragma unroll
-                    for (int u = 0; u < kRowsPerPartial; ++u)
-                        if (u < cnt) x[u] = reinterpret_cast<const u4*>(grad + (int64_t)spos[j0 + u] * D)[gi];
-                    float part[8];
-#pragma unroll
-                    for (int k = 0; k < 8; ++k) part[k] = 0.0f;
-#pragma unroll
-                    for (int u = 0; u < kRowsPerPartial; ++u) {
-                        if (u < cnt) {
-#pragma unroll
-                            for (int k = 0; k < 8; ++k)
-                                part[k] = part[k] + grad_elem((uint16_t)(x[u][k >> 1] >> ((k & 1) * 16)), scale,
-                                                              scale_mode);
-                        }
-                    }
-#pragma unroll
-                    for (int k = 0; k < 8; ++k) acc[k] = acc[k] + part[k];
-                }
-#pragma unroll
-                for (int k = 0; k < 8; k += 2)
-                    o[k >> 1] = (uint32_t)finish(acc[k], scale, scale_mode) |
-                                ((uint32_t)finish(acc[k + 1], scale, scale_mode) << 16);
-            }
-            // nontemporal: the 616 MB table is written once and not read back here (0.155 vs 0.184 ms per call)
-            nt_store(reinterpret_cast<u4*>(orow) + gi, o);
+    const int64_t ng = D / 8;
+    if (empty) {
+        // nontemporal: the 616 MB table is written once and not read back here (0.155 vs 0.184 ms per call)
+        for (int64_t gi = lane; gi < ng; gi += kEmbThreads) nt_store8(orow + gi * 8, u4{0u, 0u, 0u, 0u});
+    } else {
+        // one occurrence (most rows): G groups at a time; more: half as many, whose sums fit the registers that leave
+        // room for kEmbWgPerCu resident rows per CU
+        constexpr int H = (G + 1) / 2;
+        if (hi - lo == 1) {
+            const uint16_t* row = grad + (int64_t)spos[lo] * D;
+            for (int64_t gi = lane; gi < ng; gi += kEmbThreads * G) copy_row<G>(row, gi, ng, scale, scale_mode, orow);
+        } else {
+            for (int64_t gi = lane; gi < ng; gi += kEmbThreads * H)
+                sum_row<FEW, H>(grad, D, spos, lo, hi, gi, ng, scale, scale_mode, orow);
         }
-        return;
     }
-    for (int64_t d = lane; d < D; d += kEmbThreads) {
-        uint16_t o = 0;
-        if (FEW && !empty) {
-            float acc = 0.0f;
-            for (int64_t j0 = lo; j0 < hi;) {
-                const int32_t cid = spos[j0] / chunk;
-                float part = 0.0f;
-                int64_t j = j0;
-                for (; j < hi && spos[j] / chunk == cid; ++j)
-                    part = part + grad_elem(grad[(int64_t)spos[j] * D + d], scale, scale_mode);
-                acc = bf16f(bf16r(acc + bf16f(bf16r(part))));
-                j0 = j;
+    const int64_t d = ng * 8 + lane;
+    if (d < D) {
+        float acc = 0.0f, part = 0.0f;
+        for (int64_t j = lo; !empty && j < hi; ++j) {
+            if (j > lo && new_part<FEW>(spos, lo, j)) {
+                acc = add_part<FEW>(acc, part);
+                part = 0.0f;
             }
-            o = finish(acc, scale, scale_mode);
-        } else if (!empty) {
-            float acc = 0.0f;
-            for (int64_t j0 = lo; j0 < hi; j0 += kRowsPerPartial) {
-                const int64_t j1 = j0 + kRowsPerPartial < hi ? j0 + kRowsPerPartial : hi;
-                float part = 0.0f;
-                for (int64_t j = j0; j < j1; ++j) part = part + grad_elem(grad[(int64_t)spos[j] * D + d], scale,
-                                                                          scale_mode);
-                acc = acc + part;
-            }
-            o = finish(acc, scale, scale_mode);
+            part = part + grad_elem(grad[(int64_t)spos[j] * D + d], scale, scale_mode);
         }
-        orow[d] = o;
+        orow[d] = finish(add_part<FEW>(acc, part), scale, scale_mode);
     }
 }
 
@@ -471,6 +492,30 @@ EmbWorkspace emb_workspace(void* base, int64_t R, int64_t D, int64_t V) {
     return w;
 }
 
+// The rows kernel with as many column groups per lane and step as the row needs, at most 6 (D 3072).
+template <bool FEW, int G>
+void launch_rows_g(int64_t D, int64_t V, size_t lds, hipStream_t st, const uint16_t* grad, const EmbWorkspace& w,
+                   int64_t padding_idx, float scale, int scale_mode, uint16_t* out) {
+    hipLaunchKernelGGL((emb_rows_kernel<FEW, G>), dim3((unsigned)V), dim3(kEmbThreads), lds, st, grad, D, w.svals,
+                       w.row_lo, padding_idx, scale, scale_mode, out, w.counts, w.heavy_list, w.heavy_base,
+                       w.long_list, w.long_base, w.run_start);
+}
+
+template <bool FEW>
+void launch_rows(int64_t D, int64_t V, size_t lds, hipStream_t st, const uint16_t* grad, const EmbWorkspace& w,
+                 int64_t padding_idx, float scale, int scale_mode, uint16_t* out) {
+    const int64_t need = (D / 8 + kEmbThreads - 1) / kEmbThreads;          // groups per lane
+    const int64_t steps = (need + 5) / 6;
+    switch (need > 0 ? (need + steps - 1) / steps : 1) {
+        case 1: return launch_rows_g<FEW, 1>(D, V, lds, st, grad, w, padding_idx, scale, scale_mode, out);
+        case 2: return launch_rows_g<FEW, 2>(D, V, lds, st, grad, w, padding_idx, scale, scale_mode, out);
+        case 3: return launch_rows_g<FEW, 3>(D, V, lds, st, grad, w, padding_idx, scale, scale_mode, out);
+        case 4: return launch_rows_g<FEW, 4>(D, V, lds, st, grad, w, padding_idx, scale, scale_mode, out);
+        case 5: return launch_rows_g<FEW, 5>(D, V, lds, st, grad, w, padding_idx, scale, scale_mode, out);
+        default: return launch_rows_g<FEW, 6>(D, V, lds, st, grad, w, padding_idx, scale, scale_mode, out);
+    }
+}
+
 }  // namespace
 
 extern "C" {
@@ -513,14 +558,9 @@ int z1_embedding_backward(const int64_t* ids, const uint16_t* grad, int64_t R, i
     size_t lds = 0;
     const int rc = z1detail::occupancy_lds(dev, kEmbWgPerCu, &lds);
     if (rc) return rc;
-    if (R < kSortMinRows)   // aten's kernel for few indices: its order, no heavy passes (nothing is listed for them)
-        hipLaunchKernelGGL(emb_rows_kernel<true>, dim3((unsigned)V), dim3(kEmbThreads), lds, st, grad, D, w.svals,
-                           w.row_lo, padding_idx, scale, scale_mode, vec, out, w.counts, w.heavy_list, w.heavy_base,
-                           w.long_list, w.long_base, w.run_start);
-    else
-        hipLaunchKernelGGL(emb_rows_kernel<false>, dim3((unsigned)V), dim3(kEmbThreads), lds, st, grad, D, w.svals,
-                           w.row_lo, padding_idx, scale, scale_mode, vec, out, w.counts, w.heavy_list, w.heavy_base,
-                           w.long_list, w.long_base, w.run_start);
+    // aten's kernel for few indices: its order, no heavy passes (nothing is listed for them)
+    if (R < kSortMinRows) launch_rows<true>(D, V, lds, st, grad, w, padding_idx, scale, scale_mode, out);
+    else launch_rows<false>(D, V, lds, st, grad, w, padding_idx, scale, scale_mode, out);
     e = hipGetLastError();
     if (e != hipSuccess) return (int)e;
     if (vec)

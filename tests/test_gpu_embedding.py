@@ -104,6 +104,23 @@ def test_matches_aten_at_3072_rows_or_fewer(pkg, dev, D):
         assert np.array_equal(bits(got2), bits(ref2)) and np.array_equal(bits(got3), bits(ref3)), R
 
 
+@pytest.mark.parametrize('R', [700, 4000])
+@pytest.mark.parametrize('D', [1, 7, 8, 9, 511, 512, 513, 1027, 1536, 2563, 3079, 4104, 6151])
+def test_row_widths(pkg, dev, R, D):
+    """Widths at the edges of a lane's column groups (8 columns, 64 lanes, up to 6 groups a step, several steps) and
+    rows at odd addresses, in both summation orders: bit-exact against aten, rows of -0.0 included."""
+    from faster_yoco_amd import embedding
+    rng = np.random.default_rng(D)
+    V = 900
+    ids = torch.from_numpy(np.concatenate([rng.integers(0, V, R - 300), rng.integers(0, 9, 300)])).to(dev)
+    g = (torch.randn(R, D, device=dev) * 1e-2).to(torch.bfloat16)
+    g[::5] = -0.0
+    ref = torch.ops.aten.embedding_dense_backward(g, ids, V, 3, False)
+    got = embedding.embedding_dense_backward(g, ids, V, 3)
+    torch.cuda.synchronize()
+    assert np.array_equal(bits(got), bits(ref))
+
+
 def test_matches_oracle_and_edge_cases(pkg, dev):
     from faster_yoco_amd import embedding
     rng = np.random.default_rng(3)
