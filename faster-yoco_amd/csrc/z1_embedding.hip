@@ -8,17 +8,18 @@
 // the indices in chunks of 16: per chunk and id an fp32 sum in position order, rounded to bf16 and added to the
 // bf16 row (emb_rows_kernel<true>; no heavy passes).  padding_idx rows and ids outside [0, V) contribute nothing.
 //
-//   1. keys[i] = id_i (or V when out of range), vals[i] = i;  2. stable sort by key: hipCUB's radix sort, or,
-//      while the stream is being captured into a HIP graph, rocPRIM's merge sort, which clears nothing with
-//      memsets (the radix sort does; both are stable, so the order is the same: 0.136 vs 0.142 ms per call);
-//   3. row_lo[t] = start of id t's run in the sorted keys (one binary search per t, all in parallel);
-//   4. one wave per output row t writes the row's sums -- or zeros -- exactly once, 8 bf16 columns per lane and
+//   1. each id's occurrences in position order (spos) and where they are (rng[t] = first sorted position, count): for
+//      up to kBucketRows rows one launch, emb_bucket_kernel; beyond, keys[i] = id_i (or V when out of range) and
+//      vals[i] = i sorted stably by key -- hipCUB's radix sort, or, while the stream is being captured into a HIP
+//      graph, rocPRIM's merge sort, which clears nothing with memsets (the radix sort does; both are stable, so the
+//      order is the same) -- and one binary search per t over the sorted keys;
+//   2. one wave per output row t writes the row's sums -- or zeros -- exactly once, 8 bf16 columns per lane and
 //      group, with nontemporal stores (aten zero-fills the whole table and then scatters into it; here every row of
 //      the table is written once), for ids with at most kHeavyRows occurrences; the others are listed, with a slot
 //      range for their runs, for
-//   5. emb_heavy_parts_kernel, which forms every run partial of every heavy id in parallel over the whole chip
+//   3. emb_heavy_parts_kernel, which forms every run partial of every heavy id in parallel over the whole chip
 //      into an fp32 workspace, and
-//   6. emb_heavy_chain_kernel, which adds each heavy id's partials in run order per column.  Token frequencies in
+//   4. emb_heavy_chain_kernel, which adds each heavy id's partials in run order per column.  Token frequencies in
 //      text are skewed: one wave (or one workgroup) walking thousands of occurrences of one id would take
 //      milliseconds.
 #include <hip/hip_runtime.h>
@@ -75,24 +76,149 @@ __global__ void emb_keys_kernel(const int64_t* __restrict__ ids, int64_t R, int6
     vals[i] = (int32_t)i;
 }
 
-// row_lo[t] = first index of the sorted keys that is >= t, for t in [0, V]: row t's occurrences are
-// [row_lo[t], row_lo[t+1]).  One independent binary search per thread (the latency of the searches overlaps).
+// rng[t] = (first index of the sorted keys that is >= t, number of keys equal to t), for t in [0, V).  Independent
+// binary searches, one thread per t (the latency of the searches overlaps).
 __global__ void emb_row_ranges_kernel(const uint32_t* __restrict__ sorted, int64_t R, int64_t V,
-                                      int32_t* __restrict__ row_lo, int* __restrict__ counts) {
+                                      int2* __restrict__ rng, int* __restrict__ counts) {
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t == 0) {                               // the rows kernel appends the heavy tokens after this kernel
         counts[0] = 0;
         counts[1] = 0;
         counts[2] = 0;
     }
-    if (t > V) return;
-    int64_t lo = 0, hi = R;
-    while (lo < hi) {
-        const int64_t mid = (lo + hi) >> 1;
-        if (sorted[mid] < (uint32_t)t) lo = mid + 1;
-        else hi = mid;
+    if (t >= V) return;
+    auto lower = [&](uint32_t key) {
+        int64_t lo = 0, hi = R;
+        while (lo < hi) {
+            const int64_t mid = (lo + hi) >> 1;
+            if (sorted[mid] < key) lo = mid + 1;
+            else hi = mid;
+        }
+        return (int32_t)lo;
+    };
+    const int32_t lo = lower((uint32_t)t);
+    rng[t] = int2{lo, lower((uint32_t)t + 1) - lo};
+}
+
+// The same results (spos, the sorted keys and rng) in one launch, without a sort over the whole list.  The ids are
+// split over 2^kb buckets, granules of 2^kGranuleBits consecutive ids round robin, one workgroup per bucket (text's
+// frequent ids are the small ones: spread, no workgroup gets them all).  Every workgroup reads all R ids, wave w the
+// w-th segment: it counts its bucket's ids per wave and local id in LDS (l: the id's number within the bucket) and how
+// many ids belong to smaller buckets, which is where its range of the sorted order starts; prefix sums over the waves
+// of one id, then over the ids, give every (wave, id) its place; then each wave places its occurrences in position
+// order, lanes with the same id by rank.  No workgroup waits for another, no atomic decides an order, nothing has to be
+// cleared beforehand.  Latency bounds it: two rounds over the wave's ids (kept in registers when they are one tile) and
+// three barriers, and for a frequent id the rounds of its bucket's placement.
+// Measured in whole calls of width 64 into 100,288 rows (uniform / Zipf(1.2) ids), against the five to seven launches
+// of keys, library sort and searches: 500 rows 37 / 45 against 43 / 51 us, 4096 42 / 52 against 55 / 66, 16,384
+// 48 / 70 against 71 / 89, 65,536 98 / 143 against 104 / 144, 131,072 148 / 231 against 136 / 203; the reading of all
+// ids by every workgroup grows with R, hence kBucketRows.  Granules of 8 ids put 8 frequent ids into one bucket (Zipf
+// 80 us at 16,384 rows), single ids scatter rng in 8-byte writes (52 / 71 us); fewer than 2^8 buckets leave
+// small vocabularies to a few workgroups (2000 rows: 57 us with 8, 41 us with 256).
+constexpr int kBucketThreads = 1024;
+constexpr int kBucketWaves = kBucketThreads / kWave;
+constexpr int kBucketTile = 16;            // ids per lane and tile
+constexpr int kGranuleBits = 1;
+constexpr int kMaxLocal = 512;             // local ids of a bucket: kBucketWaves x 512 counters, 32 KB of LDS
+constexpr int kMinBucketBits = 8;
+constexpr int kMaxBucketBits = 10;
+constexpr int64_t kBucketRows = 49152;
+constexpr int64_t kBucketVocab = (int64_t)kMaxLocal << kMaxBucketBits;
+
+__global__ __launch_bounds__(kBucketThreads) void emb_bucket_kernel(const int64_t* __restrict__ ids, int R, int V,
+                                                                    int kb, int32_t* __restrict__ spos,
+                                                                    uint32_t* __restrict__ skeys,
+                                                                    int2* __restrict__ rng, int* __restrict__ counts) {
+    __shared__ int hist[kBucketWaves][kMaxLocal];
+    __shared__ int wsum[kBucketWaves], wless[kBucketWaves];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x & (kWave - 1);
+    const int k = blockIdx.x, mask = (1 << kb) - 1;
+    if (k == 0 && threadIdx.x < 3) counts[threadIdx.x] = 0;   // the rows kernel appends the heavy tokens after this
+    for (int i = lane; i < kMaxLocal; i += kWave) hist[wave][i] = 0;        // this wave's own counters
+    // a wave's segment: positions [s0, s1), 64 consecutive ones a step
+    const int steps = (R + kBucketThreads - 1) / kBucketThreads;
+    const int s0 = wave * steps * kWave, s1 = s0 + steps * kWave < R ? s0 + steps * kWave : R;
+    int loc[kBucketTile];                    // local id, -1: another bucket's (or out of range)
+    int less = 0;
+    auto load = [&](int p0) {                // the tile at p0; returns how many of the lane's ids are in smaller buckets
+        int64_t t[kBucketTile];
+#pragma unroll
+        for (int i = 0; i < kBucketTile; ++i) {
+            const int p = p0 + i * kWave + lane;
+            t[i] = p < s1 ? ids[p] : -1;
+        }
+        int c = 0;
+#pragma unroll
+        for (int i = 0; i < kBucketTile; ++i) {
+            const bool ok = t[i] >= 0 && t[i] < V;
+            const int id = (int)t[i], b = (id >> kGranuleBits) & mask;
+            loc[i] = ok && b == k ? ((id >> (kGranuleBits + kb)) << kGranuleBits) | (id & ((1 << kGranuleBits) - 1)) : -1;
+            c += ok && b < k;
+        }
+        return c;
+    };
+    for (int p0 = s0; p0 < s1; p0 += kBucketTile * kWave) {
+        less += load(p0);
+#pragma unroll
+        for (int i = 0; i < kBucketTile; ++i)
+            if (loc[i] >= 0) atomicAdd(&hist[wave][loc[i]], 1);
     }
-    row_lo[t] = (int32_t)lo;
+    for (int off = kWave / 2; off > 0; off >>= 1) less += __shfl_xor(less, off);
+    if (lane == 0) wless[wave] = less;
+    __syncthreads();
+    // thread l: local id l's occurrences wave by wave, then its start among the bucket's ids
+    const int l = threadIdx.x;
+    int cnt = 0;
+    if (l < kMaxLocal) {
+        int c[kBucketWaves];
+#pragma unroll
+        for (int w = 0; w < kBucketWaves; ++w) c[w] = hist[w][l];
+#pragma unroll
+        for (int w = 0; w < kBucketWaves; ++w) {
+            hist[w][l] = cnt;
+            cnt += c[w];
+        }
+    }
+    int incl = cnt;
+    for (int off = 1; off < kWave; off <<= 1) {
+        const int x = __shfl_up(incl, off);
+        if (lane >= off) incl += x;
+    }
+    if (lane == kWave - 1) wsum[wave] = incl;
+    __syncthreads();
+    int start = incl - cnt;
+    for (int w = 0; w < kBucketWaves; ++w) start += wless[w] + (w < wave ? wsum[w] : 0);
+    if (l < kMaxLocal) {
+#pragma unroll
+        for (int w = 0; w < kBucketWaves; ++w) hist[w][l] += start;
+        const int64_t t = ((int64_t)(l >> kGranuleBits) << (kGranuleBits + kb)) + ((int64_t)k << kGranuleBits) +
+                          (l & ((1 << kGranuleBits) - 1));
+        if (t < V) rng[t] = int2{start, cnt};
+    }
+    __syncthreads();
+    const bool one_tile = steps <= kBucketTile;
+    for (int p0 = s0; p0 < s1; p0 += kBucketTile * kWave) {
+        if (!one_tile) load(p0);
+#pragma unroll
+        for (int i = 0; i < kBucketTile; ++i) {
+            uint64_t left = __ballot(loc[i] >= 0);
+            while (left) {                   // one id of the wave's 64 positions at a time, its lanes in order
+                const int leader = __builtin_ctzll(left);
+                const int l0 = __builtin_amdgcn_readlane(loc[i], leader);
+                const bool mine = loc[i] == l0;
+                const uint64_t same = __ballot(mine);
+                const int at = hist[wave][l0];
+                if (mine) {
+                    const int pos = at + __builtin_popcountll(same & ((1ull << lane) - 1));
+                    spos[pos] = p0 + i * kWave + lane;
+                    skeys[pos] = (uint32_t)(((l0 >> kGranuleBits) << (kGranuleBits + kb)) + (k << kGranuleBits) +
+                                            (l0 & ((1 << kGranuleBits) - 1)));
+                }
+                hist[wave][l0] = at + __builtin_popcountll(same);          // every lane, the same value
+                left &= ~same;
+            }
+        }
+    }
 }
 
 typedef uint32_t u4 __attribute__((ext_vector_type(4)));
@@ -223,7 +349,7 @@ __device__ __forceinline__ void sum_row(const uint16_t* __restrict__ grad, int64
 template <bool FEW, int G>
 __global__ __launch_bounds__(kEmbThreads) void emb_rows_kernel(const uint16_t* __restrict__ grad, int64_t D,
                                                                const int32_t* __restrict__ spos,
-                                                               const int32_t* __restrict__ row_lo,
+                                                               const int2* __restrict__ rng,
                                                                int64_t padding_idx, float scale, int scale_mode,
                                                                uint16_t* __restrict__ out,
                                                                int* __restrict__ counts,
@@ -242,7 +368,8 @@ __global__ __launch_bounds__(kEmbThreads) void emb_rows_kernel(const uint16_t* _
     }
     const int lane = threadIdx.x;
     uint16_t* orow = out + t * D;
-    const int64_t lo = row_lo[t], hi = row_lo[t + 1];
+    const int2 r = rng[t];
+    const int64_t lo = r.x, hi = lo + r.y;
     const bool empty = lo == hi || t == padding_idx;
     if (!FEW && !empty && hi - lo > kHeavyRows) {
         const int nrun = (int)((hi - lo + kRowsPerPartial - 1) / kRowsPerPartial);
@@ -297,7 +424,7 @@ template <int VEC>
 __global__ __launch_bounds__(kPartsThreads) void emb_heavy_parts_kernel(const uint16_t* __restrict__ grad, int64_t D,
                                                                         const int32_t* __restrict__ spos,
                                                                         const uint32_t* __restrict__ skeys,
-                                                                        const int32_t* __restrict__ row_lo,
+                                                                        const int2* __restrict__ rng,
                                                                         const int32_t* __restrict__ run_start,
                                                                         const int* __restrict__ counts, float scale,
                                                                         int scale_mode, float* __restrict__ parts) {
@@ -312,7 +439,8 @@ __global__ __launch_bounds__(kPartsThreads) void emb_heavy_parts_kernel(const ui
         const int64_t c0 = (item % ncg) * cols_per_item + (int64_t)lane * kCols;   // D % 8 == 0 when VEC
         if (c0 >= D) continue;
         const int64_t j0 = run_start[s];
-        const int64_t hi = row_lo[(int64_t)skeys[j0] + 1];
+        const int2 r = rng[skeys[j0]];
+        const int64_t hi = (int64_t)r.x + r.y;
         const int cnt = (int)(j0 + kRowsPerPartial < hi ? kRowsPerPartial : hi - j0);
         float part[kCols];
 #pragma unroll
@@ -354,7 +482,7 @@ __global__ __launch_bounds__(kPartsThreads) void emb_heavy_parts_kernel(const ui
 //     at once and adds them in registers, with no barrier.
 __global__ __launch_bounds__(kWave * kChainWaves) void emb_heavy_chain_kernel(const float* __restrict__ parts,
                                                                              int64_t D,
-                                                                             const int32_t* __restrict__ row_lo,
+                                                                             const int2* __restrict__ rng,
                                                                              const int32_t* __restrict__ heavy_list,
                                                                              const int32_t* __restrict__ heavy_base,
                                                                              const int32_t* __restrict__ long_list,
@@ -371,7 +499,7 @@ __global__ __launch_bounds__(kWave * kChainWaves) void emb_heavy_chain_kernel(co
         const int64_t col = (item % ncg) * kWave + lane;
         const bool valid = col < D;
         const int64_t t = long_list[h];
-        const int64_t nrun = (row_lo[t + 1] - row_lo[t] + kRowsPerPartial - 1) / kRowsPerPartial;
+        const int64_t nrun = ((int64_t)rng[t].y + kRowsPerPartial - 1) / kRowsPerPartial;
         const float* src = parts + (int64_t)long_base[h] * D + col;
         float acc = 0.0f;
         for (int64_t b = 0; b < nrun; b += kChainRows) {
@@ -406,7 +534,7 @@ __global__ __launch_bounds__(kWave * kChainWaves) void emb_heavy_chain_kernel(co
         const int64_t col = (item % ncg) * kWave + lane;
         if (col >= D) continue;
         const int64_t t = heavy_list[h];
-        const int nrun = (int)((row_lo[t + 1] - row_lo[t] + kRowsPerPartial - 1) / kRowsPerPartial);
+        const int nrun = (rng[t].y + kRowsPerPartial - 1) / kRowsPerPartial;
         const float* src = parts + (int64_t)heavy_base[h] * D + col;
         float x[kWaveChainRuns];
 #pragma unroll
@@ -443,15 +571,18 @@ bool capturing(hipStream_t st) {
 
 inline size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
-// Workspace: keys, positions, sorted keys, sorted positions (R each), row_lo (V + 1), the three counters, the two
-// lists of heavy tokens and their first run slots (at most R / 21 each), the run starts and the fp32 partials (R / 7
-// slots, D each), then the sort's temporary storage.
+// Whether the occurrences are put in order by emb_bucket_kernel (else by the library sort).
+bool bucketed(int64_t R, int64_t V) { return R <= kBucketRows && V <= kBucketVocab; }
+
+// Workspace: sorted keys and positions (R each), rng (V), the three counters, the two lists of heavy tokens and their
+// first run slots (at most R / 21 each), the run starts and the fp32 partials (R / 7 slots, D each), then, for the
+// library sort, its keys and positions (R each) and its temporary storage.
 struct EmbWorkspace {
     uint32_t* keys;
     int32_t* vals;
     uint32_t* skeys;
     int32_t* svals;
-    int32_t* row_lo;
+    int2* rng;
     int* counts;
     int32_t* heavy_list;
     int32_t* heavy_base;
@@ -474,11 +605,9 @@ EmbWorkspace emb_workspace(void* base, int64_t R, int64_t D, int64_t V) {
         return q;
     };
     const size_t r = (size_t)R, heavy = (size_t)(R / (kHeavyRows + 1)), slots = (size_t)(R / 7);
-    w.keys = reinterpret_cast<uint32_t*>(take(sizeof(uint32_t) * r));
-    w.vals = reinterpret_cast<int32_t*>(take(sizeof(int32_t) * r));
     w.skeys = reinterpret_cast<uint32_t*>(take(sizeof(uint32_t) * r));
     w.svals = reinterpret_cast<int32_t*>(take(sizeof(int32_t) * r));
-    w.row_lo = reinterpret_cast<int32_t*>(take(sizeof(int32_t) * (size_t)(V + 1)));
+    w.rng = reinterpret_cast<int2*>(take(sizeof(int2) * (size_t)V));
     w.counts = reinterpret_cast<int*>(take(3 * sizeof(int)));
     w.heavy_list = reinterpret_cast<int32_t*>(take(sizeof(int32_t) * heavy));
     w.heavy_base = reinterpret_cast<int32_t*>(take(sizeof(int32_t) * heavy));
@@ -486,8 +615,12 @@ EmbWorkspace emb_workspace(void* base, int64_t R, int64_t D, int64_t V) {
     w.long_base = reinterpret_cast<int32_t*>(take(sizeof(int32_t) * heavy));
     w.run_start = reinterpret_cast<int32_t*>(take(sizeof(int32_t) * slots));
     w.parts = reinterpret_cast<float*>(take(sizeof(float) * slots * (size_t)D));
-    w.temp_bytes = sort_temp_bytes(R);
-    w.temp = take(w.temp_bytes);
+    if (!bucketed(R, V)) {
+        w.keys = reinterpret_cast<uint32_t*>(take(sizeof(uint32_t) * r));
+        w.vals = reinterpret_cast<int32_t*>(take(sizeof(int32_t) * r));
+        w.temp_bytes = sort_temp_bytes(R);
+        w.temp = take(w.temp_bytes);
+    }
     w.total = off;
     return w;
 }
@@ -497,7 +630,7 @@ template <bool FEW, int G>
 void launch_rows_g(int64_t D, int64_t V, size_t lds, hipStream_t st, const uint16_t* grad, const EmbWorkspace& w,
                    int64_t padding_idx, float scale, int scale_mode, uint16_t* out) {
     hipLaunchKernelGGL((emb_rows_kernel<FEW, G>), dim3((unsigned)V), dim3(kEmbThreads), lds, st, grad, D, w.svals,
-                       w.row_lo, padding_idx, scale, scale_mode, out, w.counts, w.heavy_list, w.heavy_base,
+                       w.rng, padding_idx, scale, scale_mode, out, w.counts, w.heavy_list, w.heavy_base,
                        w.long_list, w.long_base, w.run_start);
 }
 
@@ -536,19 +669,26 @@ int z1_embedding_backward(const int64_t* ids, const uint16_t* grad, int64_t R, i
     hipStream_t st = static_cast<hipStream_t>(stream);
     const EmbWorkspace w = emb_workspace(workspace, R, D, V);
     hipError_t e = hipSuccess;
-    if (R > 0) {
-        hipLaunchKernelGGL(emb_keys_kernel, dim3((unsigned)((R + 255) / 256)), dim3(256), 0, st, ids, R, V, w.keys,
-                           w.vals);
-        e = hipGetLastError();
-        if (e != hipSuccess) return (int)e;
-        size_t tb = w.temp_bytes;
-        int end_bit = 1;
-        while (end_bit < 32 && ((uint64_t)V >> end_bit) != 0) ++end_bit;   // keys are <= V
-        e = sort_pairs(w.temp, tb, w.keys, w.skeys, w.vals, w.svals, R, end_bit, capturing(st), st);
-        if (e != hipSuccess) return (int)e;
+    if (bucketed(R, V)) {
+        int kb = kMinBucketBits;
+        while ((((V - 1) >> (kGranuleBits + kb)) + 1) << kGranuleBits > kMaxLocal / 2 && kb < kMaxBucketBits) ++kb;
+        hipLaunchKernelGGL(emb_bucket_kernel, dim3(1u << kb), dim3(kBucketThreads), 0, st, ids, (int)R, (int)V, kb,
+                           w.svals, w.skeys, w.rng, w.counts);
+    } else {
+        if (R > 0) {
+            hipLaunchKernelGGL(emb_keys_kernel, dim3((unsigned)((R + 255) / 256)), dim3(256), 0, st, ids, R, V, w.keys,
+                               w.vals);
+            e = hipGetLastError();
+            if (e != hipSuccess) return (int)e;
+            size_t tb = w.temp_bytes;
+            int end_bit = 1;
+            while (end_bit < 32 && ((uint64_t)V >> end_bit) != 0) ++end_bit;   // keys are <= V
+            e = sort_pairs(w.temp, tb, w.keys, w.skeys, w.vals, w.svals, R, end_bit, capturing(st), st);
+            if (e != hipSuccess) return (int)e;
+        }
+        hipLaunchKernelGGL(emb_row_ranges_kernel, dim3((unsigned)((V + 255) / 256)), dim3(256), 0, st, w.skeys, R, V,
+                           w.rng, w.counts);
     }
-    hipLaunchKernelGGL(emb_row_ranges_kernel, dim3((unsigned)((V + 1 + 255) / 256)), dim3(256), 0, st, w.skeys, R, V,
-                       w.row_lo, w.counts);
     e = hipGetLastError();
     if (e != hipSuccess) return (int)e;
     const int vec = (D % 8 == 0) && ((reinterpret_cast<uintptr_t>(grad) | reinterpret_cast<uintptr_t>(out)) & 15) == 0;
@@ -565,14 +705,14 @@ int z1_embedding_backward(const int64_t* ids, const uint16_t* grad, int64_t R, i
     if (e != hipSuccess) return (int)e;
     if (vec)
         hipLaunchKernelGGL(emb_heavy_parts_kernel<1>, dim3(kPartsGrid), dim3(kPartsThreads), 0, st, grad, D, w.svals,
-                           w.skeys, w.row_lo, w.run_start, w.counts, scale, scale_mode, w.parts);
+                           w.skeys, w.rng, w.run_start, w.counts, scale, scale_mode, w.parts);
     else
         hipLaunchKernelGGL(emb_heavy_parts_kernel<0>, dim3(kPartsGrid), dim3(kPartsThreads), 0, st, grad, D, w.svals,
-                           w.skeys, w.row_lo, w.run_start, w.counts, scale, scale_mode, w.parts);
+                           w.skeys, w.rng, w.run_start, w.counts, scale, scale_mode, w.parts);
     e = hipGetLastError();
     if (e != hipSuccess) return (int)e;
     hipLaunchKernelGGL(emb_heavy_chain_kernel, dim3(kChainGrid), dim3(kWave * kChainWaves), 0, st, w.parts, D,
-                       w.row_lo, w.heavy_list, w.heavy_base, w.long_list, w.long_base, w.counts, scale, scale_mode,
+                       w.rng, w.heavy_list, w.heavy_base, w.long_list, w.long_base, w.counts, scale, scale_mode,
                        out);
     e = hipGetLastError();
     return e == hipSuccess ? Z1_OK : (int)e;

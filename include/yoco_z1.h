@@ -244,12 +244,12 @@ int z1_cast_bf16(const float* p32, uint16_t* p16, int64_t n, void* stream);
  * sum rounded to bf16 and added to the bf16 row.  Every row of
  * out is written (rows without occurrences, padding_idx and ids outside [0, V) give zeros).  workspace: device
  * memory of z1_embedding_backward_workspace(R, D, V) bytes (with D <= 2^24: about 4/7 of R x D x 4 bytes for
- * the fp32 run partials of frequent ids, and R x 16 + V x 4 bytes plus the sort's storage).  */
+ * the fp32 run partials of frequent ids, R x 8 + V x 8 bytes, and for many rows the sort's storage).  */
 int z1_embedding_backward(const int64_t* ids, const uint16_t* grad, int64_t R, int64_t D, int64_t V,
                           int64_t padding_idx, float scale, int scale_mode, uint16_t* out, void* workspace,
                           int64_t workspace_bytes, void* stream);
 int64_t z1_embedding_backward_workspace(int64_t R, int64_t D, int64_t V);
-/* (z1_embedding_backward records no memset into a graph being captured: it sorts with a memset-free sort then.) */
+/* (z1_embedding_backward records no memset into a graph being captured: it orders the ids without one then.) */
 
 /* Text for a return code (negative: argument errors; positive: hipError_t). */
 const char* z1_strerror(int code);

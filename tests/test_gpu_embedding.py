@@ -104,6 +104,30 @@ def test_matches_aten_at_3072_rows_or_fewer(pkg, dev, D):
         assert np.array_equal(bits(got2), bits(ref2)) and np.array_equal(bits(got3), bits(ref3)), R
 
 
+@pytest.mark.parametrize('R', [1, 63, 1024, 1025, 16384, 16385, 20000, 49152, 49153])
+@pytest.mark.parametrize('V', [1, 2, 513, 65537, 524288, 524289])
+def test_order_of_occurrences(pkg, dev, R, V):
+    """Row counts and vocabularies at the edges of the one-launch ordering (a wave's 64 positions, one register tile of
+    16 x 1024 ids, its largest R and V and one beyond, where the library sort takes over): bit-exact against aten, with
+    skewed ids, the first and last id and (mapped to padding for aten) ids outside the vocabulary."""
+    from faster_yoco_amd import embedding
+    rng = np.random.default_rng(R * 7 + V)
+    ids = zipf_ids(rng, R, V, 1.3)
+    ids[rng.integers(0, R, R // 3)] = rng.integers(0, V, R // 3)
+    ids[0] = V - 1
+    bad = rng.integers(0, R, R // 50)
+    D = 8 if V > 100000 else 24
+    g = (torch.randn(R, D, device=dev) * 1e-2).to(torch.bfloat16)
+    ours = ids.copy()
+    ours[bad] = rng.choice([-1, V, V + 3, 2 ** 31 - 1, 2 ** 40], bad.size)
+    theirs = ids.copy()
+    theirs[bad] = V
+    ref = torch.ops.aten.embedding_dense_backward(g, torch.from_numpy(theirs).to(dev), V + 1, V, False)[:V]
+    got = embedding.embedding_dense_backward(g, torch.from_numpy(ours).to(dev), V, -1)
+    torch.cuda.synchronize()
+    assert np.array_equal(bits(got), bits(ref))
+
+
 @pytest.mark.parametrize('R', [700, 4000])
 @pytest.mark.parametrize('D', [1, 7, 8, 9, 511, 512, 513, 1027, 1536, 2563, 3079, 4104, 6151])
 def test_row_widths(pkg, dev, R, D):
