@@ -6,27 +6,26 @@
 // indices aten sorts: occurrences of each token id in stable position order, fp32 partial sums over runs of 10
 // consecutive occurrences, the partials summed in order, one rounding to bf16.  For fewer its other kernel walks
 // the indices in chunks of 16: per chunk and id an fp32 sum in position order, rounded to bf16 and added to the
-// bf16 row (emb_rows_kernel<true>; no heavy passes).  padding_idx rows and ids outside [0, V) contribute nothing.
+// bf16 row.  padding_idx rows and ids outside [0, V) contribute nothing.
 //
-//   1. each id's occurrences in position order (spos) and where they are (rng[t] = first sorted position, count): for
-//      up to kBucketRows rows one launch, emb_bucket_kernel; beyond, keys[i] = id_i (or V when out of range) and
-//      vals[i] = i sorted stably by key -- hipCUB's radix sort, or, while the stream is being captured into a HIP
-//      graph, rocPRIM's merge sort, which clears nothing with memsets (the radix sort does; both are stable, so the
-//      order is the same) -- and one binary search per t over the sorted keys;
-//   2. one wave per output row t writes the row's sums -- or zeros -- exactly once, 8 bf16 columns per lane and
-//      group, with nontemporal stores (aten zero-fills the whole table and then scatters into it; here every row of
-//      the table is written once), for ids with at most kHeavyRows occurrences; the others are listed, with a slot
-//      range for their runs, for
-//   3. emb_heavy_parts_kernel, which forms every run partial of every heavy id in parallel over the whole chip
-//      into an fp32 workspace, and
-//   4. emb_heavy_chain_kernel, which adds each heavy id's partials in run order per column.  Token frequencies in
-//      text are skewed: one wave (or one workgroup) walking thousands of occurrences of one id would take
-//      milliseconds.
+//   1. each id's occurrences in position order -- ent, sorted by id, equal ids by position -- and info[t], where those of
+//      id t are and how many: for up to kBucketRows rows one launch, emb_bucket_kernel; beyond, keys[i] = id_i (or V when
+//      out of range) and vals[i] = i sorted stably by key -- hipCUB's radix sort, or, while the stream is being captured
+//      into a HIP graph, rocPRIM's merge sort, which clears nothing with memsets (the radix sort does; both are stable,
+//      so the order is the same) -- one binary search per t over the sorted keys, and one pass that makes ent of them;
+//   2. emb_rows_kernel writes every row of the table exactly once (aten zero-fills the whole table and then scatters
+//      into it): first waves for the runs of ids with many occurrences, then one wave per row, in order, which zeroes
+//      it or sums its few occurrences.  Token frequencies in text are skewed: one wave (or one workgroup) walking
+//      thousands of occurrences of one id would take milliseconds;
+//   3. emb_chain_kernel adds the run partials of each id with several, in run order per column.
+// (For few indices a run is an id's occurrences in one chunk of 16 indices.)
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
 #include <rocprim/device/device_merge_sort.hpp>
 
 #include <stdint.h>
+
+#include <type_traits>
 
 #include "yoco_z1.h"
 #include "z1_internal.h"
@@ -41,31 +40,51 @@ constexpr int kRowsPerPartial = 10;        // aten's NROWS_PER_THREAD
 // kFewRowsChunk (torch's ROCm build; checked bit for bit against it on MI355X)
 constexpr int64_t kSortMinRows = 3073;
 constexpr int kFewRowsChunk = 16;
-// resident row workgroups per CU, capped with a dynamic LDS reservation the kernel does not use: 0.131 ms per call
-// at 9-10 per CU against 0.148 ms at the 32 the waves allow (0.144 at 16, 0.136 at 8, 0.146 at 7, 0.180 at 6)
-constexpr int kEmbWgPerCu = 10;
 constexpr int kWave = 64;
-// tokens with more occurrences go to the heavy passes; a heavy token's ceil(n / 10) runs are at most n / 7 for
-// n >= 21, so the run slots of all heavy tokens number at most R / 7
-constexpr int kHeavyRows = 20;
-static_assert(kHeavyRows >= 20, "the run-slot bound R / 7 needs heavy tokens of at least 21 occurrences");
-constexpr int kPartsThreads = 256;         // heavy pass 1: one run x column group per wave
-constexpr int kPartsGrid = 2048;
-constexpr int kChainWaves = 16;            // heavy pass 2: waves that load a batch of partials
-constexpr int kChainDepth = 16;            // partials per lane per batch
+// The rows launch.  Figures: whole calls on 16,384 rows of 3072 into a 100,288-row table, gradients not cached, uniform /
+// Zipf(1.2) ids; 141 / 152 us as it stands.
+// Resident workgroups per CU, capped with a dynamic LDS reservation the kernel does not use: 141 / 153 at 14, 143 / 152 at
+// 20, 152 / 157 at 10, 175 / 185 at 8 (a short table, 2000 rows of 768 into 32,000: 32.4 us at 20, 33.9 at 14, 37 at 10).
+constexpr int kEmbWgPerCu = 16;
+constexpr int kDirect = 4;                 // most occurrences of an id that the wave of its row sums (2: the same)
+constexpr int kRunBlock = 40;              // sorted positions whose runs a wave sums, for one step of 512 columns
+constexpr int kFewBlock = 8;               // the same, few indices
+constexpr int kMaxWaves = 1 << 20;         // most waves that sum runs (they stride beyond that)
+// Consecutive rows of one XCD: spans of 32 to 128 rows measure alike, single rows round robin 144 / 153; one eighth of the
+// table each leaves the frequent ids, which are the first ones, to one XCD.
+constexpr uint32_t kSpan = 128;
+// Cache-policy bits of the rows' stores, sc0 sc1 nt as the update's streams have: 141 / 154 us against 147 / 158 with nt
+// alone, 159 / 164 with sc0 sc1, 161 / 164 with none.  (Waves that only zero and waves that only sum, in one launch in
+// either order or mixed, 141-161 / 160-173: a row-ordered mix suits the DRAM better than two patterns at once.)
+constexpr int kRowPolicy = 1 | 2 | 16;
+// An id with more than kDirect occurrences is summed run by run.  If it has several runs, their partials go to slots:
+// run k of an id whose occurrences start at sorted position lo to slot ceil(lo / kSlotSpan) + k.  Its n >= 11
+// occurrences have ceil(n / 10) runs and at least (n - 6) / 4 whole slots of their own, which is never fewer.  (At most
+// kSortMinRows - 1 rows, where a run may be a single occurrence: slot = its sorted position.)
+constexpr int kSlotSpan = 4;
+static_assert(kRowsPerPartial == 10 && kSlotSpan == 4 && kDirect <= kRowsPerPartial, "slots of different ids are disjoint");
+constexpr int kChainWaves = 16;            // chain pass: waves that load a batch of partials
+constexpr int kChainDepth = 16;            // partials per lane per batch (64 KB of LDS)
 constexpr int kChainRows = kChainWaves * kChainDepth;
 static_assert(kChainRows % 16 == 0, "wave 0 reads a batch 16 rows at a time");
+constexpr int kFewRuns = (int)(kSortMinRows + kFewRowsChunk - 2) / kFewRowsChunk;    // most runs of an id, few indices
+static_assert(kFewRuns % kChainWaves == 0, "each wave loads as many");
 constexpr int kChainGrid = 512;
-constexpr int kWaveChainRuns = 32;         // heavy tokens of at most this many runs are chained by one wave
+constexpr int kWaveChainRuns = 32;         // ids of at most this many runs are chained by one wave
 constexpr int64_t kMaxCols = 1 << 24;      // D limit: keeps the workspace size and offsets far from overflow
 
 __device__ __forceinline__ float bf16f(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
 
-__device__ __forceinline__ uint16_t bf16r(float x) {
-    const uint32_t u = __float_as_uint(x);
-    if ((u & 0x7fffffffu) > 0x7f800000u) return 0x7fc0u;
-    return (uint16_t)((u + 0x7fffu + ((u >> 16) & 1u)) >> 16);
-}
+// Round to nearest even, with gfx950's conversion (any NaN gives a NaN).
+__device__ __forceinline__ uint16_t bf16r(float x) { return __builtin_bit_cast(uint16_t, (__bf16)x); }
+
+// One place of the sorted order: the occurrence's position, its id, and the id's first place and count.
+struct Ent {
+    int32_t pos;
+    uint32_t id;
+    int32_t lo, n;
+};
+static_assert(sizeof(Ent) == 16, "one 16-byte load");
 
 __global__ void emb_keys_kernel(const int64_t* __restrict__ ids, int64_t R, int64_t V, uint32_t* __restrict__ keys,
                                 int32_t* __restrict__ vals) {
@@ -76,31 +95,40 @@ __global__ void emb_keys_kernel(const int64_t* __restrict__ ids, int64_t R, int6
     vals[i] = (int32_t)i;
 }
 
-// rng[t] = (first index of the sorted keys that is >= t, number of keys equal to t), for t in [0, V).  Independent
-// binary searches, one thread per t (the latency of the searches overlaps).
-__global__ void emb_row_ranges_kernel(const uint32_t* __restrict__ sorted, int64_t R, int64_t V,
-                                      int2* __restrict__ rng, int* __restrict__ counts) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t == 0) {                               // the rows kernel appends the heavy tokens after this kernel
-        counts[0] = 0;
-        counts[1] = 0;
-        counts[2] = 0;
+// info[t] = (where, count) of id t's occurrences, for t in [0, V): their first sorted place, or the position of the
+// only one.  Independent binary searches over the sorted keys, one thread per t (the latency of the searches overlaps).
+__device__ __forceinline__ int32_t lower_bound(const uint32_t* __restrict__ sorted, int64_t R, uint32_t key) {
+    int64_t lo = 0, hi = R;
+    while (lo < hi) {
+        const int64_t mid = (lo + hi) >> 1;
+        if (sorted[mid] < key) lo = mid + 1;
+        else hi = mid;
     }
-    if (t >= V) return;
-    auto lower = [&](uint32_t key) {
-        int64_t lo = 0, hi = R;
-        while (lo < hi) {
-            const int64_t mid = (lo + hi) >> 1;
-            if (sorted[mid] < key) lo = mid + 1;
-            else hi = mid;
-        }
-        return (int32_t)lo;
-    };
-    const int32_t lo = lower((uint32_t)t);
-    rng[t] = int2{lo, lower((uint32_t)t + 1) - lo};
+    return (int32_t)lo;
 }
 
-// The same results (spos, the sorted keys and rng) in one launch, without a sort over the whole list.  The ids are
+__global__ void emb_row_ranges_kernel(const uint32_t* __restrict__ sorted, const int32_t* __restrict__ spos, int64_t R,
+                                      int64_t V, int2* __restrict__ info, int* __restrict__ counts) {
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t < 2) counts[t] = 0;                   // the rows kernel appends to the chain pass's lists after this kernel
+    if (t >= V) return;
+    const int32_t lo = lower_bound(sorted, R, (uint32_t)t), hi = lower_bound(sorted, R, (uint32_t)t + 1);
+    info[t] = int2{hi - lo == 1 ? spos[lo] : lo, hi - lo};
+    if (t == V - 1) counts[2] = hi;             // the ids inside [0, V)
+}
+
+// ent of every sorted place.
+__global__ void emb_entries_kernel(const uint32_t* __restrict__ sorted, const int32_t* __restrict__ spos, int64_t R,
+                                   int64_t V, const int2* __restrict__ info, Ent* __restrict__ ent) {
+    const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (p >= R) return;
+    const uint32_t id = sorted[p];
+    if ((int64_t)id >= V) return;
+    const int2 r = info[id];
+    ent[p] = Ent{spos[p], id, r.y == 1 ? (int32_t)p : r.x, r.y};
+}
+
+// The same results (ent and info) in one launch, without a sort over the whole list.  The ids are
 // split over 2^kb buckets, granules of 2^kGranuleBits consecutive ids round robin, one workgroup per bucket (text's
 // frequent ids are the small ones: spread, no workgroup gets them all).  Every workgroup reads all R ids, wave w the
 // w-th segment: it counts its bucket's ids per wave and local id in LDS (l: the id's number within the bucket) and how
@@ -113,7 +141,7 @@ __global__ void emb_row_ranges_kernel(const uint32_t* __restrict__ sorted, int64
 // of keys, library sort and searches: 500 rows 37 / 45 against 43 / 51 us, 4096 42 / 52 against 55 / 66, 16,384
 // 48 / 70 against 71 / 89, 65,536 98 / 143 against 104 / 144, 131,072 148 / 231 against 136 / 203; the reading of all
 // ids by every workgroup grows with R, hence kBucketRows.  Granules of 8 ids put 8 frequent ids into one bucket (Zipf
-// 80 us at 16,384 rows), single ids scatter rng in 8-byte writes (52 / 71 us); fewer than 2^8 buckets leave
+// 80 us at 16,384 rows), single ids scatter info in 8-byte writes (52 / 71 us); fewer than 2^8 buckets leave
 // small vocabularies to a few workgroups (2000 rows: 57 us with 8, 41 us with 256).
 constexpr int kBucketThreads = 1024;
 constexpr int kBucketWaves = kBucketThreads / kWave;
@@ -126,14 +154,15 @@ constexpr int64_t kBucketRows = 49152;
 constexpr int64_t kBucketVocab = (int64_t)kMaxLocal << kMaxBucketBits;
 
 __global__ __launch_bounds__(kBucketThreads) void emb_bucket_kernel(const int64_t* __restrict__ ids, int R, int V,
-                                                                    int kb, int32_t* __restrict__ spos,
-                                                                    uint32_t* __restrict__ skeys,
-                                                                    int2* __restrict__ rng, int* __restrict__ counts) {
+                                                                    int kb, Ent* __restrict__ ent,
+                                                                    int2* __restrict__ info,
+                                                                    int* __restrict__ counts) {
     __shared__ int hist[kBucketWaves][kMaxLocal];
+    __shared__ int2 range[kMaxLocal];        // a local id's first place and count
     __shared__ int wsum[kBucketWaves], wless[kBucketWaves];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x & (kWave - 1);
     const int k = blockIdx.x, mask = (1 << kb) - 1;
-    if (k == 0 && threadIdx.x < 3) counts[threadIdx.x] = 0;   // the rows kernel appends the heavy tokens after this
+    if (k == 0 && threadIdx.x < 2) counts[threadIdx.x] = 0;   // the rows kernel appends to the lists after this
     for (int i = lane; i < kMaxLocal; i += kWave) hist[wave][i] = 0;        // this wave's own counters
     // a wave's segment: positions [s0, s1), 64 consecutive ones a step
     const int steps = (R + kBucketThreads - 1) / kBucketThreads;
@@ -188,12 +217,14 @@ __global__ __launch_bounds__(kBucketThreads) void emb_bucket_kernel(const int64_
     __syncthreads();
     int start = incl - cnt;
     for (int w = 0; w < kBucketWaves; ++w) start += wless[w] + (w < wave ? wsum[w] : 0);
+    if (k == mask && threadIdx.x == kBucketThreads - 1) counts[2] = start + cnt;    // the ids inside [0, V)
     if (l < kMaxLocal) {
 #pragma unroll
         for (int w = 0; w < kBucketWaves; ++w) hist[w][l] += start;
         const int64_t t = ((int64_t)(l >> kGranuleBits) << (kGranuleBits + kb)) + ((int64_t)k << kGranuleBits) +
                           (l & ((1 << kGranuleBits) - 1));
-        if (t < V) rng[t] = int2{start, cnt};
+        range[l] = int2{start, cnt};
+        if (t < V && cnt != 1) info[t] = int2{start, cnt};
     }
     __syncthreads();
     const bool one_tile = steps <= kBucketTile;
@@ -208,11 +239,13 @@ __global__ __launch_bounds__(kBucketThreads) void emb_bucket_kernel(const int64_
                 const bool mine = loc[i] == l0;
                 const uint64_t same = __ballot(mine);
                 const int at = hist[wave][l0];
+                const int2 r = range[l0];
+                const int id = ((l0 >> kGranuleBits) << (kGranuleBits + kb)) + (k << kGranuleBits) +
+                               (l0 & ((1 << kGranuleBits) - 1));
                 if (mine) {
-                    const int pos = at + __builtin_popcountll(same & ((1ull << lane) - 1));
-                    spos[pos] = p0 + i * kWave + lane;
-                    skeys[pos] = (uint32_t)(((l0 >> kGranuleBits) << (kGranuleBits + kb)) + (k << kGranuleBits) +
-                                            (l0 & ((1 << kGranuleBits) - 1)));
+                    const int p = p0 + i * kWave + lane;
+                    ent[at + __builtin_popcountll(same & ((1ull << lane) - 1))] = Ent{p, (uint32_t)id, r.x, r.y};
+                    if (r.y == 1) info[id] = int2{p, 1};
                 }
                 hist[wave][l0] = at + __builtin_popcountll(same);          // every lane, the same value
                 left &= ~same;
@@ -250,6 +283,16 @@ __device__ __forceinline__ void nt_store8(uint16_t* p, u4 x) {
     __builtin_nontemporal_store((u4_any)x, (__attribute__((address_space(1))) u4_any*)p);
 }
 
+// Stores to one row of the table: 16 bytes at byte offset off of orow (the same in the whole wave).  Rows on 16-byte
+// boundaries (wide) take buffer stores marked kRowPolicy; others plain nontemporal ones.
+__device__ __forceinline__ void row_store8(uint16_t* orow, bool wide, int bytes, int off, u4 x) {
+    if (wide)
+        __builtin_amdgcn_raw_buffer_store_b128(x, __builtin_amdgcn_make_buffer_rsrc(orow, 0, bytes, 0x00020000), off, 0,
+                                               kRowPolicy);
+    else
+        nt_store8(orow + off / 2, x);
+}
+
 // Adds a finished partial to the row's sum: aten's sort path adds fp32 partials; its few-indices kernel rounds the
 // partial to bf16 and the row after the add.
 template <bool FEW>
@@ -257,250 +300,244 @@ __device__ __forceinline__ float add_part(float acc, float part) {
     return FEW ? bf16f(bf16r(acc + bf16f(bf16r(part)))) : acc + part;
 }
 
-// Whether occurrence j of a row whose occurrences start at lo begins another partial (j > lo): every 10th occurrence,
-// or, for few indices, where the next chunk of 16 indices begins.
+// Whether the occurrence at sorted place p (position pos) of an id starting at lo begins a run: every 10th one, or, for
+// few indices, the first one in its chunk of 16 positions (prev: the position at place p - 1, read where p > lo).
 template <bool FEW>
-__device__ __forceinline__ bool new_part(const int32_t* __restrict__ spos, int64_t lo, int64_t j) {
-    return FEW ? spos[j] / kFewRowsChunk != spos[j - 1] / kFewRowsChunk : (j - lo) % kRowsPerPartial == 0;
+__device__ __forceinline__ bool run_starts(int p, int lo, int pos, int prev) {
+    return p == lo || (FEW ? pos / kFewRowsChunk != prev / kFewRowsChunk : (p - lo) % kRowsPerPartial == 0);
 }
 
-// A row with one occurrence: all G of a lane's column groups (gi, gi + 64, ... below ng, 8 columns each) loaded at once
-// -- the gradient row comes from HBM, so the wave waits for memory once a row instead of once a group -- and rounded.
-// With this and sum_row below, 16,384 rows of 3072 into a 100,288-row table, gradients not in a cache: 163 us a call
-// against 205 us with each group loaded, summed and stored before the next (Zipf ids 205 against 231 us).
-template <int G>
-__device__ __forceinline__ void copy_row(const uint16_t* __restrict__ row, int64_t gi, int64_t ng, float scale,
-                                         int scale_mode, uint16_t* __restrict__ orow) {
-    u4 x[G];
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-        x[g] = u4{0u, 0u, 0u, 0u};
-        if (gi + g * kEmbThreads < ng) x[g] = load8(row + (gi + g * kEmbThreads) * 8);
+template <bool FEW>
+__device__ __forceinline__ int64_t run_slot(int lo, int p) {
+    return FEW ? p : ((int64_t)lo + kSlotSpan - 1) / kSlotSpan + (p - lo) / kRowsPerPartial;
+}
+
+__device__ __forceinline__ uint16_t col(const u4& x, int k) { return (uint16_t)(x[k >> 1] >> ((k & 1) * 16)); }
+
+typedef float f4 __attribute__((ext_vector_type(4)));
+typedef f4 f4_any __attribute__((aligned(4)));
+
+// The runs that start at sorted places [p0, p0 + block) and belong to ids of more than kDirect occurrences, columns
+// [512 step, 512 (step + 1)) of each; the wave of the last step also takes the last D % 8 columns, one per lane.  A
+// run's rows (at most 10, or 16 for few indices) are loaded together and summed in order.  The sum of an id's only run
+// is its row; otherwise the fp32 partial goes to the run's slot, and the wave of step 0 lists the id for the chain pass.
+template <bool FEW>
+__device__ __forceinline__ void sum_runs(int64_t p0, int step, bool last_step, const uint16_t* __restrict__ grad, int64_t D,
+                                         const Ent* __restrict__ ent, int64_t padding_idx, float scale, int scale_mode,
+                                         int64_t valid, uint16_t* __restrict__ out, int* __restrict__ counts,
+                                         int32_t* __restrict__ short_list, int32_t* __restrict__ long_list,
+                                         float* __restrict__ parts) {
+    constexpr int kBlock = FEW ? kFewBlock : kRunBlock, kRows = FEW ? kFewRowsChunk : kRowsPerPartial;
+    static_assert(1 + kBlock + kRows <= kWave, "the lanes hold every place a run of the block can reach");
+    const int lane = threadIdx.x;
+    // lane i: place p0 - 1 + i
+    const int64_t p = p0 - 1 + lane;
+    Ent e = Ent{0, 0, 0, 0};
+    if (p >= 0 && p < valid && lane < 1 + kBlock + kRows) e = ent[p];
+    const int prev = __shfl_up(e.pos, 1);
+    const bool begins = p >= e.lo && e.n > 0 && run_starts<FEW>((int)p, e.lo, e.pos, prev);
+    const bool mine = begins && lane >= 1 && lane <= kBlock && e.n > kDirect && (int64_t)e.id != padding_idx;
+    const bool single = !FEW && e.n <= kRowsPerPartial;
+    if (mine && !single && p == e.lo && step == 0) {
+        const bool is_short = (FEW ? e.n : (e.n + kRowsPerPartial - 1) / kRowsPerPartial) <= kWaveChainRuns;
+        (is_short ? short_list : long_list)[atomicAdd(&counts[is_short ? 0 : 1], 1)] = e.lo;
     }
+    const int64_t ng = D / 8, gi = (int64_t)step * kEmbThreads + lane;
+    for (uint64_t left = __ballot(mine), starts = __ballot(begins); left; left &= left - 1) {
+        const int l = __builtin_ctzll(left);
+        const int lo = __builtin_amdgcn_readlane(e.lo, l), n = __builtin_amdgcn_readlane(e.n, l), s = (int)p0 - 1 + l;
+        // its rows: up to the next run's start or the id's end
+        const uint64_t next = starts >> 1 >> l;
+        int cnt = next ? 1 + __builtin_ctzll(next) : kRows;
+        if (lo + n - s < cnt) cnt = lo + n - s;
+        if (cnt > kRows) cnt = kRows;
+        const int64_t row = (int64_t)__builtin_amdgcn_readlane((int)e.id, l) & 0xffffffff;
+        const bool only = !FEW && n <= kRowsPerPartial;
+        float* dst = parts + (only ? 0 : run_slot<FEW>(lo, s)) * D;
+        if (gi < ng) {
+            u4 x[kRows];
 #pragma unroll
-    for (int g = 0; g < G; ++g) {
-        u4 o;
+            for (int u = 0; u < kRows; ++u)
+                if (u < cnt) x[u] = load8(grad + (int64_t)__builtin_amdgcn_readlane(e.pos, l + u) * D + gi * 8);
+            float part[8];
 #pragma unroll
-        for (int k = 0; k < 4; ++k)       // 0 + x: the sum of one element (-0 gives +0)
-            o[k] = (uint32_t)finish(0.0f + grad_elem((uint16_t)x[g][k], scale, scale_mode), scale, scale_mode) |
-                   ((uint32_t)finish(0.0f + grad_elem((uint16_t)(x[g][k] >> 16), scale, scale_mode), scale, scale_mode)
-                    << 16);
-        if (gi + g * kEmbThreads < ng) nt_store8(orow + (gi + g * kEmbThreads) * 8, o);
+            for (int k = 0; k < 8; ++k) part[k] = 0.0f;
+#pragma unroll
+            for (int u = 0; u < kRows; ++u) {
+                if (u < cnt) {
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) part[k] = part[k] + grad_elem(col(x[u], k), scale, scale_mode);
+                }
+            }
+            if (only) {
+                u4 o;
+#pragma unroll
+                for (int k = 0; k < 8; k += 2)
+                    o[k >> 1] = (uint32_t)finish(0.0f + part[k], scale, scale_mode) |
+                                ((uint32_t)finish(0.0f + part[k + 1], scale, scale_mode) << 16);
+                nt_store8(out + row * D + gi * 8, o);
+            } else {
+                f4_any* o = reinterpret_cast<f4_any*>(dst + gi * 8);
+                o[0] = f4{part[0], part[1], part[2], part[3]};
+                o[1] = f4{part[4], part[5], part[6], part[7]};
+            }
+        }
+        if (last_step && ng * 8 < D) {
+            const int64_t d = ng * 8 + lane;
+            float part = 0.0f;
+            for (int u = 0; u < cnt; ++u) {
+                const int64_t at = __builtin_amdgcn_readlane(e.pos, l + u);
+                if (d < D) part = part + grad_elem(grad[at * D + d], scale, scale_mode);
+            }
+            if (d < D) {
+                if (only) out[row * D + d] = finish(0.0f + part, scale, scale_mode);
+                else dst[d] = part;
+            }
+        }
     }
 }
 
-// One row's sum over its occurrences [lo, hi) for G column groups of a lane, as in copy_row: all G loads of an
-// occurrence are in flight together, the next occurrence's as well.
-template <bool FEW, int G>
-__device__ __forceinline__ void sum_row(const uint16_t* __restrict__ grad, int64_t D, const int32_t* __restrict__ spos,
-                                        int64_t lo, int64_t hi, int64_t gi, int64_t ng, float scale, int scale_mode,
-                                        uint16_t* __restrict__ orow) {
-    u4 x[G], y[G];
-    float acc[G][8], part[G][8];
-    auto load = [&](u4* d, int64_t j) {
-        const uint16_t* row = grad + (int64_t)spos[j] * D;
+// One output row without occurrences, or with at most kDirect: zeros, or all G column groups of a lane (64 groups of 8
+// columns apart) of all its occurrences in flight together, the gradient rows coming from HBM.  `at`: their positions.
+template <bool FEW, int G, int N>
+__device__ __forceinline__ void sum_direct(const int* at, int n, const uint16_t* __restrict__ grad, int64_t D, float scale,
+                                           int scale_mode, bool wide, uint16_t* __restrict__ orow) {
+    const int lane = threadIdx.x, ng = (int)(D / 8);
+    for (int gi = lane; gi < ng; gi += kEmbThreads * G) {
+        u4 x[N][G];
 #pragma unroll
-        for (int g = 0; g < G; ++g)
-            if (gi + g * kEmbThreads < ng) d[g] = load8(row + (gi + g * kEmbThreads) * 8);
-    };
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-        x[g] = y[g] = u4{0u, 0u, 0u, 0u};
-#pragma unroll
-        for (int k = 0; k < 8; ++k) acc[g][k] = part[g][k] = 0.0f;
-    }
-    load(x, lo);
-    for (int64_t j = lo; j < hi; ++j) {
-        if (j + 1 < hi) load(y, j + 1);
-        if (j > lo && new_part<FEW>(spos, lo, j)) {
+        for (int u = 0; u < N; ++u)
 #pragma unroll
             for (int g = 0; g < G; ++g)
-#pragma unroll
-                for (int k = 0; k < 8; ++k) {
-                    acc[g][k] = add_part<FEW>(acc[g][k], part[g][k]);
-                    part[g][k] = 0.0f;
-                }
-        }
+                if (u < n && gi + g * kEmbThreads < ng)
+                    x[u][g] = load8(grad + (int64_t)at[u] * D + (gi + g * kEmbThreads) * 8);
 #pragma unroll
         for (int g = 0; g < G; ++g) {
+            float acc[8], part[8];
 #pragma unroll
-            for (int k = 0; k < 8; ++k)
-                part[g][k] = part[g][k] + grad_elem((uint16_t)(x[g][k >> 1] >> ((k & 1) * 16)), scale, scale_mode);
-            x[g] = y[g];
+            for (int k = 0; k < 8; ++k) acc[k] = part[k] = 0.0f;
+#pragma unroll
+            for (int u = 0; u < N; ++u) {
+                if (u < n) {
+                    if (FEW && u > 0 && at[u] / kFewRowsChunk != at[u - 1] / kFewRowsChunk) {
+#pragma unroll
+                        for (int k = 0; k < 8; ++k) {
+                            acc[k] = add_part<FEW>(acc[k], part[k]);
+                            part[k] = 0.0f;
+                        }
+                    }
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) part[k] = part[k] + grad_elem(col(x[u][g], k), scale, scale_mode);
+                }
+            }
+            u4 o;
+#pragma unroll
+            for (int k = 0; k < 8; k += 2)
+                o[k >> 1] = (uint32_t)finish(add_part<FEW>(acc[k], part[k]), scale, scale_mode) |
+                            ((uint32_t)finish(add_part<FEW>(acc[k + 1], part[k + 1]), scale, scale_mode) << 16);
+            if (gi + g * kEmbThreads < ng) row_store8(orow, wide, ng * 16, (gi + g * kEmbThreads) * 16, o);
         }
     }
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-        u4 o;
-#pragma unroll
-        for (int k = 0; k < 8; k += 2)
-            o[k >> 1] = (uint32_t)finish(add_part<FEW>(acc[g][k], part[g][k]), scale, scale_mode) |
-                        ((uint32_t)finish(add_part<FEW>(acc[g][k + 1], part[g][k + 1]), scale, scale_mode) << 16);
-        if (gi + g * kEmbThreads < ng) nt_store8(orow + (gi + g * kEmbThreads) * 8, o);
-    }
-}
-
-// One wave per output row t (light tokens: at most kHeavyRows occurrences, and empty or padding rows): the row's
-// sums -- or zeros -- written once, G groups of 8 bf16 columns per lane and step, the last D % 8 columns one per lane.
-// A token with more occurrences is appended, with the first of its nrun run slots (from counts[1]), to the list of
-// tokens of at most kWaveChainRuns runs (heavy_list / heavy_base, count counts[0]) or to that of longer ones
-// (long_list / long_base, counts[2]); run_start[slot] = the sorted position of the run's first row.  Its row is left to
-// the heavy passes.  The atomics only decide where a token's partials are kept, not how they are summed.
-template <bool FEW, int G>
-__global__ __launch_bounds__(kEmbThreads) void emb_rows_kernel(const uint16_t* __restrict__ grad, int64_t D,
-                                                               const int32_t* __restrict__ spos,
-                                                               const int2* __restrict__ rng,
-                                                               int64_t padding_idx, float scale, int scale_mode,
-                                                               uint16_t* __restrict__ out,
-                                                               int* __restrict__ counts,
-                                                               int32_t* __restrict__ heavy_list,
-                                                               int32_t* __restrict__ heavy_base,
-                                                               int32_t* __restrict__ long_list,
-                                                               int32_t* __restrict__ long_base,
-                                                               int32_t* __restrict__ run_start) {
-    // row of workgroup b: undoes the round-robin dispatch over the 8 XCDs, so each XCD writes one contiguous
-    // eighth of the table (0.148 vs 0.153 ms per call for t = b)
-    int64_t t;
-    {
-        const int64_t b = blockIdx.x, nb = gridDim.x;
-        const int64_t x = b & 7, q = b >> 3, Q = nb >> 3, R = nb & 7;
-        t = x * Q + (x < R ? x : R) + q;
-    }
-    const int lane = threadIdx.x;
-    uint16_t* orow = out + t * D;
-    const int2 r = rng[t];
-    const int64_t lo = r.x, hi = lo + r.y;
-    const bool empty = lo == hi || t == padding_idx;
-    if (!FEW && !empty && hi - lo > kHeavyRows) {
-        const int nrun = (int)((hi - lo + kRowsPerPartial - 1) / kRowsPerPartial);
-        int base = 0;
-        if (lane == 0) {
-            const bool wave_chain = nrun <= kWaveChainRuns;
-            const int h = atomicAdd(&counts[wave_chain ? 0 : 2], 1);
-            base = atomicAdd(&counts[1], nrun);
-            (wave_chain ? heavy_list : long_list)[h] = (int32_t)t;
-            (wave_chain ? heavy_base : long_base)[h] = base;
-        }
-        base = __shfl(base, 0);
-        for (int k = lane; k < nrun; k += kEmbThreads) run_start[base + k] = (int32_t)(lo + (int64_t)k * kRowsPerPartial);
-        return;
-    }
-    const int64_t ng = D / 8;
-    if (empty) {
-        // nontemporal: the 616 MB table is written once and not read back here (0.155 vs 0.184 ms per call)
-        for (int64_t gi = lane; gi < ng; gi += kEmbThreads) nt_store8(orow + gi * 8, u4{0u, 0u, 0u, 0u});
-    } else {
-        // one occurrence (most rows): G groups at a time; more: half as many, whose sums fit the registers that leave
-        // room for kEmbWgPerCu resident rows per CU
-        constexpr int H = (G + 1) / 2;
-        if (hi - lo == 1) {
-            const uint16_t* row = grad + (int64_t)spos[lo] * D;
-            for (int64_t gi = lane; gi < ng; gi += kEmbThreads * G) copy_row<G>(row, gi, ng, scale, scale_mode, orow);
-        } else {
-            for (int64_t gi = lane; gi < ng; gi += kEmbThreads * H)
-                sum_row<FEW, H>(grad, D, spos, lo, hi, gi, ng, scale, scale_mode, orow);
-        }
-    }
-    const int64_t d = ng * 8 + lane;
+    const int d = ng * 8 + lane;
     if (d < D) {
         float acc = 0.0f, part = 0.0f;
-        for (int64_t j = lo; !empty && j < hi; ++j) {
-            if (j > lo && new_part<FEW>(spos, lo, j)) {
-                acc = add_part<FEW>(acc, part);
-                part = 0.0f;
+#pragma unroll
+        for (int u = 0; u < N; ++u) {
+            if (u < n) {
+                if (FEW && u > 0 && at[u] / kFewRowsChunk != at[u - 1] / kFewRowsChunk) {
+                    acc = add_part<FEW>(acc, part);
+                    part = 0.0f;
+                }
+                part = part + grad_elem(grad[(int64_t)at[u] * D + d], scale, scale_mode);
             }
-            part = part + grad_elem(grad[(int64_t)spos[j] * D + d], scale, scale_mode);
         }
         orow[d] = finish(add_part<FEW>(acc, part), scale, scale_mode);
     }
 }
 
-// Heavy tokens, pass 1: every run of 10 occurrences of every heavy token, for every column group (512 columns on
-// the vector path, 64 otherwise), is one wave's item; the wave sums the run's rows in order (loads issued together)
-// and stores the fp32 partial to its run slot of parts (parts[s * D + column]).  The run of slot s starts at sorted
-// position run_start[s], and its token is the sorted key there.  Items are spread over the whole
-// grid, so one token's thousands of runs are formed in parallel; every wave exits once the items run out.
-template <int VEC>
-__global__ __launch_bounds__(kPartsThreads) void emb_heavy_parts_kernel(const uint16_t* __restrict__ grad, int64_t D,
-                                                                        const int32_t* __restrict__ spos,
-                                                                        const uint32_t* __restrict__ skeys,
-                                                                        const int2* __restrict__ rng,
-                                                                        const int32_t* __restrict__ run_start,
-                                                                        const int* __restrict__ counts, float scale,
-                                                                        int scale_mode, float* __restrict__ parts) {
-    constexpr int kCols = VEC ? 8 : 1;                       // columns per lane
-    constexpr int kWaves = kPartsThreads / kWave;
-    const int wave = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
-    const int64_t cols_per_item = (int64_t)kWave * kCols;
-    const int64_t ncg = (D + cols_per_item - 1) / cols_per_item;
-    const int64_t items = (int64_t)counts[1] * ncg;
-    for (int64_t item = (int64_t)blockIdx.x * kWaves + wave; item < items; item += (int64_t)gridDim.x * kWaves) {
-        const int64_t s = item / ncg;
-        const int64_t c0 = (item % ncg) * cols_per_item + (int64_t)lane * kCols;   // D % 8 == 0 when VEC
-        if (c0 >= D) continue;
-        const int64_t j0 = run_start[s];
-        const int2 r = rng[skeys[j0]];
-        const int64_t hi = (int64_t)r.x + r.y;
-        const int cnt = (int)(j0 + kRowsPerPartial < hi ? kRowsPerPartial : hi - j0);
-        float part[kCols];
+// Workgroups [0, run_waves): runs of ids of more than kDirect occurrences; then one per output row, which writes it
+// unless the runs do.
+template <bool FEW, int G>
+__global__ __launch_bounds__(kEmbThreads) void emb_rows_kernel(const uint16_t* __restrict__ grad, int64_t D, int64_t V,
+                                                               const Ent* __restrict__ ent,
+                                                               const int2* __restrict__ info, int64_t padding_idx,
+                                                               float scale, int scale_mode, uint16_t* __restrict__ out,
+                                                               int run_waves, int steps, int* __restrict__ counts,
+                                                               int32_t* __restrict__ short_list,
+                                                               int32_t* __restrict__ long_list,
+                                                               float* __restrict__ parts) {
+    if ((int)blockIdx.x < run_waves) {
+        const int b = (int)blockIdx.x;
+        constexpr int kBlock = FEW ? kFewBlock : kRunBlock;
+        const int step = b % steps;
+        const int64_t valid = counts[2];
+        for (int64_t p0 = (int64_t)(b / steps) * kBlock; p0 < valid; p0 += (int64_t)(run_waves / steps) * kBlock)
+            sum_runs<FEW>(p0, step, step == steps - 1, grad, D, ent, padding_idx, scale, scale_mode, valid, out, counts,
+                          short_list, long_list, parts);
+        return;
+    }
+    // Row of workgroup b (run_waves is a multiple of 8: workgroup b runs on XCD b mod 8): each XCD takes kSpan consecutive
+    // rows of every 8 kSpan
+    const uint32_t b = blockIdx.x - run_waves;
+    const int64_t t = (int64_t)(b & ~(8u * kSpan - 1)) + (b & 7) * kSpan + ((b >> 3) & (kSpan - 1));
+    if (t >= V) return;
+    const int lane = threadIdx.x, ng = (int)(D / 8);
+    const int2 r = info[t];
+    uint16_t* orow = out + t * D;
+    const bool wide = D % 8 == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0;
+    if (r.y == 0 || t == padding_idx) {
+        for (int gi = lane; gi < ng; gi += kEmbThreads) row_store8(orow, wide, ng * 16, gi * 16, u4{0u, 0u, 0u, 0u});
+        if (ng * 8 + lane < D) orow[ng * 8 + lane] = 0;
+    } else if (r.y == 1) {
+        const int at[1] = {r.x};
+        sum_direct<FEW, G, 1>(at, 1, grad, D, scale, scale_mode, wide, orow);
+    } else if (r.y <= kDirect) {
+        const int pos = lane < r.y ? ent[r.x + lane].pos : 0;
+        int at[kDirect];
 #pragma unroll
-        for (int k = 0; k < kCols; ++k) part[k] = 0.0f;
-        if (VEC) {
-            u4 x[kRowsPerPartial];
-#pragma unroll
-            for (int u = 0; u < kRowsPerPartial; ++u)
-                if (u < cnt) x[u] = *reinterpret_cast<const u4*>(grad + (int64_t)spos[j0 + u] * D + c0);
-#pragma unroll
-            for (int u = 0; u < kRowsPerPartial; ++u) {
-                if (u < cnt) {
-#pragma unroll
-                    for (int k = 0; k < kCols; ++k)
-                        part[k] = part[k] + grad_elem((uint16_t)(x[u][k >> 1] >> ((k & 1) * 16)), scale, scale_mode);
-                }
-            }
-        } else {
-            uint16_t x[kRowsPerPartial];
-#pragma unroll
-            for (int u = 0; u < kRowsPerPartial; ++u)
-                if (u < cnt) x[u] = grad[(int64_t)spos[j0 + u] * D + c0];
-#pragma unroll
-            for (int u = 0; u < kRowsPerPartial; ++u)
-                if (u < cnt) part[0] = part[0] + grad_elem(x[u], scale, scale_mode);
-        }
-        float* dst = parts + s * D + c0;
-#pragma unroll
-        for (int k = 0; k < kCols; ++k) dst[k] = part[k];
+        for (int u = 0; u < kDirect; ++u) at[u] = __builtin_amdgcn_readlane(pos, u);
+        sum_direct<FEW, G, kDirect>(at, r.y, grad, D, scale, scale_mode, wide, orow);
     }
 }
 
-// Heavy tokens, pass 2: each (heavy token, 64 columns) is an item, one column per lane, whose partials are added in
-// run order -- the order of the rows kernel and of aten -- and rounded to the bf16 row.
-//   - tokens of more than kWaveChainRuns runs (long_list): workgroup g takes the items g, g + G, ...; per batch its
-//     waves load the token's next kChainRows partials into LDS (kChainDepth loads in flight per lane), then wave 0
-//     adds them to its accumulator;
-//   - the others (heavy_list): wave w of the grid takes the items w, w + W, ..., loads all of the token's partials
-//     at once and adds them in registers, with no barrier.
-__global__ __launch_bounds__(kWave * kChainWaves) void emb_heavy_chain_kernel(const float* __restrict__ parts,
-                                                                             int64_t D,
-                                                                             const int2* __restrict__ rng,
-                                                                             const int32_t* __restrict__ heavy_list,
-                                                                             const int32_t* __restrict__ heavy_base,
-                                                                             const int32_t* __restrict__ long_list,
-                                                                             const int32_t* __restrict__ long_base,
-                                                                             const int* __restrict__ counts,
-                                                                             float scale, int scale_mode,
-                                                                             uint16_t* __restrict__ out) {
+// The sum of n partials of one column in LDS rows 0 .. n - 1, added in order to acc, 16 reads in flight.
+template <bool FEW>
+__device__ __forceinline__ float chain_rows(float acc, const float (*buf)[kWave], int n, int lane) {
+    for (int k0 = 0; k0 < n; k0 += 16) {
+        float y[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) y[i] = buf[k0 + i][lane];
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+            if (k0 + i < n) acc = add_part<FEW>(acc, y[i]);
+    }
+    return acc;
+}
+
+// The ids of several runs: each (id, 64 columns) is an item, one column per lane, whose run partials are added in run
+// order -- aten's order -- and rounded to the bf16 row.
+//   - ids of more than kWaveChainRuns runs (long_list): workgroup g takes the items g, g + G, ...; per batch its waves
+//     load the id's next kChainRows partials into LDS (kChainDepth loads in flight per lane), then wave 0 adds them to
+//     its accumulator;
+//   - the others (short_list): wave w of the grid takes the items w, w + W, ..., loads all of the id's partials at once
+//     and adds them in registers, with no barrier.
+// The lists hold the ids' first sorted places.
+__global__ __launch_bounds__(kWave * kChainWaves) void emb_chain_kernel(const float* __restrict__ parts, int64_t D,
+                                                                       const Ent* __restrict__ ent,
+                                                                       const int32_t* __restrict__ short_list,
+                                                                       const int32_t* __restrict__ long_list,
+                                                                       const int* __restrict__ counts, float scale,
+                                                                       int scale_mode, uint16_t* __restrict__ out) {
     __shared__ float buf[kChainRows][kWave];
-    const int wave = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x & (kWave - 1);
     const int64_t ncg = (D + kWave - 1) / kWave;
-    const int64_t long_items = (int64_t)counts[2] * ncg;
+    const int64_t long_items = (int64_t)counts[1] * ncg;
     for (int64_t item = blockIdx.x; item < long_items; item += gridDim.x) {
-        const int h = (int)(item / ncg);
-        const int64_t col = (item % ncg) * kWave + lane;
-        const bool valid = col < D;
-        const int64_t t = long_list[h];
-        const int64_t nrun = ((int64_t)rng[t].y + kRowsPerPartial - 1) / kRowsPerPartial;
-        const float* src = parts + (int64_t)long_base[h] * D + col;
+        const int64_t c = (item % ncg) * kWave + lane;
+        const bool valid = c < D;
+        const Ent e = ent[long_list[item / ncg]];
+        const int64_t nrun = ((int64_t)e.n + kRowsPerPartial - 1) / kRowsPerPartial;
+        const float* src = parts + run_slot<false>(e.lo, e.lo) * D + c;
         float acc = 0.0f;
         for (int64_t b = 0; b < nrun; b += kChainRows) {
             float x[kChainDepth];
@@ -512,30 +549,19 @@ __global__ __launch_bounds__(kWave * kChainWaves) void emb_heavy_chain_kernel(co
 #pragma unroll
             for (int i = 0; i < kChainDepth; ++i) buf[wave + kChainWaves * i][lane] = x[i];
             __syncthreads();
-            if (wave == 0) {                                   // LDS reads issued 16 at a time, added in order
-                const int n = (int)(nrun - b < kChainRows ? nrun - b : kChainRows);
-                for (int k0 = 0; k0 < n; k0 += 16) {
-                    float y[16];
-#pragma unroll
-                    for (int i = 0; i < 16; ++i) y[i] = buf[k0 + i][lane];
-#pragma unroll
-                    for (int i = 0; i < 16; ++i)
-                        if (k0 + i < n) acc = acc + y[i];
-                }
-            }
+            if (wave == 0) acc = chain_rows<false>(acc, buf, (int)(nrun - b < kChainRows ? nrun - b : kChainRows), lane);
             __syncthreads();
         }
-        if (wave == 0 && valid) out[t * D + col] = finish(acc, scale, scale_mode);
+        if (wave == 0 && valid) out[(int64_t)e.id * D + c] = finish(acc, scale, scale_mode);
     }
     const int64_t items = (int64_t)counts[0] * ncg;
     for (int64_t item = (int64_t)blockIdx.x * kChainWaves + wave; item < items;
          item += (int64_t)gridDim.x * kChainWaves) {
-        const int h = (int)(item / ncg);
-        const int64_t col = (item % ncg) * kWave + lane;
-        if (col >= D) continue;
-        const int64_t t = heavy_list[h];
-        const int nrun = (rng[t].y + kRowsPerPartial - 1) / kRowsPerPartial;
-        const float* src = parts + (int64_t)heavy_base[h] * D + col;
+        const int64_t c = (item % ncg) * kWave + lane;
+        if (c >= D) continue;
+        const Ent e = ent[short_list[item / ncg]];
+        const int nrun = (e.n + kRowsPerPartial - 1) / kRowsPerPartial;
+        const float* src = parts + run_slot<false>(e.lo, e.lo) * D + c;
         float x[kWaveChainRuns];
 #pragma unroll
         for (int k = 0; k < kWaveChainRuns; ++k) x[k] = k < nrun ? src[(int64_t)k * D] : 0.0f;
@@ -543,7 +569,76 @@ __global__ __launch_bounds__(kWave * kChainWaves) void emb_heavy_chain_kernel(co
 #pragma unroll
         for (int k = 0; k < kWaveChainRuns; ++k)
             if (k < nrun) acc = acc + x[k];
-        out[t * D + col] = finish(acc, scale, scale_mode);
+        out[(int64_t)e.id * D + c] = finish(acc, scale, scale_mode);
+    }
+}
+
+// The same for few indices, where any occurrence may start a run, and an id has at most kFewRuns of them.
+//   - ids of more than kWaveChainRuns occurrences: the workgroup first lists their runs in LDS (each wave finds the
+//     starts among 64 places at a time, its first one's number is the runs of the waves and rounds before it), loads all
+//     of the partials, and wave 0 adds them;
+//   - the others: one wave's lanes find the starts.
+__global__ __launch_bounds__(kWave * kChainWaves) void emb_chain_few_kernel(const float* __restrict__ parts, int64_t D,
+                                                                           const Ent* __restrict__ ent,
+                                                                           const int32_t* __restrict__ short_list,
+                                                                           const int32_t* __restrict__ long_list,
+                                                                           const int* __restrict__ counts, float scale,
+                                                                           int scale_mode, uint16_t* __restrict__ out) {
+    __shared__ float buf[kFewRuns][kWave];
+    __shared__ int run[kFewRuns], found[kChainWaves];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x & (kWave - 1);
+    const int64_t ncg = (D + kWave - 1) / kWave;
+    auto starts_at = [&](const Ent& e, int p) {
+        return p < e.lo + e.n && run_starts<true>(p, e.lo, ent[p].pos, p > e.lo ? ent[p - 1].pos : 0);
+    };
+    const int64_t long_items = (int64_t)counts[1] * ncg;
+    for (int64_t item = blockIdx.x; item < long_items; item += gridDim.x) {
+        const int64_t c = (item % ncg) * kWave + lane;
+        const bool valid = c < D;
+        const Ent e = ent[long_list[item / ncg]];
+        int nrun = 0;
+        for (int b = 0; b < e.n; b += kWave * kChainWaves) {
+            const int p = e.lo + b + (int)threadIdx.x;
+            const uint64_t m = __ballot(starts_at(e, p));
+            if (lane == 0) found[wave] = __builtin_popcountll(m);
+            __syncthreads();
+            int at = nrun;
+            for (int w = 0; w < kChainWaves; ++w) {
+                at += w < wave ? found[w] : 0;
+                nrun += found[w];
+            }
+            if (m >> lane & 1) run[at + __builtin_popcountll(m & ((1ull << lane) - 1))] = p;
+            __syncthreads();
+        }
+        constexpr int kDepth = kFewRuns / kChainWaves;
+        float x[kDepth];
+#pragma unroll
+        for (int i = 0; i < kDepth; ++i) {
+            const int k = wave + kChainWaves * i;
+            x[i] = (k < nrun && valid) ? parts[(int64_t)run[k < nrun ? k : 0] * D + c] : 0.0f;
+        }
+#pragma unroll
+        for (int i = 0; i < kDepth; ++i) buf[wave + kChainWaves * i][lane] = x[i];
+        __syncthreads();
+        if (wave == 0 && valid)
+            out[(int64_t)e.id * D + c] = finish(chain_rows<true>(0.0f, buf, nrun, lane), scale, scale_mode);
+        __syncthreads();
+    }
+    const int64_t items = (int64_t)counts[0] * ncg;
+    for (int64_t item = (int64_t)blockIdx.x * kChainWaves + wave; item < items;
+         item += (int64_t)gridDim.x * kChainWaves) {
+        const int64_t c = (item % ncg) * kWave + lane;
+        const Ent e = ent[short_list[item / ncg]];
+        const uint64_t m = __ballot(starts_at(e, e.lo + lane));
+        const float* src = parts + (int64_t)e.lo * D + c;
+        float x[kWaveChainRuns];
+#pragma unroll
+        for (int k = 0; k < kWaveChainRuns; ++k) x[k] = (m >> k & 1) && c < D ? src[(int64_t)k * D] : 0.0f;
+        float acc = 0.0f;
+#pragma unroll
+        for (int k = 0; k < kWaveChainRuns; ++k)
+            if (m >> k & 1) acc = add_part<true>(acc, x[k]);
+        if (c < D) out[(int64_t)e.id * D + c] = finish(acc, scale, scale_mode);
     }
 }
 
@@ -574,22 +669,21 @@ inline size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 // Whether the occurrences are put in order by emb_bucket_kernel (else by the library sort).
 bool bucketed(int64_t R, int64_t V) { return R <= kBucketRows && V <= kBucketVocab; }
 
-// Workspace: sorted keys and positions (R each), rng (V), the three counters, the two lists of heavy tokens and their
-// first run slots (at most R / 21 each), the run starts and the fp32 partials (R / 7 slots, D each), then, for the
-// library sort, its keys and positions (R each) and its temporary storage.
+// Workspace: ent (R), info (V), the three counters (ids in short_list and in long_list, ids inside the vocabulary), the
+// two lists (ids of at least 11 occurrences, of more than kDirect for few indices), the fp32 partials (R / 4 slots, R for
+// few indices, D each), then, for the library sort, its keys and positions and their sorted copies (R each) and its
+// temporary storage.
 struct EmbWorkspace {
+    Ent* ent;
+    int2* info;
+    int* counts;
+    int32_t* short_list;
+    int32_t* long_list;
+    float* parts;
     uint32_t* keys;
     int32_t* vals;
     uint32_t* skeys;
     int32_t* svals;
-    int2* rng;
-    int* counts;
-    int32_t* heavy_list;
-    int32_t* heavy_base;
-    int32_t* long_list;
-    int32_t* long_base;
-    int32_t* run_start;
-    float* parts;
     void* temp;
     size_t temp_bytes;
     size_t total;
@@ -604,20 +698,20 @@ EmbWorkspace emb_workspace(void* base, int64_t R, int64_t D, int64_t V) {
         off += align256(bytes > 0 ? bytes : 1);
         return q;
     };
-    const size_t r = (size_t)R, heavy = (size_t)(R / (kHeavyRows + 1)), slots = (size_t)(R / 7);
-    w.skeys = reinterpret_cast<uint32_t*>(take(sizeof(uint32_t) * r));
-    w.svals = reinterpret_cast<int32_t*>(take(sizeof(int32_t) * r));
-    w.rng = reinterpret_cast<int2*>(take(sizeof(int2) * (size_t)V));
+    const bool few = R < kSortMinRows;
+    const size_t r = (size_t)R, listed = r / (few ? kDirect + 1 : kRowsPerPartial + 1);
+    const size_t slots = few ? r : r / kSlotSpan + 1;
+    w.ent = reinterpret_cast<Ent*>(take(sizeof(Ent) * r));
+    w.info = reinterpret_cast<int2*>(take(sizeof(int2) * (size_t)V));
     w.counts = reinterpret_cast<int*>(take(3 * sizeof(int)));
-    w.heavy_list = reinterpret_cast<int32_t*>(take(sizeof(int32_t) * heavy));
-    w.heavy_base = reinterpret_cast<int32_t*>(take(sizeof(int32_t) * heavy));
-    w.long_list = reinterpret_cast<int32_t*>(take(sizeof(int32_t) * heavy));
-    w.long_base = reinterpret_cast<int32_t*>(take(sizeof(int32_t) * heavy));
-    w.run_start = reinterpret_cast<int32_t*>(take(sizeof(int32_t) * slots));
+    w.short_list = reinterpret_cast<int32_t*>(take(sizeof(int32_t) * listed));
+    w.long_list = reinterpret_cast<int32_t*>(take(sizeof(int32_t) * listed));
     w.parts = reinterpret_cast<float*>(take(sizeof(float) * slots * (size_t)D));
     if (!bucketed(R, V)) {
         w.keys = reinterpret_cast<uint32_t*>(take(sizeof(uint32_t) * r));
         w.vals = reinterpret_cast<int32_t*>(take(sizeof(int32_t) * r));
+        w.skeys = reinterpret_cast<uint32_t*>(take(sizeof(uint32_t) * r));
+        w.svals = reinterpret_cast<int32_t*>(take(sizeof(int32_t) * r));
         w.temp_bytes = sort_temp_bytes(R);
         w.temp = take(w.temp_bytes);
     }
@@ -625,27 +719,43 @@ EmbWorkspace emb_workspace(void* base, int64_t R, int64_t D, int64_t V) {
     return w;
 }
 
-// The rows kernel with as many column groups per lane and step as the row needs, at most 6 (D 3072).
+struct RowsCall {
+    const uint16_t* grad;
+    int64_t R, D, V, padding_idx;
+    float scale;
+    int scale_mode;
+    uint16_t* out;
+    size_t lds;
+    hipStream_t st;
+};
+
+// The rows launch, with as many column groups per lane as the row needs, at most 6 (D 3072).
 template <bool FEW, int G>
-void launch_rows_g(int64_t D, int64_t V, size_t lds, hipStream_t st, const uint16_t* grad, const EmbWorkspace& w,
-                   int64_t padding_idx, float scale, int scale_mode, uint16_t* out) {
-    hipLaunchKernelGGL((emb_rows_kernel<FEW, G>), dim3((unsigned)V), dim3(kEmbThreads), lds, st, grad, D, w.svals,
-                       w.rng, padding_idx, scale, scale_mode, out, w.counts, w.heavy_list, w.heavy_base,
-                       w.long_list, w.long_base, w.run_start);
+void launch_rows_g(const RowsCall& c, const EmbWorkspace& w) {
+    const int64_t steps = (c.D / 8 + kEmbThreads - 1) / kEmbThreads, step_waves = steps > 0 ? steps : 1;
+    int64_t run_waves = 0;
+    if (c.R > kDirect) {
+        constexpr int kBlock = FEW ? kFewBlock : kRunBlock;
+        const int64_t blocks = (c.R + kBlock - 1) / kBlock, most = kMaxWaves / step_waves;      // steps <= 32,768
+        run_waves = ((blocks < most ? blocks : most) + 7) / 8 * 8 * step_waves;
+    }
+    const int64_t rows = (c.V + 8 * kSpan - 1) / (8 * kSpan) * (8 * kSpan);
+    hipLaunchKernelGGL((emb_rows_kernel<FEW, G>), dim3((unsigned)(run_waves + rows)), dim3(kEmbThreads), c.lds, c.st,
+                       c.grad, c.D, c.V, w.ent, w.info, c.padding_idx, c.scale, c.scale_mode, c.out, (int)run_waves,
+                       (int)step_waves, w.counts, w.short_list, w.long_list, w.parts);
 }
 
 template <bool FEW>
-void launch_rows(int64_t D, int64_t V, size_t lds, hipStream_t st, const uint16_t* grad, const EmbWorkspace& w,
-                 int64_t padding_idx, float scale, int scale_mode, uint16_t* out) {
-    const int64_t need = (D / 8 + kEmbThreads - 1) / kEmbThreads;          // groups per lane
+void launch_rows(const RowsCall& c, const EmbWorkspace& w) {
+    const int64_t need = (c.D / 8 + kEmbThreads - 1) / kEmbThreads;          // groups per lane
     const int64_t steps = (need + 5) / 6;
     switch (need > 0 ? (need + steps - 1) / steps : 1) {
-        case 1: return launch_rows_g<FEW, 1>(D, V, lds, st, grad, w, padding_idx, scale, scale_mode, out);
-        case 2: return launch_rows_g<FEW, 2>(D, V, lds, st, grad, w, padding_idx, scale, scale_mode, out);
-        case 3: return launch_rows_g<FEW, 3>(D, V, lds, st, grad, w, padding_idx, scale, scale_mode, out);
-        case 4: return launch_rows_g<FEW, 4>(D, V, lds, st, grad, w, padding_idx, scale, scale_mode, out);
-        case 5: return launch_rows_g<FEW, 5>(D, V, lds, st, grad, w, padding_idx, scale, scale_mode, out);
-        default: return launch_rows_g<FEW, 6>(D, V, lds, st, grad, w, padding_idx, scale, scale_mode, out);
+        case 1: return launch_rows_g<FEW, 1>(c, w);
+        case 2: return launch_rows_g<FEW, 2>(c, w);
+        case 3: return launch_rows_g<FEW, 3>(c, w);
+        case 4: return launch_rows_g<FEW, 4>(c, w);
+        case 5: return launch_rows_g<FEW, 5>(c, w);
+        default: return launch_rows_g<FEW, 6>(c, w);
     }
 }
 
@@ -672,12 +782,12 @@ int z1_embedding_backward(const int64_t* ids, const uint16_t* grad, int64_t R, i
     if (bucketed(R, V)) {
         int kb = kMinBucketBits;
         while ((((V - 1) >> (kGranuleBits + kb)) + 1) << kGranuleBits > kMaxLocal / 2 && kb < kMaxBucketBits) ++kb;
-        hipLaunchKernelGGL(emb_bucket_kernel, dim3(1u << kb), dim3(kBucketThreads), 0, st, ids, (int)R, (int)V, kb,
-                           w.svals, w.skeys, w.rng, w.counts);
+        hipLaunchKernelGGL(emb_bucket_kernel, dim3(1u << kb), dim3(kBucketThreads), 0, st, ids, (int)R, (int)V, kb, w.ent,
+                           w.info, w.counts);
     } else {
+        const dim3 per_row((unsigned)((R + 255) / 256));
         if (R > 0) {
-            hipLaunchKernelGGL(emb_keys_kernel, dim3((unsigned)((R + 255) / 256)), dim3(256), 0, st, ids, R, V, w.keys,
-                               w.vals);
+            hipLaunchKernelGGL(emb_keys_kernel, per_row, dim3(256), 0, st, ids, R, V, w.keys, w.vals);
             e = hipGetLastError();
             if (e != hipSuccess) return (int)e;
             size_t tb = w.temp_bytes;
@@ -686,36 +796,37 @@ int z1_embedding_backward(const int64_t* ids, const uint16_t* grad, int64_t R, i
             e = sort_pairs(w.temp, tb, w.keys, w.skeys, w.vals, w.svals, R, end_bit, capturing(st), st);
             if (e != hipSuccess) return (int)e;
         }
-        hipLaunchKernelGGL(emb_row_ranges_kernel, dim3((unsigned)((V + 255) / 256)), dim3(256), 0, st, w.skeys, R, V,
-                           w.rng, w.counts);
+        hipLaunchKernelGGL(emb_row_ranges_kernel, dim3((unsigned)((V + 255) / 256)), dim3(256), 0, st, w.skeys, w.svals,
+                           R, V, w.info, w.counts);
+        e = hipGetLastError();
+        if (e != hipSuccess) return (int)e;
+        if (R > 0)
+            hipLaunchKernelGGL(emb_entries_kernel, per_row, dim3(256), 0, st, w.skeys, w.svals, R, V, w.info, w.ent);
     }
     e = hipGetLastError();
     if (e != hipSuccess) return (int)e;
-    const int vec = (D % 8 == 0) && ((reinterpret_cast<uintptr_t>(grad) | reinterpret_cast<uintptr_t>(out)) & 15) == 0;
     int dev = 0;
     e = hipGetDevice(&dev);
     if (e != hipSuccess) return (int)e;
-    size_t lds = 0;
-    const int rc = z1detail::occupancy_lds(dev, kEmbWgPerCu, &lds);
+    RowsCall c{grad, R, D, V, padding_idx, scale, scale_mode, out, 0, st};
+    const int rc = z1detail::occupancy_lds(dev, kEmbWgPerCu, &c.lds);
     if (rc) return rc;
-    // aten's kernel for few indices: its order, no heavy passes (nothing is listed for them)
-    if (R < kSortMinRows) launch_rows<true>(D, V, lds, st, grad, w, padding_idx, scale, scale_mode, out);
-    else launch_rows<false>(D, V, lds, st, grad, w, padding_idx, scale, scale_mode, out);
+    const bool few = R < kSortMinRows;                  // aten's kernel for few indices: its order
+    if (few) launch_rows<true>(c, w);
+    else launch_rows<false>(c, w);
     e = hipGetLastError();
     if (e != hipSuccess) return (int)e;
-    if (vec)
-        hipLaunchKernelGGL(emb_heavy_parts_kernel<1>, dim3(kPartsGrid), dim3(kPartsThreads), 0, st, grad, D, w.svals,
-                           w.skeys, w.rng, w.run_start, w.counts, scale, scale_mode, w.parts);
+    // the most items the lists can hold
+    const int64_t items = R / (few ? kDirect + 1 : kRowsPerPartial + 1) * ((D + kWave - 1) / kWave);
+    if (items == 0) return Z1_OK;
+    const dim3 grid((unsigned)(items < kChainGrid ? items : kChainGrid)), threads(kWave * kChainWaves);
+    if (few)
+        hipLaunchKernelGGL(emb_chain_few_kernel, grid, threads, 0, st, w.parts, D, w.ent, w.short_list, w.long_list,
+                           w.counts, scale, scale_mode, out);
     else
-        hipLaunchKernelGGL(emb_heavy_parts_kernel<0>, dim3(kPartsGrid), dim3(kPartsThreads), 0, st, grad, D, w.svals,
-                           w.skeys, w.rng, w.run_start, w.counts, scale, scale_mode, w.parts);
-    e = hipGetLastError();
-    if (e != hipSuccess) return (int)e;
-    hipLaunchKernelGGL(emb_heavy_chain_kernel, dim3(kChainGrid), dim3(kWave * kChainWaves), 0, st, w.parts, D,
-                       w.rng, w.heavy_list, w.heavy_base, w.long_list, w.long_base, w.counts, scale, scale_mode,
-                       out);
-    e = hipGetLastError();
-    return e == hipSuccess ? Z1_OK : (int)e;
+        hipLaunchKernelGGL(emb_chain_kernel, grid, threads, 0, st, w.parts, D, w.ent, w.short_list, w.long_list, w.counts,
+                           scale, scale_mode, out);
+    return (int)hipGetLastError();
 }
 
 }  // extern "C"

@@ -104,6 +104,30 @@ def test_matches_aten_at_3072_rows_or_fewer(pkg, dev, D):
         assert np.array_equal(bits(got2), bits(ref2)) and np.array_equal(bits(got3), bits(ref3)), R
 
 
+@pytest.mark.parametrize('V', [1023, 1024, 1025, 2049])
+@pytest.mark.parametrize('few', [True, False])
+@pytest.mark.parametrize('D', [3080, 520, 5])
+def test_occurrence_counts(pkg, dev, D, few, V):
+    """Ids with as many occurrences as the parts of the work split at -- 4 and 5 (the row's own wave / by runs), 10 and 11
+    (one run / several), 32 and 33, 320 and 321 (chained by a wave / a workgroup), 1200 -- ids at both ends of tables
+    around a multiple of the rows one round of XCDs takes, an output off the 16-byte boundary, a heavy padding row.
+    Bit-exact against aten."""
+    from faster_yoco_amd import embedding
+    rng = np.random.default_rng(D + V)
+    counts = [1, 2, 3, 4, 5, 9, 10, 11, 12, 16, 17, 20, 21, 30, 31, 32, 33, 64, 65, 320, 321, 1200]
+    where = rng.choice(np.arange(1, V - 1), len(counts), replace=False)
+    ids = np.concatenate([np.repeat(where, counts), [0, V - 1, V - 1], rng.integers(0, V, 0 if few else 2000)])
+    ids = torch.from_numpy(rng.permutation(ids).astype(np.int64)).to(dev)
+    assert (ids.numel() <= 3072) == few
+    g = (torch.randn(ids.numel(), D, device=dev) * 1e-2).to(torch.bfloat16)
+    for pad in (-1, int(where[-1]), 0):
+        ref = torch.ops.aten.embedding_dense_backward(g, ids, V, pad, False)
+        out = torch.full((V * D + 1,), 7.0, dtype=torch.bfloat16, device=dev)[pad % 2:][:V * D].view(V, D)
+        embedding.embedding_dense_backward(g, ids, V, pad, out=out)
+        torch.cuda.synchronize()
+        assert np.array_equal(bits(out), bits(ref)), pad
+
+
 @pytest.mark.parametrize('R', [1, 63, 1024, 1025, 16384, 16385, 20000, 49152, 49153])
 @pytest.mark.parametrize('V', [1, 2, 513, 65537, 524288, 524289])
 def test_order_of_occurrences(pkg, dev, R, V):
