@@ -21,8 +21,7 @@
 //     lookups that start each wave, 2.175-2.177 against 2.185-2.188 ms per C2 update.
 //   * Each lane moves one 128-bit group per fp32 array (and 64 bits of bf16); a wave instruction covers 1 KiB
 //     (fp32) or 512 B (bf16) of contiguous bytes, with nontemporal hints (streams far larger than L2 and MALL).
-//     The last, partial chunk of a row (and rows whose pointers are not aligned for the vector path) run an
-//     element-wise loop.
+//     The last, partial chunk of a row (and rows off their element boundaries) run an element-wise loop.
 //   * The norm uses the same table and a FIXED grid of Z1_NORM_PARTIALS workgroups of 4 waves, split by XCD: the
 //     256 workgroups dispatched to one XCD stride through that XCD's eighth of the chunks, 1024 contiguous
 //     elements per workgroup step.  FP64 accumulation of the exact squares per lane, a wave64 xor-butterfly and
@@ -90,8 +89,8 @@ struct Row {
     uint16_t* p16;
     int64_t n;
     int64_t chunk0;
-    int32_t vec;        // bit 0: g aligned for the vector path; bit 1: p, m, v, p16 aligned as well
-    int32_t pmv_aligned;    // p, m, v, p16 aligned for the vector path (vec's bit 1 needs g aligned too)
+    int32_t vec;        // bit 0: g on its element boundary; bit 1: p, m, v, p16 as well
+    int32_t pmv_aligned;    // p, m, v, p16 on their element boundaries (vec's bit 1 needs g there too)
 };
 static_assert(sizeof(Row) == 64, "row layout");
 
@@ -107,19 +106,29 @@ struct AdamK {
 // The update's big stores go out through st_stream below, which adds the system-scope bits.
 #define Z1_GLOBAL __attribute__((address_space(1)))
 
+//
+// The vectors need no more than their elements' alignment (fp32 4, bf16 2 bytes): gfx950 loads and stores 8 and 16 bytes
+// at any address, in the same instructions, so a parameter packed behind an odd-sized one keeps the vector path; its
+// lines that straddle two waves are fetched twice.  Measured on the drop-in update of 13.7M parameters in 26 odd-sized
+// tensors, 8 contributions in slots at odd offsets, against the element-wise paths these rows took: phase sums 51 against
+// 104 us, Adam 78 against 117 us.
+template <typename T>
+struct AnyAlign;
+template <>
+struct AnyAlign<f4> { typedef f4 type __attribute__((aligned(4))); };
+template <>
+struct AnyAlign<u2> { typedef u2 type __attribute__((aligned(2))); };
+template <>
+struct AnyAlign<u4> { typedef u4 type __attribute__((aligned(2))); };
+
 template <typename T>
 __device__ __forceinline__ T ld(const T* p) {
-    return __builtin_nontemporal_load((const Z1_GLOBAL T*)p);
+    return __builtin_nontemporal_load((const Z1_GLOBAL typename AnyAlign<T>::type*)p);
 }
 
 template <typename T>
 __device__ __forceinline__ T ld_keep(const T* p) {       // ordinary load: allocates in L2 and the MALL
-    return *(const Z1_GLOBAL T*)p;
-}
-
-template <typename T>
-__device__ __forceinline__ void st(T* p, T x) {
-    __builtin_nontemporal_store(x, (Z1_GLOBAL T*)p);
+    return *(const Z1_GLOBAL typename AnyAlign<T>::type*)p;
 }
 
 // The update's streaming stores (Adam's p, m, v, BF16 copy and FP32 gradient outputs; the owner sum's average; the
@@ -137,7 +146,13 @@ __device__ __forceinline__ void st_stream(float* base, int bytes, int off, f4 x)
     const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(base, 0, bytes, 0x00020000);
     __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, x), r, off, 0, kStreamStorePolicy);
 }
+// (buffer stores want dword addresses: four bf16 at an odd element go out as a nontemporal global store)
 __device__ __forceinline__ void st_stream(uint16_t* base, int bytes, int off, u2 x) {
+    if (reinterpret_cast<uintptr_t>(base) & 3) {
+        __builtin_nontemporal_store((AnyAlign<u2>::type)x,
+                                    (Z1_GLOBAL AnyAlign<u2>::type*)(reinterpret_cast<char*>(base) + off));
+        return;
+    }
     const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(base, 0, bytes, 0x00020000);
     __builtin_amdgcn_raw_buffer_store_b64(x, r, off, 0, kStreamStorePolicy);
 }
@@ -215,7 +230,7 @@ __device__ __forceinline__ float load_g1(const void* g, int64_t i) {
 template <int GDT, int MODE, bool GOUT>
 __device__ __forceinline__ void adam_chunk(const Row& r, float* go, int64_t base, int lane, float f, const AdamK& k) {
     const int64_t rem = r.n - base;
-    if (rem >= kChunk && (r.vec & kVecAll) && (!GOUT || (reinterpret_cast<uintptr_t>(go) & 15) == 0)) {
+    if (rem >= kChunk && (r.vec & kVecAll) && (!GOUT || (reinterpret_cast<uintptr_t>(go) & 3) == 0)) {
         f4 g[kGroups], p[kGroups], m[kGroups], v[kGroups];
 #pragma unroll
         for (int u = 0; u < kGroups; ++u) {
@@ -447,7 +462,7 @@ __device__ __forceinline__ void sumsq_chunk(const Row& r, int64_t c, int lane, d
 
 // The chunks of one wave below `end` into acc, in order.  FP32: chunks c, c + step, c + 2 step, ... (one 128-bit
 // group per lane each).  BF16: runs of kSumsqBf16Span adjacent chunks starting at c, c + step, ...: a run inside one
-// row, whole and 16-byte aligned, is kSumsqBf16Span / 2 128-bit loads per lane (8 elements each: the run's
+// row and whole is kSumsqBf16Span / 2 128-bit loads per lane (8 elements each: the run's
 // lane-major order, one 1 KB load of the wave after the other); other runs are their chunks one after the other.
 // A BF16 chunk alone gives a wave 512 bytes per load, and the per-chunk latency then bounds the pass (188 us on
 // C2's size, 4.6 TB/s, even with two chunks' loads in flight); runs of 2, 4, 8 and 16 chunks measured 143, 135,
@@ -467,8 +482,7 @@ __device__ __forceinline__ void sumsq_range(const Row* __restrict__ rows, int nr
         if (GDT == Z1_BF16) {
             constexpr int S = kSumsqBf16Span, L = kSumsqBf16Span / 2;
             const uint16_t* g = static_cast<const uint16_t*>(r.g) + (c - r.chunk0) * kChunk;
-            const bool wide = c + (S - 1) < end && r.n - (c - r.chunk0) * kChunk >= S * kChunk && (r.vec & kVecG) &&
-                              (reinterpret_cast<uintptr_t>(g) & 15) == 0;
+            const bool wide = c + (S - 1) < end && r.n - (c - r.chunk0) * kChunk >= S * kChunk && (r.vec & kVecG);
             if (wide) {
                 const u4* q = reinterpret_cast<const u4*>(g) + lane;
                 u4 h[L];
@@ -590,9 +604,9 @@ constexpr int kSumVec = 4;                                    // elements per la
 constexpr int64_t kSumChunk = (int64_t)kWave * kSumVec;
 // The chunk grid is shifted by `shift` elements (0..kSumShiftMax): chunk c covers elements [c * kSumChunk - shift,
 // (c + 1) * kSumChunk - shift) of the call's range.  The host picks the shift that puts the chunk boundaries on
-// 128-byte lines of every stream (else on their 8-byte words), so a range that starts anywhere -- a CEReduce phase
-// bound, yoco/models/decoder/ce_reduce.py:178-183 -- keeps the vector path, and no line is shared by two chunks
-// (consecutive chunks run on different XCDs, whose L2s would each fetch a shared line).  A call always launches
+// 128-byte lines of the average, so that no line of it, nor of any stream at the same offset within a line, is shared by
+// two chunks (consecutive chunks run on different XCDs, whose L2s would each fetch a shared line): a range may start
+// anywhere -- a CEReduce phase bound, yoco/models/decoder/ce_reduce.py:178-183.  A call always launches
 // owner_sum_waves(n) chunks, enough for any shift; those past the end only write a zero partial.
 constexpr int64_t kSumShiftMax = 63;
 
@@ -729,7 +743,7 @@ __global__ __launch_bounds__(kRebindPerLaunch) void rebind_rows_kernel(Row* rows
     Row* r = rows + b.row[i];
     const uintptr_t pmv = reinterpret_cast<uintptr_t>(b.p[i]) | reinterpret_cast<uintptr_t>(b.m[i]) |
                           reinterpret_cast<uintptr_t>(b.v[i]);
-    const bool pmv_ok = (pmv & 15) == 0 && (reinterpret_cast<uintptr_t>(b.p16[i]) & 7) == 0;
+    const bool pmv_ok = (pmv & 3) == 0 && (reinterpret_cast<uintptr_t>(b.p16[i]) & 1) == 0;
     const bool ga = (reinterpret_cast<uintptr_t>(b.g[i]) & (uintptr_t)(b.g_align - 1)) == 0;
     r->g = b.g[i];
     r->p = b.p[i];
@@ -897,7 +911,7 @@ static void set_contig(z1_table* t) {
     const uintptr_t g0 = reinterpret_cast<uintptr_t>(r0.g), p0 = reinterpret_cast<uintptr_t>(r0.p),
                     m0 = reinterpret_cast<uintptr_t>(r0.m), v0 = reinterpret_cast<uintptr_t>(r0.v),
                     h0 = reinterpret_cast<uintptr_t>(r0.p16);
-    if ((g0 & (gsz == 4 ? 15 : 7)) || ((p0 | m0 | v0) & 15) || (h0 & 7)) return;
+    if ((g0 & (gsz - 1)) || ((p0 | m0 | v0) & 3) || (h0 & 1)) return;
     uintptr_t off = 0;                                 // elements before row i
     for (const Row& r : h) {
         if ((r.p16 != nullptr) != with16) return;
@@ -933,7 +947,7 @@ static int table_create(const z1_tensor* rows, int nrows, int g_dtype, z1_table*
     if (nrows < 0) return Z1_E_SIZE;
     if (nrows > 0 && !rows) return Z1_E_NULL;
     if (g_dtype != Z1_F32 && g_dtype != Z1_BF16) return Z1_E_DTYPE;
-    const uintptr_t galign = g_dtype == Z1_F32 ? 16 : 8;
+    const uintptr_t galign = g_dtype == Z1_F32 ? 4 : 2;
     std::vector<Row> h;
     h.reserve(nrows);
     std::vector<int64_t> first((size_t)nrows + 1);
@@ -956,7 +970,7 @@ static int table_create(const z1_tensor* rows, int nrows, int g_dtype, z1_table*
         r.p16 = t.p16;
         r.n = t.n;
         r.chunk0 = chunks;
-        r.pmv_aligned = aligned(t.p, 16) && aligned(t.m, 16) && aligned(t.v, 16) && (!t.p16 || aligned(t.p16, 8));
+        r.pmv_aligned = aligned(t.p, 4) && aligned(t.m, 4) && aligned(t.v, 4) && (!t.p16 || aligned(t.p16, 2));
         r.vec = aligned(t.g, galign) ? (kVecG | (r.pmv_aligned ? kVecAll : 0)) : 0;
         if (!t.p || !t.m || !t.v) has_pmv = 0;
         chunks += (t.n + kChunk - 1) / kChunk;
@@ -1053,7 +1067,7 @@ int z1_table_rebind(z1_table* table, const z1_tensor* rows, int nrows, void* str
     }
     RowBind b;
     memset(&b, 0, sizeof(b));
-    b.g_align = table->g_dtype == Z1_F32 ? 16 : 8;
+    b.g_align = table->g_dtype == Z1_F32 ? 4 : 2;
     hipStream_t s = static_cast<hipStream_t>(stream);
     table->contig = 0;                                 // until every rebind launch is enqueued
     for (int i = 0; i < nrows; ++i) {
@@ -1108,7 +1122,7 @@ int z1_table_set_grads(z1_table* table, const void* const* g, int nrows, void* s
     if (rc) return rc;
     GradBind b;
     b.count = 0;
-    b.g_align = table->g_dtype == Z1_F32 ? 16 : 8;
+    b.g_align = table->g_dtype == Z1_F32 ? 4 : 2;
     hipStream_t s = static_cast<hipStream_t>(stream);
     for (int i = 0; i < nrows; ++i) {
         if (table->dev_row[i] < 0) continue;
@@ -1372,25 +1386,16 @@ int64_t z1_owner_sum_workspace(int64_t n) {
     return Z1_NORM_PARTIALS + owner_sum_waves(n);   // the partials, then one per chunk
 }
 
-// Shift of the owner sum's chunk grid (owner_sum_kernel) for these streams, and whether the vector path applies:
-// when every bf16 stream lies at the same offset within a 128-byte line as out_avg, the chunk boundaries go on those
-// lines; else, when they share the offset within an 8-byte word, on the words; else the element-wise path.  The
-// FP32 sum (nullable) must then be 16-byte aligned at the same boundaries.
+// Shift of the owner sum's chunk grid (owner_sum_kernel) for these streams, and whether the vector path applies (every
+// stream on its element boundary): the chunk boundaries go on the 128-byte lines of out_avg, which are those of every
+// bf16 stream at the same offset within a line (the others' loads straddle lines).
 static int owner_sum_grid(const Srcs& s, int world, const uint16_t* out_avg, const float* out_sum, int64_t* shift) {
     const uintptr_t o = reinterpret_cast<uintptr_t>(out_avg);
+    uintptr_t odd = o;
+    for (int k = 0; k < world; ++k) odd |= reinterpret_cast<uintptr_t>(s.p[k]);
     *shift = 0;
-    if (o & 1) return 0;
-    uintptr_t diff = 0;
-    for (int k = 0; k < world; ++k) diff |= reinterpret_cast<uintptr_t>(s.p[k]) - o;
-    int64_t sh;
-    if ((diff & 127) == 0) sh = (int64_t)((o & 127) >> 1);
-    else if ((diff & 7) == 0) sh = (int64_t)((o & 7) >> 1);
-    else return 0;
-    if (out_sum) {
-        const uintptr_t f = reinterpret_cast<uintptr_t>(out_sum);
-        if ((f & 3) || (((f >> 2) - (uintptr_t)sh) & 3)) return 0;
-    }
-    *shift = sh;
+    if ((odd & 1) || (reinterpret_cast<uintptr_t>(out_sum) & 3)) return 0;
+    *shift = (int64_t)((o & 127) >> 1);
     return 1;
 }
 
@@ -1482,7 +1487,7 @@ int z1_scale_up(const uint16_t* g16, float* g32, const float* factor, int64_t n,
     if (!g16 || !g32 || !factor) return Z1_E_NULL;
     const int64_t chunks = (n + kPassChunk - 1) / kPassChunk;
     if (chunks > INT32_MAX) return Z1_E_SIZE;
-    const int vec = aligned(g16, 8) && aligned(g32, 16);
+    const int vec = aligned(g16, 2) && aligned(g32, 4);
     hipLaunchKernelGGL(scale_up_kernel, dim3((unsigned)chunks), dim3(kWave), 0, static_cast<hipStream_t>(stream),
                        g16, g32, factor, n, vec);
     return launch_status();
@@ -1494,7 +1499,7 @@ int z1_cast_bf16(const float* p32, uint16_t* p16, int64_t n, void* stream) {
     if (!p32 || !p16) return Z1_E_NULL;
     const int64_t chunks = (n + kPassChunk - 1) / kPassChunk;
     if (chunks > INT32_MAX) return Z1_E_SIZE;
-    const int vec = aligned(p32, 16) && aligned(p16, 8);
+    const int vec = aligned(p32, 4) && aligned(p16, 2);
     hipLaunchKernelGGL(cast_bf16_kernel, dim3((unsigned)chunks), dim3(kWave), 0, static_cast<hipStream_t>(stream),
                        p32, p16, n, vec);
     return launch_status();

@@ -520,6 +520,60 @@ def test_owner_sum_misaligned_ranges(pkg, dev, case):
     assert abs(float(nr.item()) - ex) <= 1e-6 * ex
 
 
+@pytest.mark.parametrize('n', [1, 3, 255, 256, 257, 70001])
+@pytest.mark.parametrize('world', [2, 8])
+def test_owner_sum_streams_each_at_its_own_offset(pkg, dev, n, world):
+    """Every stream at another element offset, even and odd (slots of an odd-sized gradient): the vector path, bit-exact,
+    the norm within an fp32 ulp; nothing outside the range is written."""
+    from faster_yoco_amd import ops
+    rng = np.random.default_rng(n + world)
+    cs = [oracle.bf16_rne((rng.standard_normal(n) * 1e-2).astype(np.float32)) for _ in range(world)]
+    for first in range(4):
+        ts = []
+        for k, c in enumerate(cs):
+            buf = torch.zeros(n + 256, dtype=torch.bfloat16, device=dev)
+            o = (first * 3 + k * 5) % 67
+            buf[o:o + n].copy_(dev_bf16(c, dev))
+            ts.append(buf[o:o + n])
+        out = torch.zeros(n + 256, dtype=torch.bfloat16, device=dev)
+        osum = torch.zeros(n + 256, dtype=torch.float32, device=dev)
+        o1, o2, norm = 64 + first, 61 + first, torch.zeros(1, device=dev)
+        ws = ops.norm_workspace(dev, n)
+        ops.owner_sum(ts, out[o1:o1 + n], 1.0 / world, out_sum=osum[o2:o2 + n], partials=ws)
+        ops.norm_clip(ws, norm_out=norm)
+        torch.cuda.synchronize()
+        want, want_sum = oracle.owner_sum(cs, scale=1.0 / world, want_sum=True)
+        got = out.view(torch.int16).cpu().numpy().view(np.uint16)
+        assert np.array_equal(got[o1:o1 + n], want) and not got[:o1].any() and not got[o1 + n:].any()
+        got = osum.cpu().numpy()
+        assert np.array_equal(got[o2:o2 + n].view(np.uint32), want_sum.view(np.uint32))
+        assert not got[:o2].any() and not got[o2 + n:].any()
+        exact = np.float32(np.sqrt(oracle.sumsq(want)))
+        assert abs(norm.item() - exact) <= np.spacing(exact)
+
+
+@pytest.mark.parametrize('n', [1, 511, 512, 513, 40003])
+def test_scale_up_and_cast_at_any_offset(pkg, dev, n):
+    from faster_yoco_amd import ops
+    rng = np.random.default_rng(n)
+    x = (rng.standard_normal(n) * 3).astype(np.float32)
+    x16, fac = oracle.bf16_rne(x), torch.tensor([0.37], device=dev)
+    for a in range(4):
+        for b in range(4):
+            g16 = torch.zeros(n + 8, dtype=torch.bfloat16, device=dev)
+            g32, p32 = torch.zeros(n + 8, device=dev), torch.zeros(n + 8, device=dev)
+            p16 = torch.zeros(n + 8, dtype=torch.bfloat16, device=dev)
+            g16[a:a + n].copy_(dev_bf16(x16, dev))
+            p32[b:b + n].copy_(torch.from_numpy(x))
+            ops.scale_up(g16[a:a + n], g32[b:b + n], fac)
+            ops.cast_bf16(p32[b:b + n], p16[a:a + n])
+            torch.cuda.synchronize()
+            want = torch.mul(g16[a:a + n].float(), fac)
+            assert torch.equal(g32[b:b + n], want) and not g32[:b].any() and not g32[b + n:].any()
+            got = p16.view(torch.int16).cpu().numpy().view(np.uint16)
+            assert np.array_equal(got[a:a + n], x16) and not got[:a].any() and not got[a + n:].any()
+
+
 def test_sum_slots_phase_partials_give_the_norm_of_the_whole_average(pkg, dev):
     """CEReduce's phases at odd bounds, each summed in place with its norm partials left in its own slice of one
     array (sum_slots' waves), then one fixed-order reduction: the average bit-exact against the oracle, the norm
