@@ -62,8 +62,12 @@ class PhaseNorm:
         self.tiles = pos == self.G
 
     def matches(self, ce):
-        return (ce.out.data_ptr() == self.out_ptr and int(ce.G) == self.G
-                and tuple((int(a), int(b)) for a, b in ce.bounds) == self.bounds)
+        if ce.out.data_ptr() != self.out_ptr or ce.G != self.G or len(ce.bounds) != len(self.bounds):
+            return False
+        for (a, b), (c, d) in zip(ce.bounds, self.bounds):
+            if a != c or b != d:
+                return False
+        return True
 
     def ready(self):
         return self.tiles and all(s or a == b for s, (a, b) in zip(self.summed, self.bounds))
@@ -103,11 +107,18 @@ def take_norm_partials(grads):
     """(waves, m) of the CEReduce whose out the BF16 gradients ``grads`` tile exactly -- every element of [0, G) of
     out in exactly one of them, in any order -- when each of its phases has been summed since the partials were
     last taken; else None.  Taking them marks them used."""
-    if not FUSE_NORM or not grads or any(g.dtype != torch.bfloat16 or not g.is_cuda or not g.is_contiguous() for g in grads):
+    if not FUSE_NORM or not grads:
         return None
-    spans = sorted((g.data_ptr(), g.numel()) for g in grads if g.numel())
+    spans, dev = [], grads[0].device
+    for g in grads:
+        if g.dtype != torch.bfloat16 or not g.is_cuda or not g.is_contiguous() or g.device != dev:
+            return None
+        n = g.numel()
+        if n:
+            spans.append((g.data_ptr(), n))
+    spans.sort()
     pn = _BY_OUT.get(spans[0][0]) if spans else None
-    if pn is None or not pn.ready() or any(g.device != pn.device for g in grads):
+    if pn is None or not pn.ready() or pn.device != dev:
         return None
     pos = pn.out_ptr
     for ptr, n in spans:

@@ -4,7 +4,8 @@ synchronisation.  The calls allocate no device memory (tables and workspaces are
 ``Table`` / ``TableCache`` / ``norm_workspace``), with one exception: a factor given as a tensor to be read but not
 written (``factor_out`` None or another tensor) is copied first -- into ``factor_out`` when one is given, else into a
 new tensor -- because the operators write the clipped factor over the one they read.  A Python-number factor and a
-device output may be mixed as the reference's fairseq surface mixes them.
+device output may be mixed as the reference's fairseq surface mixes them.  Scalars go to the operators as Python
+floats, which round each once to fp32 (as a Triton or ctypes fp32 argument is rounded).
 
 ``table`` arguments are ``Table`` objects (``kernels.Table``); without explicit tensors an operation runs on the
 tensors the table was made with (``Table.bound``).
@@ -42,7 +43,7 @@ def _factor_io(factor, factor_out):
             return factor.clone(), None                  # read only: the chain writes to a copy
         factor_out.copy_(factor)
         return factor_out, None
-    return factor_out, f32(1.0 if factor is None else factor)
+    return factor_out, 1.0 if factor is None else float(factor)
 
 
 # ------------------------------------------------------------------------------------------------------- norm
@@ -54,7 +55,7 @@ def norm_clip(partials, factor=1.0, norm_out=None, grad_norm_out=None, factor_ou
     """Final fixed-order reduction + the clip chain.  factor: Python number or 1-element fp32 device tensor (read);
     factor_out (nullable, may be `factor`) receives the clipped factor."""
     f, fv = _factor_io(factor, factor_out)
-    _OPS.norm_clip_(partials, f, norm_out, grad_norm_out, f32(max_norm), fv)
+    _OPS.norm_clip_(partials, f, norm_out, grad_norm_out, float(max_norm), fv)
 
 
 def grad_norm_clip(table, partials, factor=1.0, norm_out=None, grad_norm_out=None, factor_out=None, max_norm=0.0,
@@ -62,7 +63,7 @@ def grad_norm_clip(table, partials, factor=1.0, norm_out=None, grad_norm_out=Non
     """grad_sumsq + norm_clip in one call."""
     f, fv = _factor_io(factor, factor_out)
     _OPS.grad_norm_clip_(table.handle_int, _bound(table)[0] if g is None else g, partials, f, norm_out, grad_norm_out,
-                         f32(max_norm), fv)
+                         float(max_norm), fv)
 
 
 def update_scalars(partials, sample_size=None, numer=1.0, factor=1.0, max_norm=0.0, norm_out=None,
@@ -70,8 +71,8 @@ def update_scalars(partials, sample_size=None, numer=1.0, factor=1.0, max_norm=0
     """The trainer's per-update scalar chain in one launch: optional sample-size factor, norm + clip chain,
     [finite, consistent] flags (uint8[2]) and the "clip" metric."""
     f, fv = _factor_io(factor, factor_out)
-    _OPS.update_scalars_(partials, f, norm_out, grad_norm_out, flags_out, clip_log_out, sample_size, f32(numer),
-                         f32(max_norm), fv)
+    _OPS.update_scalars_(partials, f, norm_out, grad_norm_out, flags_out, clip_log_out, sample_size, float(numer),
+                         float(max_norm), fv)
 
 
 def grad_update_scalars(table, partials, sample_size=None, numer=1.0, factor=1.0, max_norm=0.0, norm_out=None,
@@ -79,13 +80,13 @@ def grad_update_scalars(table, partials, sample_size=None, numer=1.0, factor=1.0
     """grad_sumsq + update_scalars in one call."""
     f, fv = _factor_io(factor, factor_out)
     _OPS.grad_update_scalars_(table.handle_int, _bound(table)[0] if g is None else g, partials, f, norm_out,
-                              grad_norm_out, flags_out, clip_log_out, sample_size, f32(numer), f32(max_norm), fv)
+                              grad_norm_out, flags_out, clip_log_out, sample_size, float(numer), float(max_norm), fv)
 
 
 def clip_factor(norm, factor=1.0, grad_norm_out=None, factor_out=None, max_norm=0.0):
     """The clip chain entered at `norm` (1-element fp32 device tensor)."""
     f, fv = _factor_io(factor, factor_out)
-    _OPS.clip_factor_(norm, f, grad_norm_out, f32(max_norm), fv)
+    _OPS.clip_factor_(norm, f, grad_norm_out, float(max_norm), fv)
 
 
 # ------------------------------------------------------------------------------------------------ Adam + BF16
@@ -105,7 +106,7 @@ def adam_cast_rows(table, row_begin, row_end, factor, lr, beta1, beta2, eps, bc1
     if table.numel == 0 or row_begin == row_end:
         return                                           # nothing to update (and no tensor to dispatch on)
     g, p, m, v, p16 = _bound(table) if tensors is None else tensors
-    args = (factor, f32(lr), f32(beta1), f32(beta2), f32(eps), f32(bc1), f32(bc2), f32(weight_decay), int(mode),
+    args = (factor, float(lr), float(beta1), float(beta2), float(eps), float(bc1), float(bc2), float(weight_decay), int(mode),
             int(row_begin), int(row_end))
     if g32 is None:
         _OPS.adam_cast_(table.handle_int, g, p, m, v, p16, *args)
@@ -118,8 +119,8 @@ def adam_cast_dev(table, factor, lr, beta1, beta2, eps, bc, weight_decay, mode, 
     if table.numel == 0:
         return
     g, p, m, v, p16 = _bound(table) if tensors is None else tensors
-    _OPS.adam_cast_dev_(table.handle_int, g, p, m, v, p16, factor, bc, f32(lr), f32(beta1), f32(beta2), f32(eps),
-                        f32(weight_decay), int(mode))
+    _OPS.adam_cast_dev_(table.handle_int, g, p, m, v, p16, factor, bc, float(lr), float(beta1), float(beta2), float(eps),
+                        float(weight_decay), int(mode))
 
 
 def bias_corrections_step(step, beta1, beta2, bc, bias_correction=1):
@@ -132,7 +133,7 @@ def bias_corrections_step(step, beta1, beta2, bc, bias_correction=1):
 def owner_sum(contribs, out, scale, out_sum=None, partials=None):
     """out[e] = bf16(sum_k float(contribs[k][e]) * scale), k in list order.  contribs: bf16 tensors of
     out.numel() elements each (sum_slots is the form where out holds one rank's own contribution)."""
-    _OPS.owner_sum_(list(contribs), out, f32(scale), out_sum, partials)
+    _OPS.owner_sum_(list(contribs), out, float(scale), out_sum, partials)
 
 
 def owner_sum_update(contribs, out, scale, workspace, out_sum=None, sample_size=None, numer=1.0, factor=1.0,
@@ -143,14 +144,14 @@ def owner_sum_update(contribs, out, scale, workspace, out_sum=None, sample_size=
     if workspace is None:
         raise RuntimeError('yoco_z1: owner_sum_update needs its workspace')
     f, fv = _factor_io(factor, factor_out)
-    _OPS.owner_sum_update_(list(contribs), out, workspace, f32(scale), out_sum, f, norm_out, grad_norm_out,
-                           flags_out, clip_log_out, sample_size, f32(numer), f32(max_norm), fv)
+    _OPS.owner_sum_update_(list(contribs), out, workspace, float(scale), out_sum, f, norm_out, grad_norm_out,
+                           flags_out, clip_log_out, sample_size, float(numer), float(max_norm), fv)
 
 
 def sum_slots(S, OUT, G, BASE, END, R, scale, WORLD, waves=None):
     """The owner sum in the reference's staging layout, in place (yoco/models/decoder/ce_reduce.py:59-74).  waves
     (float64, at least owner_sum_waves(END - BASE)): the range's norm partials per chunk, for reduce_waves."""
-    _OPS.sum_slots_(S, OUT, int(G), int(BASE), int(END), int(R), f32(scale), int(WORLD), waves)
+    _OPS.sum_slots_(S, OUT, int(G), int(BASE), int(END), int(R), float(scale), int(WORLD), waves)
 
 
 def owner_sum_waves(n):

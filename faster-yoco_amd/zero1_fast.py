@@ -174,13 +174,17 @@ def clip_grad_norm(self, max_norm, aggregate_norm_fn=None):
     if plan is None:
         return _ORIG['clip'](self, max_norm, aggregate_norm_fn)
     src = [a for a, _, _ in plan.mine] if REDUCE_OWNER else [a for a in self.fp16_params if a.requires_grad]
+    grads, dtypes = [], set()
     for a in src:
-        if a.grad is None:
-            a.grad = torch.zeros_like(a)
-    grads = [a.grad for a in src]
-    if any(not (g.is_cuda and g.is_contiguous() and g.dtype in (torch.float32, torch.bfloat16)) for g in grads):
-        raise RuntimeError('zero1_fast: gradients must be contiguous fp32/bf16 GPU tensors')
-    if len({g.dtype for g in grads}) > 1:
+        g = a.grad
+        if g is None:
+            g = a.grad = torch.zeros_like(a)
+        dt = g.dtype
+        if not (g.is_cuda and g.is_contiguous() and (dt is torch.bfloat16 or dt is torch.float32)):
+            raise RuntimeError('zero1_fast: gradients must be contiguous fp32/bf16 GPU tensors')
+        dtypes.add(dt)
+        grads.append(g)
+    if len(dtypes) > 1:
         grads = [g.float() for g in grads]          # one dtype per table; the fp32 upcast of bf16 is exact
     dev = grads[0].device if grads else (self.fp16_params[0].device if self.fp16_params else torch.device('cuda'))
     if plan.partials is None:
@@ -250,26 +254,24 @@ def step(self, closure=None, groups=None):
     plan = _plan(self)
     if plan is None:
         return _ORIG['step'](self, closure, groups)
-    for a, b, _ in plan.mine:
-        if a.grad is None:
-            a.grad = torch.zeros_like(a)
-        if b.grad is None:
-            b.grad = torch.zeros_like(b)
     if plan.mine:
         dev = plan.mine[0][1].device
         f1 = _device_factor(self._multiply_factor, dev, plan.scalar(2, dev))
         folded = {}
-        if plan.fused is not None:
-            folded = {b.data_ptr(): a.grad for a, b, _ in plan.mine
-                      if a.grad.dtype == torch.bfloat16 and a.grad.is_contiguous() and a.grad.numel() == b.numel()
-                      and (FOLD_SCALE or b.grad.is_contiguous())}
         for a, b, _ in plan.mine:
-            if b.data_ptr() in folded:
-                continue
-            if a.grad.dtype == torch.bfloat16 and a.grad.is_contiguous() and b.grad.is_contiguous():
-                scale_up(a.grad, b.grad, f1)
+            g16, g32 = a.grad, b.grad
+            if g16 is None:
+                g16 = a.grad = torch.zeros_like(a)
+            if g32 is None:
+                g32 = b.grad = torch.zeros_like(b)
+            whole16 = g16.dtype is torch.bfloat16 and g16.is_contiguous()
+            whole32 = g32.is_contiguous()
+            if (plan.fused is not None and whole16 and (FOLD_SCALE or whole32) and g16.numel() == b.numel()):
+                folded[b.data_ptr()] = g16
+            elif whole16 and whole32:
+                scale_up(g16, g32, f1)
             else:
-                torch.mul(a.grad, f1, out=b.grad)
+                torch.mul(g16, f1, out=g32)
         if plan.fused is not None:
             plan.fused.fold, plan.fused.fold_factor, plan.fused.fold_writes = folded, f1, not FOLD_SCALE
     self._multiply_factor = 1.0

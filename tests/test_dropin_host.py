@@ -109,3 +109,21 @@ def test_fused_adam_cast_orders_a_tables_rows_by_gradient_address(pkg):
     assert made == [sorted(t.data_ptr() for t in g)]
     (folded, idx, _, p16), = groups
     assert not folded and idx == (1, 2, 0) and p16 == [] and written == ()
+
+
+def test_profiler_regions_are_recorded_alike(pkg):
+    """shard.region: under a profiler the event record_function makes; without one, nothing but the body; traceable."""
+    from faster_yoco_amd import shard
+    with shard.region('clip-grads'):
+        pass
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as prof:
+        with shard.region('clip-grads'):
+            torch.ones(2)
+    (event,) = [e for e in prof.events() if e.name == 'clip-grads']
+    assert event.is_user_annotation
+
+    def body(x):
+        with shard.region('clip-grads'):
+            return x + 1
+
+    assert torch.equal(torch.compile(body, fullgraph=True, backend='eager')(torch.ones(2)), torch.full((2,), 2.0))
