@@ -33,9 +33,10 @@
 //     loads, and Adam walks the chunks from the last one, so its first gradient reads hit the 256 MB MALL
 //     (measured 2.05 vs 2.10 ms for Adam on the C2 shard; 128-512 MB kept, or everything, measured the same or
 //     slower).
-//   * No atomics anywhere; nothing but vector memory instructions write memory.  (The norm's final reduction is a
-//     second, one-workgroup launch: folding it into the last workgroup of the norm grid to finish, with an arrival
-//     counter, measured 75 us slower per step, because the grid's 2048 workgroups finish together.)
+//   * No atomic orders or sums anything; nothing but vector memory instructions write memory.  (The norm's final
+//     reduction is a second, one-workgroup launch: folding it into the last workgroup of the norm grid to finish, with
+//     an arrival counter, measured 75 us slower per step, because the grid's 2048 workgroups finish together.  Small
+//     tables take a grid of at most 64, where it is faster: norm_small_kernel.)
 //
 // Numerics follow the header: one rounding per fp32 operation, explicit FMAs where the reference has them,
 // correctly rounded division and square root (built with -fhip-fp32-correctly-rounded-divide-sqrt, no fast math,
@@ -46,6 +47,7 @@
 #include <stdint.h>
 #include <string.h>
 
+#include <atomic>
 #include <mutex>
 #include <new>
 #include <vector>
@@ -522,28 +524,31 @@ __device__ __forceinline__ void sumsq_range(const Row* __restrict__ rows, int nr
 // Each wave's first row comes from the rows' first chunks staged in LDS (tables of up to kSumsqLdsRows rows): one
 // load instead of a binary search of dependent scalar loads at the start of every wave.
 constexpr int kSumsqLdsRows = 512;
-template <int GDT, int NT>
-__global__ __launch_bounds__(NT) void sumsq_kernel(const Row* __restrict__ rows, int nrows, int64_t nchunks,
-                                                   int64_t keep_from, double* __restrict__ partials) {
-    constexpr int W = NT / kWave;
-    __shared__ double lds[W];
-    __shared__ int64_t first[kSumsqLdsRows];
-    const int lane = threadIdx.x & (kWave - 1);
+
+__device__ __forceinline__ void stage_rows(const Row* __restrict__ rows, int nrows, int64_t* first) {
+    if (nrows > 1 && nrows <= kSumsqLdsRows) {            // uniform over the workgroup (kernel arguments)
+        for (int i = threadIdx.x; i < nrows; i += blockDim.x) first[i] = rows[i].chunk0;
+        __syncthreads();
+    }
+}
+
+// The squares of wave w of (virtual) workgroup b, per lane; W waves per workgroup.
+template <int GDT, int W>
+__device__ __forceinline__ double sumsq_wave(const Row* __restrict__ rows, int nrows, int64_t nchunks, int64_t keep_from,
+                                             const int64_t* first, int b, int w, int lane) {
     // workgroup b strides through eighth (b & 7) of the chunks only: the eighth the XCD it is dispatched to
     // (b mod 8) owns, as in chunk_of_block (0.257 vs 0.268 ms on C2, 2.11 vs 2.34 ms on C4 for the whole grid
     // striding over every chunk).  The decomposition depends on b alone, so the partials stay deterministic.
-    const int64_t x = blockIdx.x & 7, j = blockIdx.x >> 3;
+    const int64_t x = b & 7, j = b >> 3;
     const int64_t Q = nchunks >> 3, R = nchunks & 7;
     const int64_t lo = x * Q + (x < R ? x : R), hi = lo + Q + (x < R ? 1 : 0);
-    const int64_t nw = (int64_t)(gridDim.x >> 3) * W;
-    const int64_t span = GDT == Z1_BF16 ? kSumsqBf16Span : 1;   // chunks a wave takes per step
-    const int64_t w0 = lo + span * (j * W + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave));
+    constexpr int64_t nw = Z1_NORM_PARTIALS / 8 * W;
+    constexpr int64_t span = GDT == Z1_BF16 ? kSumsqBf16Span : 1;   // chunks a wave takes per step
+    const int64_t w0 = lo + span * (j * W + w);
     int64_t split = keep_from > lo ? (keep_from < hi ? keep_from : hi) : lo;
     split = lo + (split - lo + span - 1) / span * span;   // on the run grid: no run straddles the two loops
     int t = 0;
-    if (nrows > 1 && nrows <= kSumsqLdsRows) {            // uniform over the workgroup (kernel arguments)
-        for (int i = threadIdx.x; i < nrows; i += NT) first[i] = rows[i].chunk0;
-        __syncthreads();
+    if (nrows > 1 && nrows <= kSumsqLdsRows) {
         int a = 0, z = nrows - 1;                         // the last row whose first chunk is <= w0
         while (a < z) {
             const int mid = (a + z + 1) >> 1;
@@ -558,8 +563,86 @@ __global__ __launch_bounds__(NT) void sumsq_kernel(const Row* __restrict__ rows,
     int64_t c = w0;
     sumsq_range<GDT, false>(rows, nrows, t, r, next0, c, split < hi ? split : hi, span * nw, lane, acc);
     sumsq_range<GDT, true>(rows, nrows, t, r, next0, c, hi, span * nw, lane, acc);
+    return acc;
+}
+
+template <int GDT, int NT>
+__global__ __launch_bounds__(NT) void sumsq_kernel(const Row* __restrict__ rows, int nrows, int64_t nchunks,
+                                                   int64_t keep_from, double* __restrict__ partials) {
+    __shared__ double lds[NT / kWave];
+    __shared__ int64_t first[kSumsqLdsRows];
+    stage_rows(rows, nrows, first);
+    const double acc = sumsq_wave<GDT, NT / kWave>(rows, nrows, nchunks, keep_from, first, (int)blockIdx.x,
+                                                   __builtin_amdgcn_readfirstlane(threadIdx.x / kWave),
+                                                   threadIdx.x & (kWave - 1));
     const double s = block_sum<NT>(acc, lds);
     if (threadIdx.x == 0) partials[blockIdx.x] = s;
+}
+
+// The norm and the scalar tail of a small table in one launch: the same decomposition, partials and final order (the
+// same bits) as sumsq_kernel and scalars_kernel, whose 2048 workgroups are here virtual ones, kNormSmallWaves / W of
+// them per real workgroup; only those with chunks are formed (`used`), the others' partials are zeros.  The last
+// workgroup to arrive at the launch's counter (one of the table's) adds the partials.  They cross the XCDs as system-scope stores and loads
+// (a wave's stores have reached memory before it counts its workgroup in), so no L2 is written back or invalidated.
+// No workgroup waits for another, and the counter is left at zero.
+// Latency bounds it: launch, row, chunk, arrival, partials.  Norm and clip back to back in a graph, against the two
+// launches: FP32 36,928 elements 6.2 against 8.0 us, 262,144 6.6 / 8.2, 524,288 7.6 / 8.4; BF16 1M 7.3 / 7.8, 2M
+// 8.7 / 8.1, and a launch of host time less (the 36,928-element update 19.0 -> 17.0 us).  Grids past kNormSmallGrid, or
+// more than one round per workgroup, lose: FP32 1M 9.4 (256 workgroups) and 10.6 (64, four rounds) against 8.4 us.
+constexpr int kNormSmallThreads = 1024;
+constexpr int kNormSmallWaves = kNormSmallThreads / kWave;
+constexpr int kNormSmallGrid = 128;
+constexpr unsigned kArrivals = 64;                            // counters of a table
+template <int GDT, int W>
+__global__ __launch_bounds__(kNormSmallThreads) void norm_small_kernel(const Row* __restrict__ rows, int nrows,
+                                                                      int64_t nchunks, int64_t keep_from, int used,
+                                                                      double* partials, unsigned* arrivals,
+                                                                      z1_update_scalars u) {
+    constexpr int kSlots = kNormSmallWaves / W;           // partials formed at a time
+    __shared__ double lds[kNormSmallWaves];
+    __shared__ int64_t first[kSumsqLdsRows];
+    __shared__ int last;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x & (kWave - 1);
+    stage_rows(rows, nrows, first);
+    const int s0 = blockIdx.x * kSlots;
+    double x = 0.0;
+    if (s0 + wave / W < used)
+        x = sumsq_wave<GDT, W>(rows, nrows, nchunks, keep_from, first, s0 + wave / W, wave % W, lane);
+#pragma unroll
+    for (int off = kWave / 2; off > 0; off >>= 1) x += __shfl_xor(x, off, kWave);
+    if (lane == 0) lds[wave] = x;
+    __syncthreads();
+    if (threadIdx.x < kSlots && s0 + (int)threadIdx.x < used) {
+        double p = 0.0;
+#pragma unroll
+        for (int w = 0; w < W; ++w) p += lds[threadIdx.x * W + w];
+        __hip_atomic_store(partials + s0 + threadIdx.x, p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+    if (blockIdx.x == 0)
+        for (int i = used + threadIdx.x; i < Z1_NORM_PARTIALS; i += kNormSmallThreads) partials[i] = 0.0;
+    // the partials of this workgroup were stored by its first wave, which now counts it in
+    if (wave == 0) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        if (lane == 0)
+            last = __hip_atomic_fetch_add(arrivals, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+    }
+    __syncthreads();
+    if (!last) return;
+    if (threadIdx.x == 0) __hip_atomic_store(arrivals, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    double s = 0.0;                                       // final_sum's order: thread t adds t, t + 256, ...
+    if (threadIdx.x < kThreads)
+        for (int i = threadIdx.x; i < used; i += kThreads)
+            s += __hip_atomic_load(partials + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+#pragma unroll
+    for (int off = kWave / 2; off > 0; off >>= 1) s += __shfl_xor(s, off, kWave);
+    if (lane == 0) lds[wave] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double tot = 0.0;
+#pragma unroll
+        for (int w = 0; w < kThreads / kWave; ++w) tot += lds[w];
+        scalar_tail(tot, u);
+    }
 }
 
 // The step counter and bias corrections on the device (z1_bias_corrections_step): ++*step; bc = fp32(1 - beta^step)
@@ -881,6 +964,9 @@ struct z1_table {
     int has_pmv;          // every row has p, m and v
     int gout_rows;        // rows with an FP32 gradient output (z1_table_set_grad_out), as last enqueued
     float** gout;         // device, in the same allocation: the output of each device row (NULL: none)
+    unsigned* arrivals;   // device, in the same allocation: kArrivals counters of norm_small_kernel, zero when not in use
+    mutable std::atomic<unsigned> next_arrival;   // launches take them in turn, so that norms of one table that overlap
+                                                  // (on two streams, each into its own partials) do not share one
     int64_t numel;
     int64_t nchunks;
     std::vector<Row> host_rows;   // host copy of the device rows' pointers, kept by rebind / set_grads
@@ -984,10 +1070,11 @@ static int table_create(const z1_tensor* rows, int nrows, int g_dtype, z1_table*
     int dev = 0;
     int rc = current_device(&dev);
     if (rc) return rc;
-    // host image of [rows][chunk -> row][gradient outputs, all NULL], copied in one transfer
+    // host image of [rows][chunk -> row][gradient outputs, all NULL][counters, 0], copied in one transfer
     const size_t rows_bytes = sizeof(Row) * h.size();
     const size_t gout_off = (rows_bytes + sizeof(int32_t) * (size_t)chunks + 15) & ~(size_t)15;
-    std::vector<unsigned char> img(gout_off + sizeof(float*) * h.size() + 64, 0);
+    const size_t arrivals_off = (gout_off + sizeof(float*) * h.size() + 127) & ~(size_t)127;
+    std::vector<unsigned char> img(arrivals_off + sizeof(unsigned) * kArrivals, 0);
     if (rows_bytes) memcpy(img.data(), h.data(), rows_bytes);
     int32_t* map = reinterpret_cast<int32_t*>(img.data() + rows_bytes);
     for (size_t i = 0; i < h.size(); ++i) {
@@ -1017,6 +1104,7 @@ static int table_create(const z1_tensor* rows, int nrows, int g_dtype, z1_table*
     }
     tb->chunk_row = reinterpret_cast<int32_t*>(reinterpret_cast<unsigned char*>(tb->rows) + rows_bytes);
     tb->gout = reinterpret_cast<float**>(reinterpret_cast<unsigned char*>(tb->rows) + gout_off);
+    tb->arrivals = reinterpret_cast<unsigned*>(reinterpret_cast<unsigned char*>(tb->rows) + arrivals_off);
     tb->gout_rows = 0;
     e = hipMemcpy(tb->rows, img.data(), img.size(), hipMemcpyHostToDevice);
     if (e != hipSuccess) {
@@ -1207,7 +1295,8 @@ static int64_t keep_from(const z1_table* table) {
     return table->nchunks > keep ? table->nchunks - keep : 0;
 }
 
-// The norm kernel over the table, then, with a tail, the one-workgroup final reduction + scalar chain.  (A single
+// The norm kernel over the table, then, with a tail, the one-workgroup final reduction + scalar chain; with a tail, both
+// in one launch for a table whose chunks need no more than kNormSmallGrid workgroups (norm_small_kernel).  (A single
 // launch whose last workgroup to finish runs the tail was measured slower: the 2048 workgroups end together, and
 // their device-scope release fences and same-address counter atomics cost 15-35 us at the end of the grid, against
 // about 4 us for the second launch.)
@@ -1218,6 +1307,22 @@ static int launch_sumsq(const z1_table* table, double* partials, const z1_update
     if (table->g_failed) return Z1_E_STATE;
     hipStream_t s = static_cast<hipStream_t>(stream);
     const int64_t kf = keep_from(table);
+    const int W = (table->g_dtype == Z1_F32 ? kThreads : kSumsqBf16Threads) / kWave;
+    // workgroups of the full grid that have chunks (the same number in each eighth, rounded up), and the small grid's
+    const int64_t per = (int64_t)W * (table->g_dtype == Z1_F32 ? 1 : kSumsqBf16Span);
+    const int64_t used = 8 * (((table->nchunks + 7) / 8 + per - 1) / per);
+    const int64_t want = (used * W + kNormSmallWaves - 1) / kNormSmallWaves;
+    if (tail && want <= kNormSmallGrid) {
+        const dim3 grid((unsigned)(want < 1 ? 1 : want));
+        unsigned* arrivals = table->arrivals + table->next_arrival.fetch_add(1, std::memory_order_relaxed) % kArrivals;
+        if (table->g_dtype == Z1_F32)
+            hipLaunchKernelGGL((norm_small_kernel<Z1_F32, kThreads / kWave>), grid, dim3(kNormSmallThreads), 0, s,
+                               table->rows, table->nrows_dev, table->nchunks, kf, (int)used, partials, arrivals, *tail);
+        else
+            hipLaunchKernelGGL((norm_small_kernel<Z1_BF16, kSumsqBf16Threads / kWave>), grid, dim3(kNormSmallThreads), 0,
+                               s, table->rows, table->nrows_dev, table->nchunks, kf, (int)used, partials, arrivals, *tail);
+        return launch_status();
+    }
     if (table->g_dtype == Z1_F32)
         hipLaunchKernelGGL((sumsq_kernel<Z1_F32, kThreads>), dim3(Z1_NORM_PARTIALS), dim3(kThreads), 0, s,
                            table->rows, table->nrows_dev, table->nchunks, kf, partials);

@@ -61,6 +61,52 @@ def test_grad_norm_clip_equals_the_two_launches(pkg, dev, dtype):
     assert np.array_equal(f32_bits(f_two), f32_bits(f_one))
 
 
+# the one-launch norm's range: FP32 up to 2048 chunks of 256 elements, BF16 up to 8192; a chunk more takes two launches
+@pytest.mark.parametrize('dtype,sizes', [(torch.float32, [1]), (torch.float32, [256 * 8, 255]),
+                                         (torch.float32, [256 * 2047, 200]), (torch.float32, [256 * 2048, 1]),
+                                         (torch.float32, [300] * 700), (torch.bfloat16, [5]),
+                                         (torch.bfloat16, [256 * 64, 1]), (torch.bfloat16, [256 * 8191, 256]),
+                                         (torch.bfloat16, [256 * 8192, 3]), (torch.bfloat16, [1021] * 600)])
+def test_norm_and_clip_of_small_tables_in_one_launch(pkg, dev, dtype, sizes):
+    """The bits of the partials (all 2048) and of every output equal the two launches', call after call on one table (its
+    arrival counter is back at zero each time), with another table's calls between, and replayed in a graph."""
+    from faster_yoco_amd import ops
+    gs, table = grads_table(pkg, dev, sizes, len(sizes), dtype)
+    _, other = grads_table(pkg, dev, [4000], 9, dtype)
+    part_a, part_b, part_c = (ops.norm_workspace(dev) for _ in range(3))
+    two, one, junk = scalars(dev), scalars(dev), scalars(dev)
+
+    def call():
+        ops.grad_norm_clip(other, part_c, norm_out=junk[0], factor_out=junk[2], max_norm=1.0)
+        ops.grad_norm_clip(table, part_b, factor=0.5, norm_out=one[0], grad_norm_out=one[1], factor_out=one[2],
+                           max_norm=0.125)
+
+    def check(k):
+        torch.cuda.synchronize()
+        assert np.array_equal(f32_bits(part_a[:2048]), f32_bits(part_b[:2048])), k
+        for a, b in zip(two, one):
+            assert np.array_equal(f32_bits(a), f32_bits(b)), k
+        part_b.fill_(-1.0)
+        for t in one:
+            t.fill_(-1.0)
+
+    ops.grad_sumsq(table, part_a)
+    ops.norm_clip(part_a, factor=0.5, norm_out=two[0], grad_norm_out=two[1], factor_out=two[2], max_norm=0.125)
+    for k in range(5):
+        call()
+        check(k)
+    graph, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    with torch.cuda.graph(graph, stream=side):
+        call()
+    for k in range(3):
+        graph.replay()
+        check(('replay', k))
+        call()
+        check(('between', k))
+    ex = float(np.sqrt(sum(oracle.sumsq(x.float().cpu().numpy()) for x in gs)))
+    assert abs(float(two[0].item()) - ex) <= 1e-6 * ex
+
+
 def test_grad_update_scalars_equals_the_two_launches(pkg, dev):
     from faster_yoco_amd import ops
     gs, table = grads_table(pkg, dev, [4096, 99, 1 << 16], 3)
