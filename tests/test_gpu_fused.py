@@ -157,6 +157,29 @@ def test_owner_sum_update_equals_the_two_calls(pkg, dev, world):
         assert np.array_equal(f32_bits(sum_b), want_sum.view(np.uint32))
 
 
+# per-chunk partials per slot 1 | 2, 2 | 3 (an odd tree), 3 | 4, and the most the one-launch reduction takes | one more
+@pytest.mark.parametrize('chunks', [1, 2047, 2048, 2049, 4097, 6144, 6145, 8191, 8192, 8193])
+def test_owner_sum_update_reductions(pkg, dev, chunks):
+    """The norm of owner_sum_update (one reduction launch for small inputs) has the bits of owner_sum + norm_clip, in all
+    2048 partials and every output, and is within an fp32 ulp of the exact one."""
+    from faster_yoco_amd import ops
+    n = chunks * 256 - 63                                # owner_sum_waves(n) == chunks
+    assert ops.owner_sum_waves(n) == chunks
+    gen = torch.Generator(device='cpu').manual_seed(chunks)
+    cs = [(torch.randn(n, generator=gen) * 1e-2).to(torch.bfloat16).to(dev) for _ in range(3)]
+    ws_a, ws_b = ops.norm_workspace(dev, n), ops.norm_workspace(dev, n)
+    avg, a, b = torch.empty(n, dtype=torch.bfloat16, device=dev), scalars(dev), scalars(dev)
+    ops.owner_sum(cs, avg, 0.25, partials=ws_a)
+    ops.norm_clip(ws_a, factor=2.0, norm_out=a[0], grad_norm_out=a[1], factor_out=a[2], max_norm=0.01)
+    ops.owner_sum_update(cs, avg, 0.25, ws_b, factor=2.0, norm_out=b[0], grad_norm_out=b[1], factor_out=b[2], max_norm=0.01)
+    torch.cuda.synchronize()
+    assert torch.equal(ws_a[:2048].view(torch.int64), ws_b[:2048].view(torch.int64))
+    for x, y in zip(a, b):
+        assert np.array_equal(f32_bits(x), f32_bits(y))
+    exact = np.float32(np.sqrt(oracle.sumsq(avg.float().cpu().numpy())))
+    assert abs(b[0].item() - exact) <= np.spacing(exact)
+
+
 def test_owner_sum_update_empty_input(pkg, dev):
     from faster_yoco_amd import ops
     out = torch.empty(0, dtype=torch.bfloat16, device=dev)
