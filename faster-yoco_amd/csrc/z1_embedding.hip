@@ -52,7 +52,8 @@ constexpr int kFewBlock = 8;               // the same, few indices
 constexpr int kMaxWaves = 1 << 20;         // most waves that sum runs (they stride beyond that)
 // Consecutive rows of one XCD: spans of 32 to 128 rows measure alike, single rows round robin 144 / 153; one eighth of the
 // table each leaves the frequent ids, which are the first ones, to one XCD.
-constexpr uint32_t kSpan = 128;
+constexpr int kSpan = 128;
+constexpr int64_t kMaxRowWaves = 1 << 25;   // a multiple of 8 kSpan; with kMaxWaves within one launch's 2^32 threads
 // Cache-policy bits of the rows' stores, sc0 sc1 nt as the update's streams have: 141 / 154 us against 147 / 158 with nt
 // alone, 159 / 164 with sc0 sc1, 161 / 164 with none.  (Waves that only zero and waves that only sum, in one launch in
 // either order or mixed, 141-161 / 160-173: a row-ordered mix suits the DRAM better than two patterns at once.)
@@ -477,26 +478,27 @@ __global__ __launch_bounds__(kEmbThreads) void emb_rows_kernel(const uint16_t* _
         return;
     }
     // Row of workgroup b (run_waves is a multiple of 8: workgroup b runs on XCD b mod 8): each XCD takes kSpan consecutive
-    // rows of every 8 kSpan
-    const uint32_t b = blockIdx.x - run_waves;
-    const int64_t t = (int64_t)(b & ~(8u * kSpan - 1)) + (b & 7) * kSpan + ((b >> 3) & (kSpan - 1));
-    if (t >= V) return;
+    // rows of every 8 kSpan.  (More rows than kMaxRowWaves: in several rounds.)
     const int lane = threadIdx.x, ng = (int)(D / 8);
-    const int2 r = info[t];
-    uint16_t* orow = out + t * D;
     const bool wide = D % 8 == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0;
-    if (r.y == 0 || t == padding_idx) {
-        for (int gi = lane; gi < ng; gi += kEmbThreads) row_store8(orow, wide, ng * 16, gi * 16, u4{0u, 0u, 0u, 0u});
-        if (ng * 8 + lane < D) orow[ng * 8 + lane] = 0;
-    } else if (r.y == 1) {
-        const int at[1] = {r.x};
-        sum_direct<FEW, G, 1>(at, 1, grad, D, scale, scale_mode, wide, orow);
-    } else if (r.y <= kDirect) {
-        const int pos = lane < r.y ? ent[r.x + lane].pos : 0;
-        int at[kDirect];
+    for (int64_t b = blockIdx.x - run_waves; b < V + 8 * kSpan; b += gridDim.x - run_waves) {
+        const int64_t t = (b & ~(int64_t)(8 * kSpan - 1)) + (b & 7) * kSpan + ((b >> 3) & (kSpan - 1));
+        if (t >= V) continue;
+        const int2 r = info[t];
+        uint16_t* orow = out + t * D;
+        if (r.y == 0 || t == padding_idx) {
+            for (int gi = lane; gi < ng; gi += kEmbThreads) row_store8(orow, wide, ng * 16, gi * 16, u4{0u, 0u, 0u, 0u});
+            if (ng * 8 + lane < D) orow[ng * 8 + lane] = 0;
+        } else if (r.y == 1) {
+            const int at[1] = {r.x};
+            sum_direct<FEW, G, 1>(at, 1, grad, D, scale, scale_mode, wide, orow);
+        } else if (r.y <= kDirect) {
+            const int pos = lane < r.y ? ent[r.x + lane].pos : 0;
+            int at[kDirect];
 #pragma unroll
-        for (int u = 0; u < kDirect; ++u) at[u] = __builtin_amdgcn_readlane(pos, u);
-        sum_direct<FEW, G, kDirect>(at, r.y, grad, D, scale, scale_mode, wide, orow);
+            for (int u = 0; u < kDirect; ++u) at[u] = __builtin_amdgcn_readlane(pos, u);
+            sum_direct<FEW, G, kDirect>(at, r.y, grad, D, scale, scale_mode, wide, orow);
+        }
     }
 }
 
@@ -739,7 +741,8 @@ void launch_rows_g(const RowsCall& c, const EmbWorkspace& w) {
         const int64_t blocks = (c.R + kBlock - 1) / kBlock, most = kMaxWaves / step_waves;      // steps <= 32,768
         run_waves = ((blocks < most ? blocks : most) + 7) / 8 * 8 * step_waves;
     }
-    const int64_t rows = (c.V + 8 * kSpan - 1) / (8 * kSpan) * (8 * kSpan);
+    const int64_t spans = (c.V + 8 * kSpan - 1) / (8 * kSpan) * (8 * kSpan);
+    const int64_t rows = spans < kMaxRowWaves ? spans : kMaxRowWaves;
     hipLaunchKernelGGL((emb_rows_kernel<FEW, G>), dim3((unsigned)(run_waves + rows)), dim3(kEmbThreads), c.lds, c.st,
                        c.grad, c.D, c.V, w.ent, w.info, c.padding_idx, c.scale, c.scale_mode, c.out, (int)run_waves,
                        (int)step_waves, w.counts, w.short_list, w.long_list, w.parts);

@@ -82,8 +82,8 @@ int z1_table_info(const z1_table* table, int64_t* numel, int64_t* nchunks, int* 
  * the stream like a launch (no allocation, no host synchronisation): launches enqueued after it read the new
  * gradients.  For callers whose gradient tensors are reallocated between steps while the parameters and optimizer
  * state stay put (the reference's zero_grad drops every gradient, yoco/tasks/zero1_fast.py:238-244), so that one
- * table made at set-up serves every step.  Rows whose new gradient is not aligned for the vector path take the
- * element-wise path. */
+ * table made at set-up serves every step.  Rows may start at any element: the vector path assumes no more than the elements'
+ * own alignment. */
 int z1_table_set_grads(z1_table* table, const void* const* g, int nrows, void* stream);
 
 /* Gives the table FP32 gradient outputs: g32 is a HOST array of nrows device float pointers, one per row given to
@@ -117,8 +117,8 @@ int z1_owner_sum_bf16(const uint16_t* const* contrib, int world, int64_t n, floa
  * (negative: error code): Z1_NORM_PARTIALS + z1_owner_sum_waves(n). */
 int64_t z1_owner_sum_workspace(int64_t n);
 /* Per-chunk norm partials an owner sum over n elements writes (negative: error code).  The chunk grid follows the
- * streams' addresses (boundaries on shared 128-byte lines, else on 8-byte words, so that a range starting anywhere
- * keeps the vector path); this count covers every grid. */
+ * average's address (boundaries on its 128-byte lines; the contributions may lie at any element); this count covers
+ * every grid. */
 int64_t z1_owner_sum_waves(int64_t n);
 
 /* z1_owner_sum_bf16 with the fused norm left per chunk: waves (z1_owner_sum_waves(n) doubles; nullable: no norm)
@@ -139,7 +139,7 @@ int z1_reduce_waves(const double* waves, int64_t m, double* partials, void* stre
  * decomposition into `partials` (Z1_NORM_PARTIALS doubles), no atomics. */
 int z1_grad_sumsq(const z1_table* table, double* partials, void* stream);
 
-/* z1_grad_sumsq then z1_norm_clip in one call (the norm kernel and the one-workgroup final kernel, the same bits):
+/* z1_grad_sumsq then z1_norm_clip in one call (the same bits; for a small table in one launch):
  * the norm + clip of yoco/tasks/zero1_fast.py:150-160 (fairseq utils.clip_grad_norm_ -> apex multi_tensor_l2norm,
  * then the torch scalar ops). */
 int z1_grad_norm_clip(const z1_table* table, double* partials, const float* factor_in, float factor_value,
@@ -243,8 +243,8 @@ int z1_cast_bf16(const float* p32, uint16_t* p16, int64_t n, void* stream);
  * order, one bf16 rounding.  For R <= 3072 its kernel for few indices: chunks of 16 indices, per chunk and id an fp32
  * sum rounded to bf16 and added to the bf16 row.  Every row of
  * out is written (rows without occurrences, padding_idx and ids outside [0, V) give zeros).  workspace: device
- * memory of z1_embedding_backward_workspace(R, D, V) bytes (with D <= 2^24: about 4/7 of R x D x 4 bytes for
- * the fp32 run partials of frequent ids, R x 8 + V x 8 bytes, and for many rows the sort's storage).  */
+ * memory of z1_embedding_backward_workspace(R, D, V) bytes (with D <= 2^24: R x D bytes for the fp32 run partials of
+ * frequent ids, 4 R x D for R <= 3072, R x 16 + V x 8 bytes, and for many rows the sort's storage).  */
 int z1_embedding_backward(const int64_t* ids, const uint16_t* grad, int64_t R, int64_t D, int64_t V,
                           int64_t padding_idx, float scale, int scale_mode, uint16_t* out, void* workspace,
                           int64_t workspace_bytes, void* stream);

@@ -128,6 +128,22 @@ def test_occurrence_counts(pkg, dev, D, few, V):
         assert np.array_equal(bits(out), bits(ref)), pad
 
 
+@pytest.mark.parametrize('V', [2 ** 25, 2 ** 25 + 1, 2 ** 26 + 2000])
+def test_more_rows_than_one_round_of_waves(pkg, dev, V):
+    """Tables of 2^25 rows (the most one launch has waves for) and more, past the former limit of one grid as well:
+    bit-exact against aten."""
+    from faster_yoco_amd import embedding
+    rng = np.random.default_rng(V)
+    ids = np.concatenate([rng.integers(0, V, 500), [0, V - 1, 2 ** 25 - 1, V - 1], np.full(40, V - 2)])
+    ids = torch.from_numpy(ids.astype(np.int64)).to(dev)
+    g = (torch.randn(ids.numel(), 2, device=dev) * 1e-2).to(torch.bfloat16)
+    ref = torch.ops.aten.embedding_dense_backward(g, ids, V, -1, False)
+    out = torch.full((V, 2), 7.0, dtype=torch.bfloat16, device=dev)
+    embedding.embedding_dense_backward(g, ids, V, -1, out=out)
+    torch.cuda.synchronize()
+    assert torch.equal(out.view(torch.int16), ref.view(torch.int16))
+
+
 @pytest.mark.parametrize('R', [1, 63, 1024, 1025, 16384, 16385, 20000, 49152, 49153])
 @pytest.mark.parametrize('V', [1, 2, 513, 65537, 524288, 524289])
 def test_order_of_occurrences(pkg, dev, R, V):
