@@ -140,7 +140,7 @@ __device__ __forceinline__ T ld_keep(const T* p) {       // ordinary load: alloc
 // interleaved on one box: C2 update 2.179 against 2.197-2.228 ms, C3 2.995-3.002 against 3.051-3.053 ms, the drop-in
 // step 3.268-3.282 against 3.325-3.329 ms, the scale pass over 430M elements 0.403 against 0.410 ms.  The same stores
 // with nt alone, through a buffer, measured like the global ones; the loads marked the same way were slower (C3
-// 3.27 ms), and so were the embedding gradient's row stores, which keep nt.  The descriptor covers one wave's chunk
+// 3.27 ms).  The descriptor covers one wave's chunk
 // (word 3 = 0x00020000: the raw 32-bit data format of gfx9 buffer resources), so the offset is the lane's byte offset
 // within it.
 constexpr int kStreamStorePolicy = 1 | 2 | 16;
