@@ -76,7 +76,7 @@ constexpr int64_t kMaxCols = 1 << 24;      // D limit: keeps the workspace size 
 
 __device__ __forceinline__ float bf16f(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
 
-// Round to nearest even, with gfx950's conversion (any NaN gives a NaN).
+// Round to nearest even, with gfx950's conversion (a NaN keeps its sign and payload: finish makes aten's of it).
 __device__ __forceinline__ uint16_t bf16r(float x) { return __builtin_bit_cast(uint16_t, (__bf16)x); }
 
 // One place of the sorted order: the occurrence's position, its id, and the id's first place and count.
@@ -266,11 +266,11 @@ __device__ __forceinline__ float grad_elem(uint16_t h, float scale, int scale_mo
 }
 
 // The finished fp32 sum to bf16; scale_mode 2 multiplies the bf16 result by scale and rounds again
-// (layer_graphs.py:93).
+// (layer_graphs.py:93).  Every NaN comes out as 0x7fc0, the one aten's conversion gives.
 __device__ __forceinline__ uint16_t finish(float acc, float scale, int scale_mode) {
     uint16_t o = bf16r(acc);
     if (scale_mode == 2) o = bf16r(bf16f(o) * scale);
-    return o;
+    return (o & 0x7fffu) > 0x7f80u ? (uint16_t)0x7fc0u : o;
 }
 
 // Rows start wherever t * D puts them: the wide accesses below assume 2-byte alignment only (gfx950 loads and stores 16

@@ -185,6 +185,29 @@ def test_row_widths(pkg, dev, R, D):
     assert np.array_equal(bits(got), bits(ref))
 
 
+@pytest.mark.parametrize('few', [True, False])
+def test_every_bf16_value(pkg, dev, few):
+    """All 65,536 bf16 patterns (every NaN, infinities, denormals, both zeros) as an id's first occurrence, alone and
+    before 3, 4, 10 and 40 others (the row's own wave, one run, several, a long chain), in the three placements of the
+    scale: the bits of aten and aten's multiplication, whose NaN is 0x7fc0."""
+    from faster_yoco_amd import embedding
+    counts, D = [1, 4, 5, 11, 41], 16384
+    pattern = torch.arange(-2 ** 15, 2 ** 15, device=dev).to(torch.int16).view(torch.bfloat16).view(4, D)
+    for n in counts:
+        g = (torch.randn(4 * n + (0 if few else 3100), D, device=dev) * 1e-2).to(torch.bfloat16)
+        g[:4] = pattern
+        ids = torch.full((g.shape[0],), 9, device=dev)
+        ids[:4 * n] = torch.arange(4 * n, device=dev) % 4
+        aten = torch.ops.aten.embedding_dense_backward
+        ref, ref_ce = aten(g, ids, 10, 9, False), aten(g * 0.125, ids, 10, 9, False)
+        got = embedding.embedding_dense_backward(g, ids, 10, 9)
+        got_owner = embedding.owner_embedding_grad(g, ids, 10, 9, 8)
+        got_ce = embedding.ce_owner_embedding_grad(g, ids, 10, 9, 8)
+        torch.cuda.synchronize()
+        for a, b in ((got, ref), (got_owner, ref * 0.125), (got_ce, ref_ce)):
+            assert torch.equal(a.view(torch.int16), b.view(torch.int16)), n
+
+
 def test_matches_oracle_and_edge_cases(pkg, dev):
     from faster_yoco_amd import embedding
     rng = np.random.default_rng(3)
