@@ -47,7 +47,6 @@
 #include <stdint.h>
 #include <string.h>
 
-#include <atomic>
 #include <mutex>
 #include <new>
 #include <vector>
@@ -582,7 +581,7 @@ __global__ __launch_bounds__(NT) void sumsq_kernel(const Row* __restrict__ rows,
 // The norm and the scalar tail of a small table in one launch: the same decomposition, partials and final order (the
 // same bits) as sumsq_kernel and scalars_kernel, whose 2048 workgroups are here virtual ones, kNormSmallWaves / W of
 // them per real workgroup; only those with chunks are formed (`used`), the others' partials are zeros.  The last
-// workgroup to arrive at the launch's counter (one of the table's) adds the partials.  They cross the XCDs as system-scope stores and loads
+// workgroup to arrive at the launch's counter (the workspace's, in the table) adds the partials.  They cross the XCDs as system-scope stores and loads
 // (a wave's stores have reached memory before it counts its workgroup in), so no L2 is written back or invalidated.
 // No workgroup waits for another, and the counter is left at zero.
 // Latency bounds it: launch, row, chunk, arrival, partials.  Norm and clip back to back in a graph, against the two
@@ -592,7 +591,7 @@ __global__ __launch_bounds__(NT) void sumsq_kernel(const Row* __restrict__ rows,
 constexpr int kNormSmallThreads = 1024;
 constexpr int kNormSmallWaves = kNormSmallThreads / kWave;
 constexpr int kNormSmallGrid = 128;
-constexpr unsigned kArrivals = 64;                            // counters of a table
+constexpr int kArrivals = 64;                                 // counters of a table: workspaces that take this launch
 template <int GDT, int W>
 __global__ __launch_bounds__(kNormSmallThreads) void norm_small_kernel(const Row* __restrict__ rows, int nrows,
                                                                       int64_t nchunks, int64_t keep_from, int used,
@@ -1006,8 +1005,8 @@ struct z1_table {
     int gout_rows;        // rows with an FP32 gradient output (z1_table_set_grad_out), as last enqueued
     float** gout;         // device, in the same allocation: the output of each device row (NULL: none)
     unsigned* arrivals;   // device, in the same allocation: kArrivals counters of norm_small_kernel, zero when not in use
-    mutable std::atomic<unsigned> next_arrival;   // launches take them in turn, so that norms of one table that overlap
-                                                  // (on two streams, each into its own partials) do not share one
+    mutable z1detail::WorkspaceSlots<kArrivals> arrival_slots;   // which counter a norm uses, by its partials: norms that
+                                                                 // overlap (graph replays included) have their own
     int64_t numel;
     int64_t nchunks;
     std::vector<Row> host_rows;   // host copy of the device rows' pointers, kept by rebind / set_grads
@@ -1337,7 +1336,8 @@ static int64_t keep_from(const z1_table* table) {
 }
 
 // The norm kernel over the table, then, with a tail, the one-workgroup final reduction + scalar chain; with a tail, both
-// in one launch for a table whose chunks need no more than kNormSmallGrid workgroups (norm_small_kernel).  (A single
+// in one launch for a table whose chunks need no more than kNormSmallGrid workgroups (norm_small_kernel) and the first
+// kArrivals workspaces used with it.  (A single
 // launch whose last workgroup to finish runs the tail was measured slower: the 2048 workgroups end together, and
 // their device-scope release fences and same-address counter atomics cost 15-35 us at the end of the grid, against
 // about 4 us for the second launch.)
@@ -1353,9 +1353,10 @@ static int launch_sumsq(const z1_table* table, double* partials, const z1_update
     const int64_t per = (int64_t)W * (table->g_dtype == Z1_F32 ? 1 : kSumsqBf16Span);
     const int64_t used = 8 * (((table->nchunks + 7) / 8 + per - 1) / per);
     const int64_t want = (used * W + kNormSmallWaves - 1) / kNormSmallWaves;
-    if (tail && want <= kNormSmallGrid) {
+    const int slot = tail && want <= kNormSmallGrid ? table->arrival_slots.slot(partials) : -1;
+    if (slot >= 0) {
         const dim3 grid((unsigned)(want < 1 ? 1 : want));
-        unsigned* arrivals = table->arrivals + table->next_arrival.fetch_add(1, std::memory_order_relaxed) % kArrivals;
+        unsigned* arrivals = table->arrivals + slot;
         if (table->g_dtype == Z1_F32)
             hipLaunchKernelGGL((norm_small_kernel<Z1_F32, kThreads / kWave>), grid, dim3(kNormSmallThreads), 0, s,
                                table->rows, table->nrows_dev, table->nchunks, kf, (int)used, partials, arrivals, *tail);

@@ -141,7 +141,8 @@ int z1_grad_sumsq(const z1_table* table, double* partials, void* stream);
 
 /* z1_grad_sumsq then z1_norm_clip in one call (the same bits; for a small table in one launch):
  * the norm + clip of yoco/tasks/zero1_fast.py:150-160 (fairseq utils.clip_grad_norm_ -> apex multi_tensor_l2norm,
- * then the torch scalar ops). */
+ * then the torch scalar ops).  Norms of one table, replays of captured ones included, may overlap when each has its own
+ * partials; calls and replays that share partials are ordered by the caller. */
 int z1_grad_norm_clip(const z1_table* table, double* partials, const float* factor_in, float factor_value,
                       float* norm_out, float* grad_norm_out, float* factor_out, float max_norm, void* stream);
 

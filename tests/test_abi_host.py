@@ -5,6 +5,7 @@ import ctypes
 import math
 import os
 import re
+import subprocess
 
 import numpy as np
 import pytest
@@ -164,7 +165,6 @@ def test_layout_place_params_cpu(pkg):
 def test_header_is_plain_c_and_links(pkg, tmp_path):
     """include/yoco_z1.h compiles as C11 with gcc and a C program links and runs against libyoco_z1.so (argument
     errors only: no device work)."""
-    import subprocess
     from faster_yoco_amd import _lib
     libdir = os.path.dirname(_lib.LIB_PATH)
     exe = tmp_path / 'abi_smoke'
@@ -173,3 +173,53 @@ def test_header_is_plain_c_and_links(pkg, tmp_path):
                     f'-Wl,-rpath,{libdir}', '-o', str(exe)], check=True)
     res = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
     assert res.returncode == 0 and res.stdout.strip() == 'ok', res.stdout + res.stderr
+
+
+def test_norm_workspaces_have_their_own_counters(tmp_path):
+    """z1detail::WorkspaceSlots, which names the arrival counter of a one-launch norm: whatever order calls come in, two
+    workspaces never share a slot (65 of them neither: the last gets none), one workspace keeps its own, and threads that
+    meet on their first calls agree."""
+    src = tmp_path / 'slots.cpp'
+    src.write_text(r"""
+#include <cstdio>
+#include <set>
+#include <thread>
+#include <vector>
+#include "z1_internal.h"
+int main() {
+    static const char ws[80] = {};
+    z1detail::WorkspaceSlots<64> s;
+    const int first = s.slot(ws);
+    std::set<int> seen{first};
+    for (int i = 1; i < 64; ++i) {
+        seen.insert(s.slot(ws + i));
+        if (s.slot(ws) != first) return 1;              // a call fixed in a graph, beside others
+    }
+    if (seen.size() != 64 || *seen.begin() != 0 || *seen.rbegin() != 63) return 2;
+    for (int i = 64; i < 80; ++i)
+        if (s.slot(ws + i) != -1) return 3;
+    for (int i = 0; i < 64; ++i)
+        if (s.slot(ws + i) != i) return 4;
+    for (int round = 0; round < 200; ++round) {
+        z1detail::WorkspaceSlots<64> t;
+        int got[8][64];
+        std::vector<std::thread> threads;
+        for (int k = 0; k < 8; ++k)
+            threads.emplace_back([&, k] { for (int i = 0; i < 64; ++i) got[k][(i + 8 * k) % 64] = t.slot(ws + (i + 8 * k) % 64); });
+        for (auto& x : threads) x.join();
+        std::set<int> all;
+        for (int i = 0; i < 64; ++i) {
+            all.insert(got[0][i]);
+            for (int k = 0; k < 8; ++k)
+                if (got[k][i] != got[0][i] || got[k][i] < 0) return 5;
+        }
+        if (all.size() != 64) return 6;
+    }
+    std::puts("ok");
+}
+""")
+    exe = tmp_path / 'slots'
+    subprocess.run(['g++', '-std=c++17', '-O2', '-Wall', '-Werror', '-pthread',
+                    '-I', os.path.join(ROOT, 'faster-yoco_amd', 'csrc'), str(src), '-o', str(exe)], check=True)
+    res = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
+    assert res.returncode == 0 and res.stdout.strip() == 'ok', (res.returncode, res.stdout)

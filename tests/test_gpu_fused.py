@@ -107,6 +107,54 @@ def test_norm_and_clip_of_small_tables_in_one_launch(pkg, dev, dtype, sizes):
     assert abs(float(two[0].item()) - ex) <= 1e-6 * ex
 
 
+def test_norms_of_one_table_overlap(pkg, dev):
+    """Norms of one table on three streams at once, each into its own workspace: a graph's replays, eager calls into one
+    workspace, and eager calls into 70 others (more than the one-launch norm has counters for).  Every result has the two
+    launches' bits, and so has the next one of each workspace."""
+    from faster_yoco_amd import _lib, ops
+    gs, table = grads_table(pkg, dev, [256 * 60, 3001, 77], 5)
+    L, want = _lib.lib(), scalars(dev)
+    part = ops.norm_workspace(dev)
+    ops.grad_sumsq(table, part)
+    ops.norm_clip(part, factor=0.5, norm_out=want[0], grad_norm_out=want[1], factor_out=want[2], max_norm=0.125)
+    slots = [(ops.norm_workspace(dev), scalars(dev)) for _ in range(72)]
+    torch.cuda.synchronize()
+
+    def norm(k):                # at the C ABI: the operators order calls of one table, the caller of these need not
+        ws, out = slots[k]
+        rc = L.z1_grad_norm_clip(table.handle, ws.data_ptr(), None, 0.5, out[0].data_ptr(), out[1].data_ptr(),
+                                 out[2].data_ptr(), 0.125, torch.cuda.current_stream().cuda_stream)
+        assert rc == 0
+
+    def check(when):
+        torch.cuda.synchronize()
+        for k, (_, out) in enumerate(slots):
+            for a, b in zip(want, out):
+                assert np.array_equal(f32_bits(a), f32_bits(b)), (when, k)
+                b.fill_(-1.0)
+        torch.cuda.synchronize()
+
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=streams[0]):
+        for _ in range(20):
+            norm(0)
+    for when in range(5):
+        for i in range(10):
+            with torch.cuda.stream(streams[0]):
+                graph.replay()
+            with torch.cuda.stream(streams[1]):
+                for _ in range(20):
+                    norm(1)
+            with torch.cuda.stream(streams[2]):
+                for k in range(2, 72):
+                    norm(k)
+        check(when)
+    for k in range(72):
+        norm(k)
+    check('after')
+
+
 def test_grad_update_scalars_equals_the_two_launches(pkg, dev):
     from faster_yoco_amd import ops
     gs, table = grads_table(pkg, dev, [4096, 99, 1 << 16], 3)
