@@ -355,11 +355,14 @@ __device__ __forceinline__ void sum_runs(int64_t p0, int step, bool last_step, c
         const int64_t row = (int64_t)__builtin_amdgcn_readlane((int)e.id, l) & 0xffffffff;
         const bool only = !FEW && n <= kRowsPerPartial;
         float* dst = parts + (only ? 0 : run_slot<FEW>(lo, s)) * D;
+        int at[kRows];               // read with every lane active: lanes without a group hold places too
+#pragma unroll
+        for (int u = 0; u < kRows; ++u) at[u] = __builtin_amdgcn_readlane(e.pos, l + u);
         if (gi < ng) {
             u4 x[kRows];
 #pragma unroll
             for (int u = 0; u < kRows; ++u)
-                if (u < cnt) x[u] = load8(grad + (int64_t)__builtin_amdgcn_readlane(e.pos, l + u) * D + gi * 8);
+                if (u < cnt) x[u] = load8(grad + (int64_t)at[u] * D + gi * 8);
             float part[8];
 #pragma unroll
             for (int k = 0; k < 8; ++k) part[k] = 0.0f;
@@ -387,8 +390,8 @@ __device__ __forceinline__ void sum_runs(int64_t p0, int step, bool last_step, c
             const int64_t d = ng * 8 + lane;
             float part = 0.0f;
             for (int u = 0; u < cnt; ++u) {
-                const int64_t at = __builtin_amdgcn_readlane(e.pos, l + u);
-                if (d < D) part = part + grad_elem(grad[at * D + d], scale, scale_mode);
+                const int64_t row_at = __builtin_amdgcn_readlane(e.pos, l + u);
+                if (d < D) part = part + grad_elem(grad[row_at * D + d], scale, scale_mode);
             }
             if (d < D) {
                 if (only) out[row * D + d] = finish(0.0f + part, scale, scale_mode);

@@ -223,3 +223,23 @@ int main() {
                     '-I', os.path.join(ROOT, 'faster-yoco_amd', 'csrc'), str(src), '-o', str(exe)], check=True)
     res = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
     assert res.returncode == 0 and res.stdout.strip() == 'ok', (res.returncode, res.stdout)
+
+
+def test_no_cross_lane_read_under_a_lane_dependent_branch():
+    """A value read from another lane is only sure to be there while that lane is active: no readlane, shuffle or ballot
+    of the kernels stands in a block whose condition differs from lane to lane."""
+    cross = re.compile(r'__builtin_amdgcn_read(?:first)?lane|__shfl|__ballot')
+    found = []
+    for name in ('z1_kernels.hip', 'z1_embedding.hip'):
+        text = open(os.path.join(ROOT, 'faster-yoco_amd', 'csrc', name)).read()
+        text = re.sub(r'//[^\n]*', '', text)
+        for m in re.finditer(r'\bif (?:constexpr )?\(((?:[^()]|\([^()]*\))*)\) \{', text):
+            if not re.search(r'\b(?:lane|gi|d|mine|loc\[i\])\b', m.group(1)):
+                continue
+            depth, end = 1, m.end()
+            while depth:
+                depth += {'{': 1, '}': -1}.get(text[end], 0)
+                end += 1
+            if cross.search(text, m.end(), end):
+                found.append((name, m.group(1)))
+    assert not found
