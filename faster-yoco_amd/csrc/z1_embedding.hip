@@ -267,10 +267,13 @@ __device__ __forceinline__ float grad_elem(uint16_t h, float scale, int scale_mo
 
 // The finished fp32 sum to bf16; scale_mode 2 multiplies the bf16 result by scale and rounds again
 // (layer_graphs.py:93).  Every NaN comes out as 0x7fc0, the one aten's conversion gives.
+__device__ __forceinline__ float scaled(float acc, float scale, int scale_mode) {
+    return scale_mode == 2 ? bf16f(bf16r(acc)) * scale : acc;
+}
+
 __device__ __forceinline__ uint16_t finish(float acc, float scale, int scale_mode) {
-    uint16_t o = bf16r(acc);
-    if (scale_mode == 2) o = bf16r(bf16f(o) * scale);
-    return (o & 0x7fffu) > 0x7f80u ? (uint16_t)0x7fc0u : o;
+    const float v = scaled(acc, scale, scale_mode);
+    return v != v ? (uint16_t)0x7fc0u : bf16r(v);
 }
 
 // Rows start wherever t * D puts them: the wide accesses below assume 2-byte alignment only (gfx950 loads and stores 16
@@ -311,6 +314,24 @@ __device__ __forceinline__ bool run_starts(int p, int lo, int pos, int prev) {
 template <bool FEW>
 __device__ __forceinline__ int64_t run_slot(int lo, int p) {
     return FEW ? p : ((int64_t)lo + kSlotSpan - 1) / kSlotSpan + (p - lo) / kRowsPerPartial;
+}
+
+// Eight finished sums.  One compare looks for a NaN in two of them, and lanes without one skip the rest.
+__device__ __forceinline__ u4 finish8(const float (&acc)[8], float scale, int scale_mode) {
+    float v[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = scaled(acc[k], scale, scale_mode);
+    bool nan = false;
+#pragma unroll
+    for (int k = 0; k < 8; k += 2) nan |= __builtin_isunordered(v[k], v[k + 1]);
+    if (nan) {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v[k] = v[k] != v[k] ? __uint_as_float(0x7fc00000u) : v[k];
+    }
+    u4 o;
+#pragma unroll
+    for (int k = 0; k < 8; k += 2) o[k >> 1] = (uint32_t)bf16r(v[k]) | ((uint32_t)bf16r(v[k + 1]) << 16);
+    return o;
 }
 
 __device__ __forceinline__ uint16_t col(const u4& x, int k) { return (uint16_t)(x[k >> 1] >> ((k & 1) * 16)); }
@@ -374,12 +395,9 @@ __device__ __forceinline__ void sum_runs(int64_t p0, int step, bool last_step, c
                 }
             }
             if (only) {
-                u4 o;
 #pragma unroll
-                for (int k = 0; k < 8; k += 2)
-                    o[k >> 1] = (uint32_t)finish(0.0f + part[k], scale, scale_mode) |
-                                ((uint32_t)finish(0.0f + part[k + 1], scale, scale_mode) << 16);
-                nt_store8(out + row * D + gi * 8, o);
+                for (int k = 0; k < 8; ++k) part[k] = 0.0f + part[k];
+                nt_store8(out + row * D + gi * 8, finish8(part, scale, scale_mode));
             } else {
                 f4_any* o = reinterpret_cast<f4_any*>(dst + gi * 8);
                 o[0] = f4{part[0], part[1], part[2], part[3]};
@@ -434,11 +452,9 @@ __device__ __forceinline__ void sum_direct(const int* at, int n, const uint16_t*
                     for (int k = 0; k < 8; ++k) part[k] = part[k] + grad_elem(col(x[u][g], k), scale, scale_mode);
                 }
             }
-            u4 o;
 #pragma unroll
-            for (int k = 0; k < 8; k += 2)
-                o[k >> 1] = (uint32_t)finish(add_part<FEW>(acc[k], part[k]), scale, scale_mode) |
-                            ((uint32_t)finish(add_part<FEW>(acc[k + 1], part[k + 1]), scale, scale_mode) << 16);
+            for (int k = 0; k < 8; ++k) acc[k] = add_part<FEW>(acc[k], part[k]);
+            const u4 o = finish8(acc, scale, scale_mode);
             if (gi + g * kEmbThreads < ng) row_store8(orow, wide, ng * 16, (gi + g * kEmbThreads) * 16, o);
         }
     }
