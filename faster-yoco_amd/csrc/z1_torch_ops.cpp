@@ -21,9 +21,12 @@
  */
 #include <ATen/core/Tensor.h>
 #include <ATen/ops/empty.h>
+#include <ATen/record_function.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 #include <torch/library.h>
 
 #include <dlfcn.h>
@@ -829,6 +832,12 @@ int z1t_table_register(z1_table* table, int device, int g_dtype, int has_pmv, in
     std::lock_guard<std::mutex> lock(g_mu);
     g_tables[reinterpret_cast<uintptr_t>(table)] = std::move(t);
     return 0;
+}
+
+/* Whether anything on this thread would see a profiler region: a RecordFunction observer (profilers, execution traces; of
+ * this thread or of all), a dispatch mode, or a trace being recorded. */
+int z1t_observed() {
+    return at::hasCallbacks() || c10::impl::TorchDispatchModeTLS::any_modes_set() || torch::jit::tracer::isTracing();
 }
 
 /* Forgets a table (before z1_table_destroy). */

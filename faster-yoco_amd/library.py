@@ -56,6 +56,8 @@ def _load():
 
 
 OPS_LIB = _load()
+# whether a profiler region would be seen (z1t_observed): called with the interpreter lock held, 0.1 us
+observed = ctypes.PyDLL(OPS_LIB_PATH).z1t_observed
 
 
 def _none(*args, **kwargs):

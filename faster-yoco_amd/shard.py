@@ -10,20 +10,24 @@ plus a device-resident offset table (one row per tensor) built once.  One optimi
 norm (fixed-order partials) -> its final reduction + the clip chain (one workgroup) -> Adam + BF16 over the table.
 With owner-side contributions (``reduce_grads`` / ``reduce_clip``) the norm is fused into the owner sum.
 """
+import contextlib
 import math
 
 import torch
 from torch.autograd.profiler import record_function
 
-from . import ops
+from . import library, ops
+
+
+_UNSEEN = contextlib.nullcontext()
 
 
 def region(name):
-    """A profiler region.  torch's record_function takes about 10 us of host time even when nothing records (an update of
-    the smallest shards takes 20); without a profiler the C++ form of it, 0.5 us, tells any other observer."""
-    if torch.compiler.is_compiling() or torch.autograd._profiler_enabled():
+    """A profiler region where anything would see it.  torch's record_function takes about 10 us of host time even when
+    nothing records (an update of the smallest shards takes 20)."""
+    if torch.compiler.is_compiling() or library.observed():
         return record_function(name)
-    return torch._C._profiler._RecordFunctionFast(name)
+    return _UNSEEN
 
 
 def _numel(shape):

@@ -127,3 +127,53 @@ def test_profiler_regions_are_recorded_alike(pkg):
             return x + 1
 
     assert torch.equal(torch.compile(body, fullgraph=True, backend='eager')(torch.ones(2)), torch.full((2,), 2.0))
+
+
+def test_profiler_regions_reach_every_observer(pkg, tmp_path):
+    """shard.region where no profiler runs on the calling thread: what an execution trace, a profiler of all threads, a
+    dispatch mode and a recorded trace see is what record_function shows them; nothing is entered when nothing looks."""
+    import json
+    import threading
+    from torch._C._profiler import _ExperimentalConfig
+    from torch.autograd.profiler import record_function
+    from torch.profiler import ExecutionTraceObserver, ProfilerActivity, profile
+    from torch.utils._python_dispatch import TorchDispatchMode
+    from faster_yoco_amd import shard
+
+    class Seen(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.names.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    def seen(make):
+        def body():
+            with make('clip-grads'):
+                torch.ones(2)
+
+        path = str(tmp_path / make.__name__)
+        trace = ExecutionTraceObserver().register_callback(path)
+        trace.start()
+        body()
+        trace.stop()
+        trace.unregister_callback()
+        nodes = [n['name'] for n in json.load(open(path))['nodes']]
+        config = _ExperimentalConfig(profile_all_threads=True)
+        with profile(activities=[ProfilerActivity.CPU], experimental_config=config) as prof:
+            thread = threading.Thread(target=body)
+            thread.start()
+            thread.join()
+        events = [e.is_user_annotation for e in prof.events() if e.name == 'clip-grads']
+        mode = Seen()
+        mode.names = []
+        with mode:
+            body()
+
+        def traced(x):
+            with make('clip-grads'):
+                return x + 1
+
+        graph = str(torch.jit.trace(traced, torch.ones(2)).graph).count('clip-grads')
+        return nodes.count('clip-grads'), events, mode.names, graph
+
+    assert seen(shard.region) == seen(record_function)
+    assert type(shard.region('clip-grads')) is not record_function
