@@ -47,6 +47,16 @@ constexpr int kWave = 64;
 // 20, 152 / 157 at 10, 175 / 185 at 8 (a short table, 2000 rows of 768 into 32,000: 32.4 us at 20, 33.9 at 14, 37 at 10).
 constexpr int kEmbWgPerCu = 16;
 constexpr int kDirect = 4;                 // most occurrences of an id that the wave of its row sums (2: the same)
+// In a dense table, of kDenseMean indices per row or more on average, the wave of a row sums up to kDirectDense occurrences
+// (two runs): most ids have between 5 and 20 there, and the row waves alone fill the chip, so that partials sent through
+// memory only add traffic.  Whole calls, gradients not cached, run by run / by the row's wave (us, uniform and Zipf(1.2)
+// ids): 1.2M indices of width 768 into 100,288 rows 1376 / 557 and 1160 / 1139; 256,000 of 768 into 32,000 rows 305 / 204
+// and 340 / 332; 64,000 of 3072 into 32,000 rows 209 / 183 and 227 / 214; 32,000 of 768 into 8000 rows 42 / 38 and 70 / 69.
+// With 1.5 indices per row 48,000 of 768 take 56 / 57 us.  Fewer indices than kDenseRows leave long waves alone on the
+// chip: 12,000 Zipf ones of 3072 into 1000 rows 49 / 53 us, 20,000 80 / 77 us.
+constexpr int kDirectDense = 2 * kRowsPerPartial;
+constexpr int64_t kDenseMean = 2;
+constexpr int64_t kDenseRows = 16384;
 constexpr int kRunBlock = 40;              // sorted positions whose runs a wave sums, for one step of 512 columns
 constexpr int kFewBlock = 8;               // the same, few indices
 constexpr int kMaxWaves = 1 << 20;         // most waves that sum runs (they stride beyond that)
@@ -339,11 +349,11 @@ __device__ __forceinline__ uint16_t col(const u4& x, int k) { return (uint16_t)(
 typedef float f4 __attribute__((ext_vector_type(4)));
 typedef f4 f4_any __attribute__((aligned(4)));
 
-// The runs that start at sorted places [p0, p0 + block) and belong to ids of more than kDirect occurrences, columns
+// The runs that start at sorted places [p0, p0 + block) and belong to ids of more than DIRECT occurrences, columns
 // [512 step, 512 (step + 1)) of each; the wave of the last step also takes the last D % 8 columns, one per lane.  A
 // run's rows (at most 10, or 16 for few indices) are loaded together and summed in order.  The sum of an id's only run
 // is its row; otherwise the fp32 partial goes to the run's slot, and the wave of step 0 lists the id for the chain pass.
-template <bool FEW>
+template <bool FEW, int DIRECT>
 __device__ __forceinline__ void sum_runs(int64_t p0, int step, bool last_step, const uint16_t* __restrict__ grad, int64_t D,
                                          const Ent* __restrict__ ent, int64_t padding_idx, float scale, int scale_mode,
                                          int64_t valid, uint16_t* __restrict__ out, int* __restrict__ counts,
@@ -358,7 +368,7 @@ __device__ __forceinline__ void sum_runs(int64_t p0, int step, bool last_step, c
     if (p >= 0 && p < valid && lane < 1 + kBlock + kRows) e = ent[p];
     const int prev = __shfl_up(e.pos, 1);
     const bool begins = p >= e.lo && e.n > 0 && run_starts<FEW>((int)p, e.lo, e.pos, prev);
-    const bool mine = begins && lane >= 1 && lane <= kBlock && e.n > kDirect && (int64_t)e.id != padding_idx;
+    const bool mine = begins && lane >= 1 && lane <= kBlock && e.n > DIRECT && (int64_t)e.id != padding_idx;
     const bool single = !FEW && e.n <= kRowsPerPartial;
     if (mine && !single && p == e.lo && step == 0) {
         const bool is_short = (FEW ? e.n : (e.n + kRowsPerPartial - 1) / kRowsPerPartial) <= kWaveChainRuns;
@@ -475,9 +485,63 @@ __device__ __forceinline__ void sum_direct(const int* at, int n, const uint16_t*
     }
 }
 
-// Workgroups [0, run_waves): runs of ids of more than kDirect occurrences; then one per output row, which writes it
-// unless the runs do.
-template <bool FEW, int G>
+// One output row of n <= kDirectDense occurrences, the sorted places from lo on, group by group: the rows of a run (at
+// most 10) are loaded together.
+__device__ __forceinline__ void sum_row_runs(const Ent* __restrict__ ent, int lo, int n,
+                                             const uint16_t* __restrict__ grad, int64_t D, float scale, int scale_mode,
+                                             bool wide, uint16_t* __restrict__ orow) {
+    const int lane = threadIdx.x, ng = (int)(D / 8);
+    const int pos = lane < n ? ent[lo + lane].pos : 0;
+    int at[kDirectDense];
+#pragma unroll
+    for (int u = 0; u < kDirectDense; ++u) at[u] = __builtin_amdgcn_readlane(pos, u);
+    for (int gi = lane; gi < ng; gi += kEmbThreads) {
+        float acc[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) acc[k] = 0.0f;
+#pragma unroll
+        for (int k0 = 0; k0 < kDirectDense; k0 += kRowsPerPartial) {
+            if (k0 < n) {
+                u4 x[kRowsPerPartial];
+#pragma unroll
+                for (int u = 0; u < kRowsPerPartial; ++u)
+                    if (k0 + u < n) x[u] = load8(grad + (int64_t)at[k0 + u] * D + (int64_t)gi * 8);
+                float part[8];
+#pragma unroll
+                for (int k = 0; k < 8; ++k) part[k] = 0.0f;
+#pragma unroll
+                for (int u = 0; u < kRowsPerPartial; ++u) {
+                    if (k0 + u < n) {
+#pragma unroll
+                        for (int k = 0; k < 8; ++k) part[k] = part[k] + grad_elem(col(x[u], k), scale, scale_mode);
+                    }
+                }
+#pragma unroll
+                for (int k = 0; k < 8; ++k) acc[k] = acc[k] + part[k];
+            }
+        }
+        row_store8(orow, wide, ng * 16, gi * 16, finish8(acc, scale, scale_mode));
+    }
+    const int d = ng * 8 + lane;
+    if (d < D) {
+        float acc = 0.0f;
+#pragma unroll
+        for (int k0 = 0; k0 < kDirectDense; k0 += kRowsPerPartial) {
+            if (k0 < n) {
+                float part = 0.0f;
+#pragma unroll
+                for (int u = 0; u < kRowsPerPartial; ++u)
+                    if (k0 + u < n) part = part + grad_elem(grad[(int64_t)at[k0 + u] * D + d], scale, scale_mode);
+                acc = acc + part;
+            }
+        }
+        orow[d] = finish(acc, scale, scale_mode);
+    }
+}
+
+// Workgroups [0, run_waves): runs of ids of more than kDirect occurrences (DENSE: kDirectDense); then one per output row,
+// which writes it unless the runs do.
+template <bool FEW, int G, bool DENSE>
 __global__ __launch_bounds__(kEmbThreads) void emb_rows_kernel(const uint16_t* __restrict__ grad, int64_t D, int64_t V,
                                                                const Ent* __restrict__ ent,
                                                                const int2* __restrict__ info, int64_t padding_idx,
@@ -492,8 +556,8 @@ __global__ __launch_bounds__(kEmbThreads) void emb_rows_kernel(const uint16_t* _
         const int step = b % steps;
         const int64_t valid = counts[2];
         for (int64_t p0 = (int64_t)(b / steps) * kBlock; p0 < valid; p0 += (int64_t)(run_waves / steps) * kBlock)
-            sum_runs<FEW>(p0, step, step == steps - 1, grad, D, ent, padding_idx, scale, scale_mode, valid, out, counts,
-                          short_list, long_list, parts);
+            sum_runs<FEW, DENSE ? kDirectDense : kDirect>(p0, step, step == steps - 1, grad, D, ent, padding_idx, scale,
+                                                          scale_mode, valid, out, counts, short_list, long_list, parts);
         return;
     }
     // Row of workgroup b (run_waves is a multiple of 8: workgroup b runs on XCD b mod 8): each XCD takes kSpan consecutive
@@ -517,6 +581,8 @@ __global__ __launch_bounds__(kEmbThreads) void emb_rows_kernel(const uint16_t* _
 #pragma unroll
             for (int u = 0; u < kDirect; ++u) at[u] = __builtin_amdgcn_readlane(pos, u);
             sum_direct<FEW, G, kDirect>(at, r.y, grad, D, scale, scale_mode, wide, orow);
+        } else if (DENSE && r.y <= kDirectDense) {
+            sum_row_runs(ent, r.x, r.y, grad, D, scale, scale_mode, wide, orow);
         }
     }
 }
@@ -740,6 +806,8 @@ EmbWorkspace emb_workspace(void* base, int64_t R, int64_t D, int64_t V) {
     return w;
 }
 
+bool dense(int64_t R, int64_t V) { return R >= kDenseRows && R >= kDenseMean * V; }
+
 struct RowsCall {
     const uint16_t* grad;
     int64_t R, D, V, padding_idx;
@@ -751,7 +819,7 @@ struct RowsCall {
 };
 
 // The rows launch, with as many column groups per lane as the row needs, at most 6 (D 3072).
-template <bool FEW, int G>
+template <bool FEW, int G, bool DENSE = false>
 void launch_rows_g(const RowsCall& c, const EmbWorkspace& w) {
     const int64_t steps = (c.D / 8 + kEmbThreads - 1) / kEmbThreads, step_waves = steps > 0 ? steps : 1;
     int64_t run_waves = 0;
@@ -762,7 +830,7 @@ void launch_rows_g(const RowsCall& c, const EmbWorkspace& w) {
     }
     const int64_t spans = (c.V + 8 * kSpan - 1) / (8 * kSpan) * (8 * kSpan);
     const int64_t rows = spans < kMaxRowWaves ? spans : kMaxRowWaves;
-    hipLaunchKernelGGL((emb_rows_kernel<FEW, G>), dim3((unsigned)(run_waves + rows)), dim3(kEmbThreads), c.lds, c.st,
+    hipLaunchKernelGGL((emb_rows_kernel<FEW, G, DENSE>), dim3((unsigned)(run_waves + rows)), dim3(kEmbThreads), c.lds, c.st,
                        c.grad, c.D, c.V, w.ent, w.info, c.padding_idx, c.scale, c.scale_mode, c.out, (int)run_waves,
                        (int)step_waves, w.counts, w.short_list, w.long_list, w.parts);
 }
@@ -835,6 +903,7 @@ int z1_embedding_backward(const int64_t* ids, const uint16_t* grad, int64_t R, i
     if (rc) return rc;
     const bool few = R < kSortMinRows;                  // aten's kernel for few indices: its order
     if (few) launch_rows<true>(c, w);
+    else if (dense(R, V)) launch_rows_g<false, 1, true>(c, w);
     else launch_rows<false>(c, w);
     e = hipGetLastError();
     if (e != hipSuccess) return (int)e;

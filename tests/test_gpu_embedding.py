@@ -128,6 +128,34 @@ def test_occurrence_counts(pkg, dev, D, few, V):
         assert np.array_equal(bits(out), bits(ref)), pad
 
 
+# the bounds of a dense table: 2 indices per row, 16,384 indices
+@pytest.mark.parametrize('R,V', [(16383, 700), (16384, 700), (16384, 8192), (16384, 8193), (40000, 1500), (60000, 30000)])
+@pytest.mark.parametrize('D', [5, 520, 3083])
+def test_dense_tables(pkg, dev, R, V, D):
+    """Tables of many indices per row, where the wave of a row sums up to 20 occurrences: ids with as many as the parts of
+    the work split at, ids at both ends, an output off the 16-byte boundary, a heavy and a light padding row, all three
+    placements of the scale.  Bit-exact against aten."""
+    from faster_yoco_amd import embedding
+    rng = np.random.default_rng(R + V + D)
+    counts = [1, 2, 4, 5, 9, 10, 11, 19, 20, 21, 30, 31, 320, 321]
+    where = rng.choice(np.arange(1, V - 1), len(counts), replace=False)
+    rest = np.setdiff1d(np.arange(V), where)
+    ids = np.concatenate([np.repeat(where, counts), rng.choice(rest, R - sum(counts))])
+    ids = torch.from_numpy(rng.permutation(ids).astype(np.int64)).to(dev)
+    g = (torch.randn(R, D, device=dev) * 1e-2).to(torch.bfloat16)
+    aten = torch.ops.aten.embedding_dense_backward
+    for pad in (-1, int(where[-1]), int(where[8])):
+        ref = aten(g, ids, V, pad, False)
+        out = torch.full((V * D + 1,), 7.0, dtype=torch.bfloat16, device=dev)[pad % 2:][:V * D].view(V, D)
+        embedding.embedding_dense_backward(g, ids, V, pad, out=out)
+        torch.cuda.synchronize()
+        assert np.array_equal(bits(out), bits(ref)), pad
+    got, got_ce = (f(g, ids, V, 1, 8) for f in (embedding.owner_embedding_grad, embedding.ce_owner_embedding_grad))
+    ref, ref_ce = aten(g, ids, V, 1, False) * 0.125, aten(g * 0.125, ids, V, 1, False)
+    torch.cuda.synchronize()
+    assert np.array_equal(bits(got), bits(ref)) and np.array_equal(bits(got_ce), bits(ref_ce))
+
+
 @pytest.mark.parametrize('V', [2 ** 25, 2 ** 25 + 1, 2 ** 26 + 2000])
 def test_more_rows_than_one_round_of_waves(pkg, dev, V):
     """Tables of 2^25 rows (the most one launch has waves for) and more, past the former limit of one grid as well:
