@@ -196,6 +196,23 @@ def test_order_of_occurrences(pkg, dev, R, V):
     assert np.array_equal(bits(got), bits(ref))
 
 
+@pytest.mark.parametrize('step', [2, 256, 512, 514, 1024, 4096])
+@pytest.mark.parametrize('V', [1000, 65536, 100288, 524288])
+def test_ids_a_step_apart(pkg, dev, V, step):
+    """Multiples of a step, which the one-launch ordering spreads over its buckets by turning each round of them: bit-exact
+    against aten, an id next to each among them."""
+    from faster_yoco_amd import embedding
+    rng = np.random.default_rng(V + step)
+    ids = rng.integers(0, V, 6000) // step * step
+    ids[::97] = np.minimum(ids[::97] + 1, V - 1)
+    ids = torch.from_numpy(ids.astype(np.int64)).to(dev)
+    g = (torch.randn(6000, 16, device=dev) * 1e-2).to(torch.bfloat16)
+    ref = torch.ops.aten.embedding_dense_backward(g, ids, V, -1, False)
+    got = embedding.embedding_dense_backward(g, ids, V, -1)
+    torch.cuda.synchronize()
+    assert np.array_equal(bits(got), bits(ref))
+
+
 @pytest.mark.parametrize('R', [700, 4000])
 @pytest.mark.parametrize('D', [1, 7, 8, 9, 511, 512, 513, 1027, 1536, 2563, 3079, 4104, 6151])
 def test_row_widths(pkg, dev, R, D):
