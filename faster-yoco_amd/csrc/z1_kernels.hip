@@ -147,15 +147,19 @@ __device__ __forceinline__ void st_stream(float* base, int bytes, int off, f4 x)
     const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(base, 0, bytes, 0x00020000);
     __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, x), r, off, 0, kStreamStorePolicy);
 }
-// (buffer stores want dword addresses: four bf16 at an odd element go out as a nontemporal global store)
 __device__ __forceinline__ void st_stream(uint16_t* base, int bytes, int off, u2 x) {
-    if (reinterpret_cast<uintptr_t>(base) & 3) {
-        __builtin_nontemporal_store((AnyAlign<u2>::type)x,
-                                    (Z1_GLOBAL AnyAlign<u2>::type*)(reinterpret_cast<char*>(base) + off));
-        return;
-    }
     const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(base, 0, bytes, 0x00020000);
     __builtin_amdgcn_raw_buffer_store_b64(x, r, off, 0, kStreamStorePolicy);
+}
+// Four bf16 anywhere: buffer stores want dword addresses, so at an odd element they go out as a nontemporal global store.
+// The choice costs where stores are all a wave does beside one round of loads (the cast pass over 120M elements 108.4 us
+// without it, 111.2 with; the sum of two contributions 198.0 / 201.1): those kernels take st_stream.
+__device__ __forceinline__ void st_stream_any(uint16_t* base, int bytes, int off, u2 x) {
+    if (reinterpret_cast<uintptr_t>(base) & 3)
+        __builtin_nontemporal_store((AnyAlign<u2>::type)x,
+                                    (Z1_GLOBAL AnyAlign<u2>::type*)(reinterpret_cast<char*>(base) + off));
+    else
+        st_stream(base, bytes, off, x);
 }
 
 // Chunk of workgroup b: undoes the round-robin dispatch over the 8 XCDs (workgroup b runs on XCD b mod 8), so that
@@ -262,7 +266,7 @@ __device__ __forceinline__ void adam_chunk(const Row& r, float* go, int64_t base
             st_stream(r.v + base, (int)kChunk * 4, o4, v[u]);
             if (r.p16) {
                 const u2 h = u2{pack_bf16(p[u][0], p[u][1]), pack_bf16(p[u][2], p[u][3])};
-                st_stream(r.p16 + base, (int)kChunk * 2, o2, h);
+                st_stream_any(r.p16 + base, (int)kChunk * 2, o2, h);
             }
             if (GOUT && go) st_stream(go + base, (int)kChunk * 4, o4, g[u]);
         }
@@ -721,9 +725,9 @@ __global__ __launch_bounds__(kWave) void owner_sum_kernel(Srcs s, int64_t n, flo
         u2 o;
 #pragma unroll
         for (int w = 0; w < kSumVec / 2; ++w) o[w] = pack_bf16(a[2 * w] * scale, a[2 * w + 1] * scale);
-        // the chunk's first element (the range's, for a first chunk the shift moves before it): every lane of this
-        // path writes [e0, e0 + 4) within [cb, cb + kSumChunk)
-        const int64_t cb = c * kSumChunk - shift > 0 ? c * kSumChunk - shift : 0;
+        // the chunk's first element, on a line of the average (before the range's first element for a first chunk that the
+        // shift moves there): every lane of this path writes [e0, e0 + 4) within [cb, cb + kSumChunk)
+        const int64_t cb = c * kSumChunk - shift;
         st_stream(out + cb, (int)kSumChunk * 2, (int)(e0 - cb) * 2, o);
         if (out_sum) st_stream(out_sum + cb, (int)kSumChunk * 4, (int)(e0 - cb) * 4, f4{a[0], a[1], a[2], a[3]});
         if (wave_partials) {
@@ -903,6 +907,7 @@ __global__ __launch_bounds__(kWave) void scale_up_kernel(const uint16_t* __restr
     for (int64_t e = e0 + lane; e < e1; e += kWave) g32[e] = bf16_to_f32(g16[e]) * f;
 }
 
+template <bool ODD>      // p16 at an odd element
 __global__ __launch_bounds__(kWave) void cast_bf16_kernel(const float* __restrict__ p32, uint16_t* __restrict__ p16,
                                                           int64_t n, int vec) {
     const int64_t e0 = chunk_of_block(blockIdx.x, gridDim.x) * kPassChunk;
@@ -912,9 +917,12 @@ __global__ __launch_bounds__(kWave) void cast_bf16_kernel(const float* __restric
 #pragma unroll
         for (int u = 0; u < 2; ++u) a[u] = ld(reinterpret_cast<const f4*>(p32 + e0 + u * (kPassChunk / 2)) + lane);
 #pragma unroll
-        for (int u = 0; u < 2; ++u)
-            st_stream(p16 + e0, (int)kPassChunk * 2, (int)((u * (kPassChunk / 2) + lane * 4) * 2),
-                      u2{pack_bf16(a[u].x, a[u].y), pack_bf16(a[u].z, a[u].w)});
+        for (int u = 0; u < 2; ++u) {
+            const int off = (int)((u * (kPassChunk / 2) + lane * 4) * 2);
+            const u2 h = u2{pack_bf16(a[u].x, a[u].y), pack_bf16(a[u].z, a[u].w)};
+            if (ODD) st_stream_any(p16 + e0, (int)kPassChunk * 2, off, h);
+            else st_stream(p16 + e0, (int)kPassChunk * 2, off, h);
+        }
         return;
     }
     const int64_t e1 = e0 + kPassChunk < n ? e0 + kPassChunk : n;
@@ -1652,8 +1660,12 @@ int z1_cast_bf16(const float* p32, uint16_t* p16, int64_t n, void* stream) {
     const int64_t chunks = (n + kPassChunk - 1) / kPassChunk;
     if (chunks > INT32_MAX) return Z1_E_SIZE;
     const int vec = aligned(p32, 4) && aligned(p16, 2);
-    hipLaunchKernelGGL(cast_bf16_kernel, dim3((unsigned)chunks), dim3(kWave), 0, static_cast<hipStream_t>(stream),
-                       p32, p16, n, vec);
+    if (aligned(p16, 4))
+        hipLaunchKernelGGL(cast_bf16_kernel<false>, dim3((unsigned)chunks), dim3(kWave), 0,
+                           static_cast<hipStream_t>(stream), p32, p16, n, vec);
+    else
+        hipLaunchKernelGGL(cast_bf16_kernel<true>, dim3((unsigned)chunks), dim3(kWave), 0,
+                           static_cast<hipStream_t>(stream), p32, p16, n, vec);
     return launch_status();
 }
 
