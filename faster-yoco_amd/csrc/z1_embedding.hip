@@ -107,15 +107,18 @@ __global__ void emb_keys_kernel(const int64_t* __restrict__ ids, int64_t R, int6
 }
 
 // info[t] = (where, count) of id t's occurrences, for t in [0, V): their first sorted place, or the position of the
-// only one.  Independent binary searches over the sorted keys, one thread per t (the latency of the searches overlaps).
-__device__ __forceinline__ int32_t lower_bound(const uint32_t* __restrict__ sorted, int64_t R, uint32_t key) {
-    int64_t lo = 0, hi = R;
-    while (lo < hi) {
-        const int64_t mid = (lo + hi) >> 1;
-        if (sorted[mid] < key) lo = mid + 1;
-        else hi = mid;
+// only one.  Independent binary searches over the sorted keys, one thread per t (the latency of the searches overlaps),
+// for both ends of t's occurrences side by side (one after the other 7.6 us for 65,536 keys, 5.4 for one end alone).
+__device__ __forceinline__ int2 key_range(const uint32_t* __restrict__ sorted, int64_t R, uint32_t key) {
+    int lo = 0, hi = 0;                         // the first places of keys >= key and > key lie in [lo, lo + n], [hi, hi + n]
+    for (int n = (int)R; n > 0;) {
+        const int half = n >> 1;
+        const uint32_t a = sorted[lo + half], b = sorted[hi + half];
+        if (a < key) lo += n - half;
+        if (b <= key) hi += n - half;
+        n = half;
     }
-    return (int32_t)lo;
+    return int2{lo, hi};
 }
 
 __global__ void emb_row_ranges_kernel(const uint32_t* __restrict__ sorted, const int32_t* __restrict__ spos, int64_t R,
@@ -123,7 +126,8 @@ __global__ void emb_row_ranges_kernel(const uint32_t* __restrict__ sorted, const
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t < 2) counts[t] = 0;                   // the rows kernel appends to the chain pass's lists after this kernel
     if (t >= V) return;
-    const int32_t lo = lower_bound(sorted, R, (uint32_t)t), hi = lower_bound(sorted, R, (uint32_t)t + 1);
+    const int2 r = key_range(sorted, R, (uint32_t)t);
+    const int32_t lo = r.x, hi = r.y;
     info[t] = int2{hi - lo == 1 ? spos[lo] : lo, hi - lo};
     if (t == V - 1) counts[2] = hi;             // the ids inside [0, V)
 }
