@@ -58,6 +58,10 @@ constexpr int kDirectDense = 2 * kRowsPerPartial;
 constexpr int64_t kDenseMean = 2;
 constexpr int64_t kDenseRows = 16384;
 constexpr int kRunBlock = 40;              // sorted positions whose runs a wave sums, for one step of 512 columns
+// In a dense table of this many indices per row or more most ids are summed by runs, and half the block gives twice the
+// waves: 65,536 ids of width 256 into 256 rows, uniform / Zipf, 78.5 / 107.4 us with 40, 72.1 / 101.8 with 20; 131,072 of 768
+// into 1000 rows 152 / 195 and 147 / 187.  At 8 per row it loses (262,144 of 768 into 32,000 rows 205 / 334 and 209 / 337).
+constexpr int64_t kShortBlockMean = 16;
 constexpr int kFewBlock = 8;               // the same, few indices
 constexpr int kMaxWaves = 1 << 20;         // most waves that sum runs (they stride beyond that)
 // Consecutive rows of one XCD: spans of 32 to 128 rows measure alike, single rows round robin 144 / 153; one eighth of the
@@ -366,21 +370,21 @@ typedef f4 f4_any __attribute__((aligned(4)));
 // run's rows (at most 10, or 16 for few indices) are loaded together and summed in order.  The sum of an id's only run
 // is its row; otherwise the fp32 partial goes to the run's slot, and the wave of step 0 lists the id for the chain pass.
 template <bool FEW, int DIRECT>
-__device__ __forceinline__ void sum_runs(int64_t p0, int step, bool last_step, const uint16_t* __restrict__ grad, int64_t D,
+__device__ __forceinline__ void sum_runs(int64_t p0, int block, int step, bool last_step, const uint16_t* __restrict__ grad, int64_t D,
                                          const Ent* __restrict__ ent, int64_t padding_idx, float scale, int scale_mode,
                                          int64_t valid, uint16_t* __restrict__ out, int* __restrict__ counts,
                                          int32_t* __restrict__ short_list, int32_t* __restrict__ long_list,
                                          float* __restrict__ parts) {
-    constexpr int kBlock = FEW ? kFewBlock : kRunBlock, kRows = FEW ? kFewRowsChunk : kRowsPerPartial;
-    static_assert(1 + kBlock + kRows <= kWave, "the lanes hold every place a run of the block can reach");
+    constexpr int kRows = FEW ? kFewRowsChunk : kRowsPerPartial;
+    static_assert(1 + (FEW ? kFewBlock : kRunBlock) + kRows <= kWave, "the lanes hold every place a run of the block can reach");
     const int lane = threadIdx.x;
     // lane i: place p0 - 1 + i
     const int64_t p = p0 - 1 + lane;
     Ent e = Ent{0, 0, 0, 0};
-    if (p >= 0 && p < valid && lane < 1 + kBlock + kRows) e = ent[p];
+    if (p >= 0 && p < valid && lane < 1 + block + kRows) e = ent[p];
     const int prev = __shfl_up(e.pos, 1);
     const bool begins = p >= e.lo && e.n > 0 && run_starts<FEW>((int)p, e.lo, e.pos, prev);
-    const bool mine = begins && lane >= 1 && lane <= kBlock && e.n > DIRECT && (int64_t)e.id != padding_idx;
+    const bool mine = begins && lane >= 1 && lane <= block && e.n > DIRECT && (int64_t)e.id != padding_idx;
     const bool single = !FEW && e.n <= kRowsPerPartial;
     if (mine && !single && p == e.lo && step == 0) {
         const bool is_short = (FEW ? e.n : (e.n + kRowsPerPartial - 1) / kRowsPerPartial) <= kWaveChainRuns;
@@ -558,17 +562,17 @@ __global__ __launch_bounds__(kEmbThreads) void emb_rows_kernel(const uint16_t* _
                                                                const Ent* __restrict__ ent,
                                                                const int2* __restrict__ info, int64_t padding_idx,
                                                                float scale, int scale_mode, uint16_t* __restrict__ out,
-                                                               int run_waves, int steps, int* __restrict__ counts,
+                                                               int run_waves, int steps, int block,
+                                                               int* __restrict__ counts,
                                                                int32_t* __restrict__ short_list,
                                                                int32_t* __restrict__ long_list,
                                                                float* __restrict__ parts) {
     if ((int)blockIdx.x < run_waves) {
         const int b = (int)blockIdx.x;
-        constexpr int kBlock = FEW ? kFewBlock : kRunBlock;
-        const int step = b % steps;
+        const int step = b % steps, run_block = DENSE ? block : FEW ? kFewBlock : kRunBlock;
         const int64_t valid = counts[2];
-        for (int64_t p0 = (int64_t)(b / steps) * kBlock; p0 < valid; p0 += (int64_t)(run_waves / steps) * kBlock)
-            sum_runs<FEW, DENSE ? kDirectDense : kDirect>(p0, step, step == steps - 1, grad, D, ent, padding_idx, scale,
+        for (int64_t p0 = (int64_t)(b / steps) * run_block; p0 < valid; p0 += (int64_t)(run_waves / steps) * run_block)
+            sum_runs<FEW, DENSE ? kDirectDense : kDirect>(p0, run_block, step, step == steps - 1, grad, D, ent, padding_idx, scale,
                                                           scale_mode, valid, out, counts, short_list, long_list, parts);
         return;
     }
@@ -835,16 +839,17 @@ template <bool FEW, int G, bool DENSE = false>
 void launch_rows_g(const RowsCall& c, const EmbWorkspace& w) {
     const int64_t steps = (c.D / 8 + kEmbThreads - 1) / kEmbThreads, step_waves = steps > 0 ? steps : 1;
     int64_t run_waves = 0;
+    int block = FEW ? kFewBlock : kRunBlock;
     if (c.R > kDirect) {
-        constexpr int kBlock = FEW ? kFewBlock : kRunBlock;
-        const int64_t blocks = (c.R + kBlock - 1) / kBlock, most = kMaxWaves / step_waves;      // steps <= 32,768
+        if (DENSE && c.R >= kShortBlockMean * c.V) block = kRunBlock / 2;
+        const int64_t blocks = (c.R + block - 1) / block, most = kMaxWaves / step_waves;      // steps <= 32,768
         run_waves = ((blocks < most ? blocks : most) + 7) / 8 * 8 * step_waves;
     }
     const int64_t spans = (c.V + 8 * kSpan - 1) / (8 * kSpan) * (8 * kSpan);
     const int64_t rows = spans < kMaxRowWaves ? spans : kMaxRowWaves;
     hipLaunchKernelGGL((emb_rows_kernel<FEW, G, DENSE>), dim3((unsigned)(run_waves + rows)), dim3(kEmbThreads), c.lds, c.st,
                        c.grad, c.D, c.V, w.ent, w.info, c.padding_idx, c.scale, c.scale_mode, c.out, (int)run_waves,
-                       (int)step_waves, w.counts, w.short_list, w.long_list, w.parts);
+                       (int)step_waves, block, w.counts, w.short_list, w.long_list, w.parts);
 }
 
 template <bool FEW>
