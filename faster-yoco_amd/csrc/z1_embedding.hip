@@ -93,7 +93,8 @@ __device__ __forceinline__ float bf16f(uint16_t h) { return __uint_as_float((uin
 // Round to nearest even, with gfx950's conversion (a NaN keeps its sign and payload: finish makes aten's of it).
 __device__ __forceinline__ uint16_t bf16r(float x) { return __builtin_bit_cast(uint16_t, (__bf16)x); }
 
-// One place of the order (each id's occurrences next to each other, by position): the occurrence's position, its id, and the id's first place and count.
+// One place of the order (each id's occurrences next to each other, by position): the occurrence's position, its id, and
+// the id's first place and count.
 struct Ent {
     int32_t pos;
     uint32_t id;
@@ -370,13 +371,13 @@ typedef f4 f4_any __attribute__((aligned(4)));
 // run's rows (at most 10, or 16 for few indices) are loaded together and summed in order.  The sum of an id's only run
 // is its row; otherwise the fp32 partial goes to the run's slot, and the wave of step 0 lists the id for the chain pass.
 template <bool FEW, int DIRECT>
-__device__ __forceinline__ void sum_runs(int64_t p0, int block, int step, bool last_step, const uint16_t* __restrict__ grad, int64_t D,
-                                         const Ent* __restrict__ ent, int64_t padding_idx, float scale, int scale_mode,
+__device__ __forceinline__ void sum_runs(int64_t p0, int block, int step, bool last_step,
+                                         const uint16_t* __restrict__ grad, int64_t D, const Ent* __restrict__ ent, int64_t padding_idx, float scale, int scale_mode,
                                          int64_t valid, uint16_t* __restrict__ out, int* __restrict__ counts,
                                          int32_t* __restrict__ short_list, int32_t* __restrict__ long_list,
                                          float* __restrict__ parts) {
     constexpr int kRows = FEW ? kFewRowsChunk : kRowsPerPartial;
-    static_assert(1 + (FEW ? kFewBlock : kRunBlock) + kRows <= kWave, "the lanes hold every place a run of the block can reach");
+    static_assert(1 + (FEW ? kFewBlock : kRunBlock) + kRows <= kWave, "lanes for every place a run of the block reaches");
     const int lane = threadIdx.x;
     // lane i: place p0 - 1 + i
     const int64_t p = p0 - 1 + lane;

@@ -36,7 +36,7 @@
 //   * No atomic orders or sums anything; nothing but vector memory instructions write memory.  (The norm's final
 //     reduction is a second, one-workgroup launch: folding it into the last workgroup of the norm grid to finish, with
 //     an arrival counter, measured 75 us slower per step, because the grid's 2048 workgroups finish together.  Small
-//     tables take a grid of at most 64, where it is faster: norm_small_kernel.)
+//     tables take a grid of at most kNormSmallGrid, where it is faster: norm_small_kernel.)
 //
 // Numerics follow the header: one rounding per fp32 operation, explicit FMAs where the reference has them,
 // correctly rounded division and square root (built with -fhip-fp32-correctly-rounded-divide-sqrt, no fast math,
@@ -90,6 +90,8 @@ struct Row {
     uint16_t* p16;
     int64_t n;
     int64_t chunk0;
+    // Pointers off their elements' boundaries, which no tensor has but a C caller's row may, take the element loops of the
+    // rows' last chunks throughout.
     int32_t vec;        // bit 0: g on its element boundary; bit 1: p, m, v, p16 as well
     int32_t pmv_aligned;    // p, m, v, p16 on their element boundaries (vec's bit 1 needs g there too)
 };
@@ -107,7 +109,6 @@ struct AdamK {
 // The update's big stores go out through st_stream below, which adds the system-scope bits.
 #define Z1_GLOBAL __attribute__((address_space(1)))
 
-//
 // The vectors need no more than their elements' alignment (fp32 4, bf16 2 bytes): gfx950 loads and stores 8 and 16 bytes
 // at any address, in the same instructions, so a parameter packed behind an odd-sized one keeps the vector path; its
 // lines that straddle two waves are fetched twice.  Measured on the drop-in update of 13.7M parameters in 26 odd-sized
@@ -231,7 +232,7 @@ __device__ __forceinline__ float load_g1(const void* g, int64_t i) {
 // the update consumes, is also stored to gout[row] (NULL: not for that row) -- the FP32 gradient the reference's
 // scale pass writes before its Adam reads it back (yoco/tasks/zero1_fast.py:175-192, fused_adam_cast.py:75-89).
 // One chunk of a row: elements [base, base + min(r.n - base, kChunk)) of r; the vector path when the chunk is whole
-// and the row's pointers are aligned, else an element-wise loop.
+// and the row's pointers are on their elements, else an element-wise loop.
 template <int GDT, int MODE, bool GOUT>
 __device__ __forceinline__ void adam_chunk(const Row& r, float* go, int64_t base, int lane, float f, const AdamK& k) {
     const int64_t rem = r.n - base;
@@ -588,13 +589,15 @@ __global__ __launch_bounds__(NT) void sumsq_kernel(const Row* __restrict__ rows,
 // The norm and the scalar tail of a small table in one launch: the same decomposition, partials and final order (the
 // same bits) as sumsq_kernel and scalars_kernel, whose 2048 workgroups are here virtual ones, kNormSmallWaves / W of
 // them per real workgroup; only those with chunks are formed (`used`), the others' partials are zeros.  The last
-// workgroup to arrive at the launch's counter (the workspace's, in the table) adds the partials.  They cross the XCDs as system-scope stores and loads
-// (a wave's stores have reached memory before it counts its workgroup in), so no L2 is written back or invalidated.
-// No workgroup waits for another, and the counter is left at zero.
+// workgroup to arrive at the launch's counter (the workspace's, in the table) adds the partials.  They cross the XCDs
+// as system-scope stores and loads (a wave's stores have reached memory before it counts its workgroup in), so no L2 is
+// written back or invalidated.  No workgroup waits for another, and the counter is left at zero.
 // Latency bounds it: launch, row, chunk, arrival, partials.  Norm and clip back to back in a graph, against the two
-// launches: FP32 36,928 elements 6.2 against 8.0 us, 262,144 6.6 / 8.2, 524,288 7.6 / 8.4; BF16 1M 7.3 / 7.8, 2M
-// 8.7 / 8.1, and a launch of host time less (the 36,928-element update 19.0 -> 17.0 us).  Grids past kNormSmallGrid, or
-// more than one round per workgroup, lose: FP32 1M 9.4 (256 workgroups) and 10.6 (64, four rounds) against 8.4 us.
+// launches: FP32 36,928 elements 5.8 against 8.0 us, 262,144 6.2 / 7.9, 524,288 7.2 / 8.1; BF16 1M 6.8 / 7.6, 1.8M
+// 7.8 / 7.8, 2.0M 8.1 / 7.8, 2.1M 7.9 / 7.9.  Where the two meet by themselves, an update with Adam behind is still the
+// faster with one: BF16 2.0M captured 21.7 against 22.2 us, eager (a launch of host time less) 17.7 against 19.5.  Grids
+// past kNormSmallGrid, or more than one round per workgroup, lose: FP32 1M 9.4 (256 workgroups) and 10.6 (64, four
+// rounds) against 8.4 us.
 constexpr int kNormSmallThreads = 1024;
 constexpr int kNormSmallWaves = kNormSmallThreads / kWave;
 constexpr int kNormSmallGrid = 128;
@@ -1037,7 +1040,7 @@ int occupancy_lds(int dev, int per_cu, size_t* bytes) { return ::occupancy_lds(d
 
 // Whether the table's rows, as the host last bound them, are one flat allocation per stream: row i's g, p, m, v
 // (and p16, if any row has one) start where row i - 1's end, every row has p, m and v, and the first row's pointers
-// are aligned for the vector path.  Then a whole-table Adam launch walks the buffers directly (adam_flat_kernel).
+// are on their elements.  Then a whole-table Adam launch walks the buffers directly (adam_flat_kernel).
 static void set_contig(z1_table* t) {
     t->contig = 0;
     const std::vector<Row>& h = t->host_rows;
@@ -1306,8 +1309,7 @@ int z1_table_set_grad_out(z1_table* table, float* const* g32, int nrows, void* s
     int rc = check_table_device(table, &dev);
     if (rc) return rc;
     GradBind b;
-    b.count = 0;
-    b.g_align = 16;
+    b.count = b.g_align = 0;                           // an output's alignment is looked at where it is written
     hipStream_t s = static_cast<hipStream_t>(stream);
     int set = 0;
     for (int i = 0; i < table->nrows; ++i) {

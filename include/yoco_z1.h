@@ -82,8 +82,8 @@ int z1_table_info(const z1_table* table, int64_t* numel, int64_t* nchunks, int* 
  * the stream like a launch (no allocation, no host synchronisation): launches enqueued after it read the new
  * gradients.  For callers whose gradient tensors are reallocated between steps while the parameters and optimizer
  * state stay put (the reference's zero_grad drops every gradient, yoco/tasks/zero1_fast.py:238-244), so that one
- * table made at set-up serves every step.  Rows may start at any element: the vector path assumes no more than the elements'
- * own alignment. */
+ * table made at set-up serves every step.  Rows may start at any element: the vector path assumes no more than the
+ * elements' own alignment. */
 int z1_table_set_grads(z1_table* table, const void* const* g, int nrows, void* stream);
 
 /* Gives the table FP32 gradient outputs: g32 is a HOST array of nrows device float pointers, one per row given to

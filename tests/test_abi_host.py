@@ -205,7 +205,9 @@ int main() {
         int got[8][64];
         std::vector<std::thread> threads;
         for (int k = 0; k < 8; ++k)
-            threads.emplace_back([&, k] { for (int i = 0; i < 64; ++i) got[k][(i + 8 * k) % 64] = t.slot(ws + (i + 8 * k) % 64); });
+            threads.emplace_back([&, k] {
+                for (int i = 8 * k; i < 8 * k + 64; ++i) got[k][i % 64] = t.slot(ws + i % 64);
+            });
         for (auto& x : threads) x.join();
         std::set<int> all;
         for (int i = 0; i < 64; ++i) {

@@ -337,8 +337,8 @@ def test_operators_follow_moved_state_tensors(pkg, dev):
 def test_adam_writes_the_scaled_gradients(pkg, dev, mode):
     """adam_cast with FP32 gradient outputs (z1_table_set_grad_out): BF16 gradients read times the factor, every
     output row holding fp32(float(g16) * factor) bit for bit as the scale pass writes it, and m / v / master / BF16
-    copy as scale pass + Adam give them.  Rows: aligned, an output off the 16-byte alignment (element-wise path), a
-    row without an output, an empty row, tails.  A later launch without outputs leaves them untouched."""
+    copy as scale pass + Adam give them.  Rows: aligned, an output off the 16-byte alignment, a row without an output,
+    an empty row, tails.  A later launch without outputs leaves them untouched."""
     from faster_yoco_amd import ops
     sizes = [5000, 256 * 9, 0, 33, 1 << 14]
     gen = torch.Generator(device='cpu').manual_seed(21 + mode)
@@ -348,7 +348,7 @@ def test_adam_writes_the_scaled_gradients(pkg, dev, mode):
     v = [(torch.randn(n, generator=gen) * 1e-8).abs().to(dev) for n in sizes]
     p16 = [torch.zeros(n, dtype=torch.bfloat16, device=dev) for n in sizes]
     raw = torch.full((sum(sizes) + 8,), -7.0, device=dev)
-    outs, off = [], 1                                       # row 1's output is 4 bytes off the vector alignment
+    outs, off = [], 1                                       # row 1's output is 4 bytes off the 16-byte alignment
     for i, n in enumerate(sizes):
         outs.append(torch.empty(0, device=dev) if i == 3 else raw[off:off + n])
         off += n
@@ -429,8 +429,8 @@ def test_gradient_outputs_either_side_of_the_row_search(pkg, dev, nrows):
 
 @pytest.mark.parametrize('total', [300_000, 150_000_000])
 def test_bf16_norm_pass(pkg, dev, total):
-    """The norm pass over BF16 gradients (chunk pairs, one 128-bit load per lane where a pair is whole and aligned,
-    the two chunks one after the other elsewhere): rows off the vector alignment, short rows, an empty row and, at
+    """The norm pass over BF16 gradients (runs of chunks in 128-bit loads where a run is whole, its chunks one after the
+    other elsewhere): rows at any element, short rows, an empty row and, at
     150M elements, the allocating loads of the MALL-kept part.  Its partials are the same bits on every run, their
     FP64 total is the FP32 pass's over the upcast values and the oracle's sequential sum to 1e-10 (sums of the same
     exact squares in other orders), and the norm is within 1e-6 of the exact one."""

@@ -129,7 +129,8 @@ def test_adam_tables_either_side_of_the_row_search(pkg, dev, nrows, g_bf16):
     check_rows(rows, got, g_bf16, 0.8125, 12)
 
 
-def test_adam_misaligned_rows_use_the_element_path(pkg, dev):
+def test_adam_rows_at_any_element(pkg, dev):
+    """Rows 1, 2 and 3 elements off the vectors' own alignment."""
     sizes = [4096 * 3, 5000, 17]
     rows = [rand_state(n, 300 + i) for i, n in enumerate(sizes)]
     for off in (1, 2, 3):
@@ -185,6 +186,39 @@ def test_adam_contiguous_rows_take_the_flat_launch(pkg, dev, g_bf16, mode, with_
     for a, b in zip(got, sep):
         assert all(same_f32(x, y) for x, y in zip(a[:3], b[:3]))
         assert (a[3] is None) == (b[3] is None) and (a[3] is None or same_bf16(a[3], b[3]))
+
+
+@pytest.mark.parametrize('g_bf16', [False, True])
+@pytest.mark.parametrize('at', [(1, 0, 0, 0, 0), (0, 1, 2, 3, 0), (0, 0, 0, 0, 1), (0, 0, 0, 0, 2), (3, 3, 3, 3, 3),
+                                (5, 2, 7, 1, 65)])
+def test_adam_flat_buffers_at_any_element(pkg, dev, at, g_bf16):
+    """The launch that walks flat buffers, its g, p, m, v and p16 beginning at any element of their allocations, several rows
+    with boundaries inside chunks: bit-exact against the oracle, as the same rows in separate allocations are, and
+    nothing written beside them."""
+    from faster_yoco_amd import ops
+    sizes = [1000, 333, 4096, 5, 256, 70001]
+    rows = []
+    for i, n in enumerate(sizes):
+        g, p, m, v = rand_state(n, 800 + i)
+        rows.append((oracle.bf16_rne(g) if g_bf16 else g, p, m, v))
+    flat, _ = flat_rows(rows, g_bf16, dev)
+    total, raw, moved = sum(sizes), [], []
+    for t, o in zip(flat, at):
+        buf = torch.full((total + 128,), 3.0, dtype=t.dtype, device=dev)
+        buf[o:o + total].copy_(t)
+        raw.append(buf)
+        moved.append(buf[o:o + total])
+    offsets = np.concatenate([[0], np.cumsum(sizes)[:-1]]).tolist()
+    table = ops.Table.flat(offsets, sizes, *moved)
+    bc1, bc2 = ops.bias_corrections(HP['beta1'], HP['beta2'], 7)
+    f = torch.tensor([0.625], dtype=torch.float32, device=dev)
+    ops.adam_cast(table, f, HP['lr'], HP['beta1'], HP['beta2'], HP['eps'], bc1, bc2, HP['weight_decay'], 1)
+    torch.cuda.synchronize()
+    got = host_rows([tuple(t[o:o + n] for t in moved) + (n,) for o, n in zip(offsets, sizes)])
+    check_rows(rows, got, g_bf16, 0.625, 7)
+    for buf, o in zip(raw, at):
+        assert bool((buf[:o] == 3.0).all()) and bool((buf[o + total:] == 3.0).all())
+    table.close()
 
 
 def test_adam_table_rebound_between_flat_and_separate_rows(pkg, dev):
@@ -338,8 +372,8 @@ def test_norm_heavy_tails_deterministic_and_scaling(pkg, dev):
 def test_norm_over_many_rows(pkg, dev, nrows, g_bf16):
     """Tables of nrows device rows around the norm kernel's LDS staging of the rows' first chunks (up to 512; more
     fall back to the search from row 0), plus zero-size rows (absent from the device table), sizes off the
-    256-element chunk, and the same rows as views of one buffer at odd offsets (BF16: not 8-byte aligned, the
-    element-wise path): within 1 ulp of the exact norm, bit-identical on a second run."""
+    256-element chunk, and the same rows as views of one buffer at odd offsets: within 1 ulp of the exact norm,
+    bit-identical on a second run."""
     from faster_yoco_amd import ops
     rng = np.random.default_rng(nrows + 7 * g_bf16)
     sizes = rng.integers(1, 1200, nrows)                 # nrows device rows
@@ -484,17 +518,16 @@ MISALIGNED = {
     'lines_shared_134B': (67, (67, 67, 67, 67), 67),  # 6 bytes into the second line of each
     'lines_apart_by_128B': (5, (69, 5, 133, 5), None),
     'words_shared': (1, (5, 1, 9, 13), None),          # same offset within 8-byte words only
-    'no_common_word': (1, (2, 1, 1, 1), None),         # element-wise path
-    'fp32_sum_off_grid': (1, (1, 1, 1, 1), 0),         # the fp32 sum not 16-byte aligned on the grid: element path
+    'one_stream_apart': (1, (2, 1, 1, 1), None),       # one contribution 2 bytes off the others
+    'fp32_sum_apart': (1, (1, 1, 1, 1), 0),            # the fp32 sum off the average's element grid
 }
 
 
 @pytest.mark.parametrize('case', sorted(MISALIGNED))
 def test_owner_sum_misaligned_ranges(pkg, dev, case):
     """Streams that start off the 16-byte boundaries -- a CEReduce phase starts at any parameter boundary of the
-    owner's gradient: the chunk grid follows the offset the streams share (a 128-byte line offset, else an 8-byte
-    word offset, else the element-wise path); the average and the fp32 sum stay bit-exact, the fused norm within
-    1e-6 of the exact one."""
+    owner's gradient: the chunk grid follows the average's offset in a 128-byte line, and the other streams are loaded
+    wherever they lie; the average and the fp32 sum stay bit-exact, the fused norm within 1e-6 of the exact one."""
     from faster_yoco_amd import ops
     oo, co, so = MISALIGNED[case]
     rng = np.random.default_rng(len(case))
