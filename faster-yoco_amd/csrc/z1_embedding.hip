@@ -42,7 +42,7 @@ constexpr int64_t kSortMinRows = 3073;
 constexpr int kFewRowsChunk = 16;
 constexpr int kWave = 64;
 // The rows launch.  Figures: whole calls on 16,384 rows of 3072 into a 100,288-row table, gradients not cached, uniform /
-// Zipf(1.2) ids; 141 / 152 us as it stands.
+// Zipf(1.2) ids; 143 / 154 us as it stands, 141 / 152 when they were taken.
 // Resident workgroups per CU, capped with a dynamic LDS reservation the kernel does not use: 141 / 153 at 14, 143 / 152 at
 // 20, 152 / 157 at 10, 175 / 185 at 8 (a short table, 2000 rows of 768 into 32,000: 32.4 us at 20, 33.9 at 14, 37 at 10).
 constexpr int kEmbWgPerCu = 16;
