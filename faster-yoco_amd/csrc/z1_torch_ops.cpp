@@ -19,6 +19,7 @@
  * yoco/models/decoder/ce_reduce.py:182) and the torch scalar ops of the norm and clip chain
  * (yoco/tasks/zero1_fast.py:150-160, yoco/tasks/trainer_nosync.py:273-286).
  */
+#include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/core/Tensor.h>
 #include <ATen/ops/empty.h>
 #include <ATen/record_function.h>
@@ -835,9 +836,10 @@ int z1t_table_register(z1_table* table, int device, int g_dtype, int has_pmv, in
 }
 
 /* Whether anything on this thread would see a profiler region: a RecordFunction observer (profilers, execution traces; of
- * this thread or of all), a dispatch mode, or a trace being recorded. */
+ * this thread or of all), a dispatch mode, a function mode, or a trace being recorded. */
 int z1t_observed() {
-    return at::hasCallbacks() || c10::impl::TorchDispatchModeTLS::any_modes_set() || torch::jit::tracer::isTracing();
+    return at::hasCallbacks() || c10::impl::TorchDispatchModeTLS::any_modes_set() ||
+           at::impl::PythonTorchFunctionTLS::stack_len() > 0 || torch::jit::tracer::isTracing();
 }
 
 /* Forgets a table (before z1_table_destroy). */

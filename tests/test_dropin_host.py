@@ -177,3 +177,28 @@ def test_profiler_regions_reach_every_observer(pkg, tmp_path):
 
     assert seen(shard.region) == seen(record_function)
     assert type(shard.region('clip-grads')) is not record_function
+
+
+def test_profiler_regions_reach_a_function_mode(pkg):
+    """shard.region under a torch function mode without any profiler: the calls record_function makes."""
+    from torch.autograd.profiler import record_function
+    from torch.overrides import TorchFunctionMode
+    from faster_yoco_amd import shard
+
+    class Seen(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            names.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    def calls(make):
+        names.clear()
+        with Seen():
+            with make('clip-grads'):
+                torch.ones(2)
+        return list(names)
+
+    names = []
+    expected = calls(record_function)
+    assert any('_record_function_enter' in n for n in expected)
+    assert calls(shard.region) == expected
+    assert type(shard.region('clip-grads')) is not record_function
