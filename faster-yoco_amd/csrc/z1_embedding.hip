@@ -126,21 +126,39 @@ __device__ __forceinline__ int2 key_range(const uint32_t* __restrict__ sorted, i
     return int2{lo, hi};
 }
 
-__global__ void emb_row_ranges_kernel(const uint32_t* __restrict__ sorted, const int32_t* __restrict__ spos, int64_t R,
-                                      int64_t V, int2* __restrict__ info, int* __restrict__ counts) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < 2) counts[t] = 0;                   // the rows kernel appends to the chain pass's lists after this kernel
-    if (t >= V) return;
-    const int2 r = key_range(sorted, R, (uint32_t)t);
-    const int32_t lo = r.x, hi = r.y;
-    info[t] = int2{hi - lo == 1 ? spos[lo] : lo, hi - lo};
-    if (t == V - 1) counts[2] = hi;             // the ids inside [0, V)
+// info, and ent of every sorted place: the first `vocab_blocks` workgroups have a thread per id, the others (up to
+// kSearchRows indices) one per place, which searches for its own id's range rather than wait for info in a launch of its
+// own.  Whole calls, two launches / one: 50,000 indices of width 64 into 8000 rows 63.1 / 61.1 us, 100,000 87.0 / 85.0,
+// 200,000 of 768 into 32,000 rows 149.9 / 149.3; 262,144 are even, and 500,000 of 256 take 256.6 / 262.5, 1.2M of 64 into
+// 8000 rows 318 / 326: a search per place then costs more than a launch.
+constexpr int64_t kSearchRows = 1 << 18;
+constexpr int kPlaceThreads = 256;
+__global__ __launch_bounds__(kPlaceThreads) void emb_places_kernel(const uint32_t* __restrict__ sorted,
+                                                                   const int32_t* __restrict__ spos, int64_t R, int64_t V,
+                                                                   int vocab_blocks, int2* __restrict__ info,
+                                                                   Ent* __restrict__ ent, int* __restrict__ counts) {
+    if (blockIdx.x == 0 && threadIdx.x < 2) counts[threadIdx.x] = 0;   // the rows kernel appends to the lists after this
+    if ((int)blockIdx.x < vocab_blocks) {
+        const int64_t t = (int64_t)blockIdx.x * kPlaceThreads + threadIdx.x;
+        if (t >= V) return;
+        const int2 r = key_range(sorted, R, (uint32_t)t);
+        info[t] = int2{r.y - r.x == 1 ? spos[r.x] : r.x, r.y - r.x};
+        if (t == V - 1) counts[2] = r.y;        // the ids inside [0, V)
+        return;
+    }
+    const int64_t p = (int64_t)((int)blockIdx.x - vocab_blocks) * kPlaceThreads + threadIdx.x;
+    if (p >= R) return;
+    const uint32_t id = sorted[p];
+    if ((int64_t)id >= V) return;
+    const int2 r = key_range(sorted, R, id);
+    ent[p] = Ent{spos[p], id, r.x, r.y - r.x};
 }
 
-// ent of every sorted place.
-__global__ void emb_entries_kernel(const uint32_t* __restrict__ sorted, const int32_t* __restrict__ spos, int64_t R,
-                                   int64_t V, const int2* __restrict__ info, Ent* __restrict__ ent) {
-    const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+// ent of every sorted place, from info.
+__global__ __launch_bounds__(kPlaceThreads) void emb_entries_kernel(const uint32_t* __restrict__ sorted,
+                                                                    const int32_t* __restrict__ spos, int64_t R, int64_t V,
+                                                                    const int2* __restrict__ info, Ent* __restrict__ ent) {
+    const int64_t p = (int64_t)blockIdx.x * kPlaceThreads + threadIdx.x;
     if (p >= R) return;
     const uint32_t id = sorted[p];
     if ((int64_t)id >= V) return;
@@ -904,12 +922,15 @@ int z1_embedding_backward(const int64_t* ids, const uint16_t* grad, int64_t R, i
             e = sort_pairs(w.temp, tb, w.keys, w.skeys, w.vals, w.svals, R, end_bit, capturing(st), st);
             if (e != hipSuccess) return (int)e;
         }
-        hipLaunchKernelGGL(emb_row_ranges_kernel, dim3((unsigned)((V + 255) / 256)), dim3(256), 0, st, w.skeys, w.svals,
-                           R, V, w.info, w.counts);
+        const int64_t vocab_blocks = (V + kPlaceThreads - 1) / kPlaceThreads, blocks = (R + kPlaceThreads - 1) / kPlaceThreads;
+        const bool search = R <= kSearchRows;
+        hipLaunchKernelGGL(emb_places_kernel, dim3((unsigned)(vocab_blocks + (search ? blocks : 0))), dim3(kPlaceThreads), 0,
+                           st, w.skeys, w.svals, R, V, (int)vocab_blocks, w.info, w.ent, w.counts);
         e = hipGetLastError();
         if (e != hipSuccess) return (int)e;
-        if (R > 0)
-            hipLaunchKernelGGL(emb_entries_kernel, per_row, dim3(256), 0, st, w.skeys, w.svals, R, V, w.info, w.ent);
+        if (!search)
+            hipLaunchKernelGGL(emb_entries_kernel, dim3((unsigned)blocks), dim3(kPlaceThreads), 0, st, w.skeys, w.svals, R, V,
+                               w.info, w.ent);
     }
     e = hipGetLastError();
     if (e != hipSuccess) return (int)e;
