@@ -45,6 +45,9 @@ constexpr int kWave = 64;
 // Zipf(1.2) ids; 143 / 154 us as it stands, 141 / 152 when they were taken.
 // Resident workgroups per CU, capped with a dynamic LDS reservation the kernel does not use: 141 / 153 at 14, 143 / 152 at
 // 20, 152 / 157 at 10, 175 / 185 at 8 (a short table, 2000 rows of 768 into 32,000: 32.4 us at 20, 33.9 at 14, 37 at 10).
+// Dense tables (below) run as many as fit: they read more than they write, in waves that sum up to 20 rows.  At 16 / all:
+// 100,000 of 768 into 32,000 rows 117.9 / 108.0 and 157.8 / 148.6, 50,000 of 768 into 256 88.7 / 81.5 and 104.5 / 98.4, 1.2M
+// of 768 into 32,000 879 / 813 and 1033 / 976, 50,000 of 64 into 8000 61.0 / 59.4 and 88.4 / 90.0.
 constexpr int kEmbWgPerCu = 16;
 constexpr int kDirect = 4;                 // most occurrences of an id that the wave of its row sums (2: the same)
 // In a dense table, of kDenseMean indices per row or more on average, the wave of a row sums up to kDirectDense occurrences
@@ -58,10 +61,13 @@ constexpr int kDirectDense = 2 * kRowsPerPartial;
 constexpr int64_t kDenseMean = 2;
 constexpr int64_t kDenseRows = 16384;
 constexpr int kRunBlock = 40;              // sorted positions whose runs a wave sums, for one step of 512 columns
-// In a dense table of this many indices per row or more most ids are summed by runs, and half the block gives twice the
-// waves: 65,536 ids of width 256 into 256 rows, uniform / Zipf, 78.5 / 107.4 us with 40, 72.1 / 101.8 with 20; 131,072 of 768
-// into 1000 rows 152 / 195 and 147 / 187.  At 8 per row it loses (262,144 of 768 into 32,000 rows 205 / 334 and 209 / 337).
+// In a dense table of this many indices per row or more most ids are summed by runs, and shorter blocks give more waves:
+// half the length (65,536 ids of width 256 into 256 rows, uniform / Zipf, 78.5 / 107.4 us with 40, 72.1 / 101.8 with 20;
+// 131,072 of 768 into 1000 rows 152 / 195 and 147 / 187; at 8 per row it loses: 262,144 of 768 into 32,000 rows 205 / 334 and
+// 209 / 337), and a quarter where a half gives at most kQuarterWaves waves: 20,000 of 256 into 256 rows 37.4 / 48.6 and
+// 34.3 / 45.6, 100,000 of 64 (5000 waves) 85.8 / 122.1 and 83.8 / 119.6, but 20,000 of 3072 (6000) 64.6 / 75.7 and 66.9 / 83.2.
 constexpr int64_t kShortBlockMean = 16;
+constexpr int64_t kQuarterWaves = 5120;
 constexpr int kFewBlock = 8;               // the same, few indices
 constexpr int kMaxWaves = 1 << 20;         // most waves that sum runs (they stride beyond that)
 // Consecutive rows of one XCD: spans of 32 to 128 rows measure alike, single rows round robin 144 / 153; one eighth of the
@@ -390,8 +396,8 @@ typedef f4 f4_any __attribute__((aligned(4)));
 // is its row; otherwise the fp32 partial goes to the run's slot, and the wave of step 0 lists the id for the chain pass.
 template <bool FEW, int DIRECT>
 __device__ __forceinline__ void sum_runs(int64_t p0, int block, int step, bool last_step,
-                                         const uint16_t* __restrict__ grad, int64_t D, const Ent* __restrict__ ent, int64_t padding_idx, float scale, int scale_mode,
-                                         int64_t valid, uint16_t* __restrict__ out, int* __restrict__ counts,
+                                         const uint16_t* __restrict__ grad, int64_t D, const Ent* __restrict__ ent,
+                                         int64_t padding_idx, float scale, int scale_mode, int64_t valid, uint16_t* __restrict__ out, int* __restrict__ counts,
                                          int32_t* __restrict__ short_list, int32_t* __restrict__ long_list,
                                          float* __restrict__ parts) {
     constexpr int kRows = FEW ? kFewRowsChunk : kRowsPerPartial;
@@ -860,7 +866,8 @@ void launch_rows_g(const RowsCall& c, const EmbWorkspace& w) {
     int64_t run_waves = 0;
     int block = FEW ? kFewBlock : kRunBlock;
     if (c.R > kDirect) {
-        if (DENSE && c.R >= kShortBlockMean * c.V) block = kRunBlock / 2;
+        if (DENSE && c.R >= kShortBlockMean * c.V)
+            block = c.R * step_waves <= kQuarterWaves * (kRunBlock / 2) ? kRunBlock / 4 : kRunBlock / 2;
         const int64_t blocks = (c.R + block - 1) / block, most = kMaxWaves / step_waves;      // steps <= 32,768
         run_waves = ((blocks < most ? blocks : most) + 7) / 8 * 8 * step_waves;
     }
@@ -938,12 +945,15 @@ int z1_embedding_backward(const int64_t* ids, const uint16_t* grad, int64_t R, i
     e = hipGetDevice(&dev);
     if (e != hipSuccess) return (int)e;
     RowsCall c{grad, R, D, V, padding_idx, scale, scale_mode, out, 0, st};
-    const int rc = z1detail::occupancy_lds(dev, kEmbWgPerCu, &c.lds);
-    if (rc) return rc;
     const bool few = R < kSortMinRows;                  // aten's kernel for few indices: its order
-    if (few) launch_rows<true>(c, w);
-    else if (dense(R, V)) launch_rows_g<false, 1, true>(c, w);
-    else launch_rows<false>(c, w);
+    if (dense(R, V)) {
+        launch_rows_g<false, 1, true>(c, w);
+    } else {
+        const int rc = z1detail::occupancy_lds(dev, kEmbWgPerCu, &c.lds);
+        if (rc) return rc;
+        if (few) launch_rows<true>(c, w);
+        else launch_rows<false>(c, w);
+    }
     e = hipGetLastError();
     if (e != hipSuccess) return (int)e;
     // the most items the lists can hold
