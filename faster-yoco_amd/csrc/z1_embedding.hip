@@ -397,7 +397,8 @@ typedef f4 f4_any __attribute__((aligned(4)));
 template <bool FEW, int DIRECT>
 __device__ __forceinline__ void sum_runs(int64_t p0, int block, int step, bool last_step,
                                          const uint16_t* __restrict__ grad, int64_t D, const Ent* __restrict__ ent,
-                                         int64_t padding_idx, float scale, int scale_mode, int64_t valid, uint16_t* __restrict__ out, int* __restrict__ counts,
+                                         int64_t padding_idx, float scale, int scale_mode, int64_t valid,
+                                         uint16_t* __restrict__ out, int* __restrict__ counts,
                                          int32_t* __restrict__ short_list, int32_t* __restrict__ long_list,
                                          float* __restrict__ parts) {
     constexpr int kRows = FEW ? kFewRowsChunk : kRowsPerPartial;
@@ -628,10 +629,20 @@ __global__ __launch_bounds__(kEmbThreads) void emb_rows_kernel(const uint16_t* _
     }
 }
 
-// The sum of n partials of one column in LDS rows 0 .. n - 1, added in order to acc, 16 reads in flight.
+// The sum of n partials of one column in LDS rows 0 .. n - 1, added in order to acc, 16 reads in flight.  The adds of a
+// whole 16 follow each other at their own latency; with a choice after each the chain launch of 65,536 Zipf ids of width
+// 256 into 256 rows took 28.2 us, without 21.2 (50,000 of 64 into 8000 rows 21.6 / 16.4, few indices 15.4 / 14.0).
 template <bool FEW>
 __device__ __forceinline__ float chain_rows(float acc, const float (*buf)[kWave], int n, int lane) {
-    for (int k0 = 0; k0 < n; k0 += 16) {
+    int k0 = 0;
+    for (; k0 + 16 <= n; k0 += 16) {
+        float y[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) y[i] = buf[k0 + i][lane];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc = add_part<FEW>(acc, y[i]);
+    }
+    if (k0 < n) {
         float y[16];
 #pragma unroll
         for (int i = 0; i < 16; ++i) y[i] = buf[k0 + i][lane];
