@@ -92,12 +92,20 @@ struct Row {
     int64_t chunk0;
     // Pointers off their elements' boundaries, which no tensor has but a C caller's row may, take the element loops of the
     // rows' last chunks throughout.
-    int32_t vec;        // bit 0: g on its element boundary; bit 1: p, m, v, p16 as well
-    int32_t pmv_aligned;    // p, m, v, p16 on their element boundaries (vec's bit 1 needs g there too)
+    int32_t vec;        // kVecG: g on its element boundary; with it pmv_vec's bits, else 0
+    int32_t pmv_vec;    // pmv_bits of p, m, v, p16
 };
 static_assert(sizeof(Row) == 64, "row layout");
 
-enum { kVecG = 1, kVecAll = 2 };
+enum { kVecG = 1, kVecAll = 2, kCopyWord = 4 };
+
+// kVecAll: p, m, v, p16 on their element boundaries; kCopyWord: there is a p16, and it is on a dword too.
+__host__ __device__ inline int32_t pmv_bits(const float* p, const float* m, const float* v, const uint16_t* p16) {
+    const uintptr_t h = reinterpret_cast<uintptr_t>(p16);
+    if (((reinterpret_cast<uintptr_t>(p) | reinterpret_cast<uintptr_t>(m) | reinterpret_cast<uintptr_t>(v)) & 3) || (h & 1))
+        return 0;
+    return kVecAll | (h && !(h & 3) ? kCopyWord : 0);
+}
 
 struct AdamK {
     float lr, b1, b2, eps, bc1, bc2, wd, omb1, omb2;
@@ -152,15 +160,12 @@ __device__ __forceinline__ void st_stream(uint16_t* base, int bytes, int off, u2
     const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(base, 0, bytes, 0x00020000);
     __builtin_amdgcn_raw_buffer_store_b64(x, r, off, 0, kStreamStorePolicy);
 }
-// Four bf16 anywhere: buffer stores want dword addresses, so at an odd element they go out as a nontemporal global store.
-// The choice costs where stores are all a wave does beside one round of loads (the cast pass over 120M elements 108.4 us
-// without it, 111.2 with; the sum of two contributions 198.0 / 201.1): those kernels take st_stream.
-__device__ __forceinline__ void st_stream_any(uint16_t* base, int bytes, int off, u2 x) {
-    if (reinterpret_cast<uintptr_t>(base) & 3)
-        __builtin_nontemporal_store((AnyAlign<u2>::type)x,
-                                    (Z1_GLOBAL AnyAlign<u2>::type*)(reinterpret_cast<char*>(base) + off));
-    else
-        st_stream(base, bytes, off, x);
+// Four bf16 at an odd element: buffer stores want dword addresses, so they go out as a nontemporal global store.  No kernel
+// looks at the address to choose: the choice costs where stores are all a wave does beside one round of loads (the cast
+// pass over 120M elements 108.4 us without it, 111.2 with; the sum of two contributions 198.0 / 201.1; Adam over 134M
+// elements in 15 rows with BF16 gradients 548 / 552).
+__device__ __forceinline__ void st_odd(uint16_t* p, u2 x) {
+    __builtin_nontemporal_store((AnyAlign<u2>::type)x, (Z1_GLOBAL AnyAlign<u2>::type*)p);
 }
 
 // Chunk of workgroup b: undoes the round-robin dispatch over the 8 XCDs (workgroup b runs on XCD b mod 8), so that
@@ -267,7 +272,8 @@ __device__ __forceinline__ void adam_chunk(const Row& r, float* go, int64_t base
             st_stream(r.v + base, (int)kChunk * 4, o4, v[u]);
             if (r.p16) {
                 const u2 h = u2{pack_bf16(p[u][0], p[u][1]), pack_bf16(p[u][2], p[u][3])};
-                st_stream_any(r.p16 + base, (int)kChunk * 2, o2, h);
+                if (r.vec & kCopyWord) st_stream(r.p16 + base, (int)kChunk * 2, o2, h);
+                else st_odd(r.p16 + base + o2 / 2, h);
             }
             if (GOUT && go) st_stream(go + base, (int)kChunk * 4, o4, g[u]);
         }
@@ -847,7 +853,7 @@ __global__ __launch_bounds__(kBindPerLaunch) void set_grads_kernel(Row* rows, Gr
     Row* r = rows + b.row[i];
     const bool ga = (reinterpret_cast<uintptr_t>(b.g[i]) & (uintptr_t)(b.g_align - 1)) == 0;
     r->g = b.g[i];
-    r->vec = ga ? (kVecG | (r->pmv_aligned ? kVecAll : 0)) : 0;
+    r->vec = ga ? kVecG | r->pmv_vec : 0;
 }
 
 // FP32 gradient outputs of up to kBindPerLaunch rows (z1_table_set_grad_out), passed by value like the gradients.
@@ -874,17 +880,14 @@ __global__ __launch_bounds__(kRebindPerLaunch) void rebind_rows_kernel(Row* rows
     const int i = threadIdx.x;
     if (i >= b.count) return;
     Row* r = rows + b.row[i];
-    const uintptr_t pmv = reinterpret_cast<uintptr_t>(b.p[i]) | reinterpret_cast<uintptr_t>(b.m[i]) |
-                          reinterpret_cast<uintptr_t>(b.v[i]);
-    const bool pmv_ok = (pmv & 3) == 0 && (reinterpret_cast<uintptr_t>(b.p16[i]) & 1) == 0;
     const bool ga = (reinterpret_cast<uintptr_t>(b.g[i]) & (uintptr_t)(b.g_align - 1)) == 0;
     r->g = b.g[i];
     r->p = b.p[i];
     r->m = b.m[i];
     r->v = b.v[i];
     r->p16 = b.p16[i];
-    r->pmv_aligned = pmv_ok;
-    r->vec = ga ? (kVecG | (pmv_ok ? kVecAll : 0)) : 0;
+    r->pmv_vec = pmv_bits(b.p[i], b.m[i], b.v[i], b.p16[i]);
+    r->vec = ga ? kVecG | r->pmv_vec : 0;
 }
 
 // ------------------------------------------------------------------------------------- scale / cast passes
@@ -926,7 +929,7 @@ __global__ __launch_bounds__(kWave) void cast_bf16_kernel(const float* __restric
         for (int u = 0; u < 2; ++u) {
             const int off = (int)((u * (kPassChunk / 2) + lane * 4) * 2);
             const u2 h = u2{pack_bf16(a[u].x, a[u].y), pack_bf16(a[u].z, a[u].w)};
-            if (ODD) st_stream_any(p16 + e0, (int)kPassChunk * 2, off, h);
+            if (ODD) st_odd(p16 + e0 + off / 2, h);
             else st_stream(p16 + e0, (int)kPassChunk * 2, off, h);
         }
         return;
@@ -1051,7 +1054,8 @@ static void set_contig(z1_table* t) {
     const uintptr_t g0 = reinterpret_cast<uintptr_t>(r0.g), p0 = reinterpret_cast<uintptr_t>(r0.p),
                     m0 = reinterpret_cast<uintptr_t>(r0.m), v0 = reinterpret_cast<uintptr_t>(r0.v),
                     h0 = reinterpret_cast<uintptr_t>(r0.p16);
-    if ((g0 & (gsz - 1)) || ((p0 | m0 | v0) & 3) || (h0 & 1)) return;
+    const int32_t pmv = pmv_bits(r0.p, r0.m, r0.v, r0.p16);
+    if ((g0 & (gsz - 1)) || !(pmv & kVecAll)) return;
     uintptr_t off = 0;                                 // elements before row i
     for (const Row& r : h) {
         if ((r.p16 != nullptr) != with16) return;
@@ -1064,8 +1068,8 @@ static void set_contig(z1_table* t) {
     t->whole = r0;
     t->whole.n = (int64_t)off;
     t->whole.chunk0 = 0;
-    t->whole.pmv_aligned = 1;
-    t->whole.vec = kVecG | kVecAll;
+    t->whole.pmv_vec = pmv;
+    t->whole.vec = kVecG | pmv;
     t->contig = 1;
 }
 
@@ -1110,8 +1114,8 @@ static int table_create(const z1_tensor* rows, int nrows, int g_dtype, z1_table*
         r.p16 = t.p16;
         r.n = t.n;
         r.chunk0 = chunks;
-        r.pmv_aligned = aligned(t.p, 4) && aligned(t.m, 4) && aligned(t.v, 4) && (!t.p16 || aligned(t.p16, 2));
-        r.vec = aligned(t.g, galign) ? (kVecG | (r.pmv_aligned ? kVecAll : 0)) : 0;
+        r.pmv_vec = pmv_bits(r.p, r.m, r.v, r.p16);
+        r.vec = aligned(t.g, galign) ? kVecG | r.pmv_vec : 0;
         if (!t.p || !t.m || !t.v) has_pmv = 0;
         chunks += (t.n + kChunk - 1) / kChunk;
         numel += t.n;

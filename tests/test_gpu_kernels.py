@@ -251,6 +251,33 @@ def test_adam_table_rebound_between_flat_and_separate_rows(pkg, dev):
     table.close()
 
 
+def test_adam_table_rebound_between_copies_at_any_element(pkg, dev):
+    """One table whose BF16 copies lie in turn on dwords, at odd elements, at odd ones with the gradients moved alone, and on
+    dwords again: how a row's copy is stored follows each binding.  Bit-exact against the oracle, nothing written beside
+    the copies."""
+    from faster_yoco_amd import ops
+    sizes = [3000, 1, 4096 + 17, 513]
+    rows = [rand_state(n, 900 + i) for i, n in enumerate(sizes)]
+    _, views = flat_rows(rows, False, dev, with_p16=False)
+    moved = [dev_f32(r[0], dev) for r in rows]
+    raw = [[torch.full((n + 4,), 3.0, dtype=torch.bfloat16, device=dev) for n in sizes] for _ in range(2)]
+    table, want = None, rows
+    bc1, bc2 = ops.bias_corrections(HP['beta1'], HP['beta2'], 3)
+    for off, grads in ((2, None), (1, None), (1, moved), (2, moved)):
+        bound = [(v[0] if grads is None else grads[i], v[1], v[2], v[3], raw[off - 1][i][off:off + v[5]], v[5])
+                 for i, v in enumerate(views)]
+        table = table or ops.Table(bound, dev)
+        ops.adam_cast(table, None, HP['lr'], HP['beta1'], HP['beta2'], HP['eps'], bc1, bc2, HP['weight_decay'], 1,
+                      tensors=ops.rows_lists(bound))
+        torch.cuda.synchronize()
+        got = host_rows(bound)
+        check_rows(want, got, False, None, 3)
+        for t, n in zip(raw[off - 1], sizes):
+            assert bool((t[:off] == 3.0).all()) and bool((t[off + n:] == 3.0).all())
+        want = [(g, gp, gm, gv) for (g, _, _, _), (gp, gm, gv, _) in zip(rows, got)]
+    table.close()
+
+
 def test_adam_flat_rows_with_gradients_moved_apart(pkg, dev):
     """A table over views of flat buffers whose gradients are then given as separate allocations (the operators
     rebind only the gradient column, as when autograd reallocates gradients): the rows are no longer one allocation
