@@ -12,7 +12,7 @@
 //      id t are and how many: for up to kBucketRows rows one launch, emb_bucket_kernel; beyond, keys[i] = id_i (or V when
 //      out of range) and vals[i] = i sorted stably by key -- hipCUB's radix sort, or, while the stream is being captured
 //      into a HIP graph, rocPRIM's merge sort, which clears nothing with memsets (the radix sort does; both are stable,
-//      so the order is the same) -- one binary search per t over the sorted keys, and one pass that makes ent of them;
+//      so the order is the same) -- and binary searches over the sorted keys, one per t and one per place;
 //   2. emb_rows_kernel writes every row of the table exactly once (aten zero-fills the whole table and then scatters
 //      into it): first waves for the runs of ids with many occurrences, then one wave per row, in order, which zeroes
 //      it or sums its few occurrences.  Token frequencies in text are skewed: one wave (or one workgroup) walking
@@ -42,7 +42,7 @@ constexpr int64_t kSortMinRows = 3073;
 constexpr int kFewRowsChunk = 16;
 constexpr int kWave = 64;
 // The rows launch.  Figures: whole calls on 16,384 rows of 3072 into a 100,288-row table, gradients not cached, uniform /
-// Zipf(1.2) ids; 143 / 154 us as it stands, 141 / 152 when they were taken.
+// Zipf(1.2) ids; 141 / 153 us as it stands, 141 / 152 when they were taken.
 // Resident workgroups per CU, capped with a dynamic LDS reservation the kernel does not use: 141 / 153 at 14, 143 / 152 at
 // 20, 152 / 157 at 10, 175 / 185 at 8 (a short table, 2000 rows of 768 into 32,000: 32.4 us at 20, 33.9 at 14, 37 at 10).
 // Dense tables (below) run as many as fit: they read more than they write, in waves that sum up to 20 rows.  At 16 / all:
@@ -53,7 +53,7 @@ constexpr int kDirect = 4;                 // most occurrences of an id that the
 // In a dense table, of kDenseMean indices per row or more on average, the wave of a row sums up to kDirectDense occurrences
 // (two runs): most ids have between 5 and 20 there, and the row waves alone fill the chip, so that partials sent through
 // memory only add traffic.  Whole calls, gradients not cached, run by run / by the row's wave (us, uniform and Zipf(1.2)
-// ids): 1.2M indices of width 768 into 100,288 rows 1376 / 557 and 1160 / 1139; 256,000 of 768 into 32,000 rows 305 / 204
+// ids, both at kEmbWgPerCu): 1.2M indices of width 768 into 100,288 rows 1376 / 557 and 1160 / 1139; 256,000 of 768 into 32,000 rows 305 / 204
 // and 340 / 332; 64,000 of 3072 into 32,000 rows 209 / 183 and 227 / 214; 32,000 of 768 into 8000 rows 42 / 38 and 70 / 69.
 // With 1.5 indices per row 48,000 of 768 take 56 / 57 us.  Fewer indices than kDenseRows leave long waves alone on the
 // chip: 12,000 Zipf ones of 3072 into 1000 rows 49 / 53 us, 20,000 80 / 77 us.
@@ -62,9 +62,9 @@ constexpr int64_t kDenseMean = 2;
 constexpr int64_t kDenseRows = 16384;
 constexpr int kRunBlock = 40;              // sorted positions whose runs a wave sums, for one step of 512 columns
 // In a dense table of this many indices per row or more most ids are summed by runs, and shorter blocks give more waves:
-// half the length (65,536 ids of width 256 into 256 rows, uniform / Zipf, 78.5 / 107.4 us with 40, 72.1 / 101.8 with 20;
-// 131,072 of 768 into 1000 rows 152 / 195 and 147 / 187; at 8 per row it loses: 262,144 of 768 into 32,000 rows 205 / 334 and
-// 209 / 337), and a quarter where a half gives at most kQuarterWaves waves: 20,000 of 256 into 256 rows 37.4 / 48.6 and
+// half the length (at kEmbWgPerCu: 65,536 ids of width 256 into 256 rows, uniform / Zipf, 78.5 / 107.4 us with 40, 72.1 / 101.8
+// with 20; 131,072 of 768 into 1000 rows 152 / 195 and 147 / 187; at 8 per row it loses: 262,144 of 768 into 32,000 rows
+// 205 / 334 and 209 / 337), and a quarter where a half gives at most kQuarterWaves waves: 20,000 of 256 into 256 rows 37.4 / 48.6 and
 // 34.3 / 45.6, 100,000 of 64 (5000 waves) 85.8 / 122.1 and 83.8 / 119.6, but 20,000 of 3072 (6000) 64.6 / 75.7 and 66.9 / 83.2.
 constexpr int64_t kShortBlockMean = 16;
 constexpr int64_t kQuarterWaves = 5120;
