@@ -196,6 +196,27 @@ def test_order_of_occurrences(pkg, dev, R, V):
     assert np.array_equal(bits(got), bits(ref))
 
 
+@pytest.mark.parametrize('R', [262144, 262145])
+@pytest.mark.parametrize('V', [1, 255, 256, 257, 70001])
+def test_places_of_the_library_sort(pkg, dev, R, V):
+    """Either side of the largest row count whose places are found in one launch, vocabularies at the edge of a workgroup:
+    skewed ids, the last id among them, and ids outside the vocabulary.  Bit-exact against aten."""
+    from faster_yoco_amd import embedding
+    rng = np.random.default_rng(R + V)
+    ids = zipf_ids(rng, R, V, 1.3)
+    ids[rng.integers(0, R, R // 3)] = rng.integers(0, V, R // 3)
+    ids[0] = V - 1
+    g = (torch.randn(R, 24, device=dev) * 1e-2).to(torch.bfloat16)
+    ours, theirs = ids.copy(), ids.copy()
+    bad = rng.integers(1, R, R // 50)
+    ours[bad] = rng.choice([-1, V, V + 3, 2 ** 31 - 1, 2 ** 40], bad.size)
+    theirs[bad] = V
+    ref = torch.ops.aten.embedding_dense_backward(g, torch.from_numpy(theirs).to(dev), V + 1, V, False)[:V]
+    got = embedding.embedding_dense_backward(g, torch.from_numpy(ours).to(dev), V, -1)
+    torch.cuda.synchronize()
+    assert np.array_equal(bits(got), bits(ref))
+
+
 @pytest.mark.parametrize('step', [2, 256, 512, 514, 1024, 4096])
 @pytest.mark.parametrize('V', [1000, 65536, 100288, 524288])
 def test_ids_a_step_apart(pkg, dev, V, step):
