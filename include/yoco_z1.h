@@ -244,8 +244,9 @@ int z1_cast_bf16(const float* p32, uint16_t* p16, int64_t n, void* stream);
  * order, one bf16 rounding.  For R <= 3072 its kernel for few indices: chunks of 16 indices, per chunk and id an fp32
  * sum rounded to bf16 and added to the bf16 row.  Every row of
  * out is written (rows without occurrences, padding_idx and ids outside [0, V) give zeros); a NaN is 0x7fc0, as aten's
- * is.  workspace: device memory of z1_embedding_backward_workspace(R, D, V) bytes (with D <= 2^24: R x D bytes for the fp32 run partials of
- * frequent ids, 4 R x D for R <= 3072, R x 16 + V x 8 bytes, and for many rows the sort's storage).  */
+ * is.  workspace: device memory of z1_embedding_backward_workspace(R, D, V) bytes (with D <= 2^24: R x D bytes for the
+ * fp32 run partials of frequent ids, 4 R x D for R <= 3072, R x 16 + V x 8 bytes, and for many rows the sort's
+ * storage).  */
 int z1_embedding_backward(const int64_t* ids, const uint16_t* grad, int64_t R, int64_t D, int64_t V,
                           int64_t padding_idx, float scale, int scale_mode, uint16_t* out, void* workspace,
                           int64_t workspace_bytes, void* stream);
