@@ -53,19 +53,20 @@ constexpr int kDirect = 4;                 // most occurrences of an id that the
 // In a dense table, of kDenseMean indices per row or more on average, the wave of a row sums up to kDirectDense occurrences
 // (two runs): most ids have between 5 and 20 there, and the row waves alone fill the chip, so that partials sent through
 // memory only add traffic.  Whole calls, gradients not cached, run by run / by the row's wave (us, uniform and Zipf(1.2)
-// ids, both at kEmbWgPerCu): 1.2M indices of width 768 into 100,288 rows 1376 / 557 and 1160 / 1139; 256,000 of 768 into 32,000 rows 305 / 204
-// and 340 / 332; 64,000 of 3072 into 32,000 rows 209 / 183 and 227 / 214; 32,000 of 768 into 8000 rows 42 / 38 and 70 / 69.
-// With 1.5 indices per row 48,000 of 768 take 56 / 57 us.  Fewer indices than kDenseRows leave long waves alone on the
-// chip: 12,000 Zipf ones of 3072 into 1000 rows 49 / 53 us, 20,000 80 / 77 us.
+// ids, both at kEmbWgPerCu): 1.2M indices of width 768 into 100,288 rows 1376 / 557 and 1160 / 1139; 256,000 of 768 into
+// 32,000 rows 305 / 204 and 340 / 332; 64,000 of 3072 into 32,000 rows 209 / 183 and 227 / 214; 32,000 of 768 into 8000 rows
+// 42 / 38 and 70 / 69. With 1.5 indices per row 48,000 of 768 take 56 / 57 us.  Fewer indices than kDenseRows leave long
+// waves alone on the chip: 12,000 Zipf ones of 3072 into 1000 rows 49 / 53 us, 20,000 80 / 77 us.
 constexpr int kDirectDense = 2 * kRowsPerPartial;
 constexpr int64_t kDenseMean = 2;
 constexpr int64_t kDenseRows = 16384;
 constexpr int kRunBlock = 40;              // sorted positions whose runs a wave sums, for one step of 512 columns
 // In a dense table of this many indices per row or more most ids are summed by runs, and shorter blocks give more waves:
-// half the length (at kEmbWgPerCu: 65,536 ids of width 256 into 256 rows, uniform / Zipf, 78.5 / 107.4 us with 40, 72.1 / 101.8
-// with 20; 131,072 of 768 into 1000 rows 152 / 195 and 147 / 187; at 8 per row it loses: 262,144 of 768 into 32,000 rows
-// 205 / 334 and 209 / 337), and a quarter where a half gives at most kQuarterWaves waves: 20,000 of 256 into 256 rows 37.4 / 48.6 and
-// 34.3 / 45.6, 100,000 of 64 (5000 waves) 85.8 / 122.1 and 83.8 / 119.6, but 20,000 of 3072 (6000) 64.6 / 75.7 and 66.9 / 83.2.
+// half the length (at kEmbWgPerCu: 65,536 ids of width 256 into 256 rows, uniform / Zipf, 78.5 / 107.4 us with 40, 72.1 /
+// 101.8 with 20; 131,072 of 768 into 1000 rows 152 / 195 and 147 / 187; at 8 per row it loses: 262,144 of 768 into 32,000
+// rows 205 / 334 and 209 / 337), and a quarter where a half gives at most kQuarterWaves waves: 20,000 of 256 into 256 rows
+// 37.4 / 48.6 and 34.3 / 45.6, 100,000 of 64 (5000 waves) 85.8 / 122.1 and 83.8 / 119.6, but 20,000 of 3072 (6000) 64.6 /
+// 75.7 and 66.9 / 83.2.
 constexpr int64_t kShortBlockMean = 16;
 constexpr int64_t kQuarterWaves = 5120;
 constexpr int kFewBlock = 8;               // the same, few indices
@@ -598,8 +599,9 @@ __global__ __launch_bounds__(kEmbThreads) void emb_rows_kernel(const uint16_t* _
         const int step = b % steps, run_block = DENSE ? block : FEW ? kFewBlock : kRunBlock;
         const int64_t valid = counts[2];
         for (int64_t p0 = (int64_t)(b / steps) * run_block; p0 < valid; p0 += (int64_t)(run_waves / steps) * run_block)
-            sum_runs<FEW, DENSE ? kDirectDense : kDirect>(p0, run_block, step, step == steps - 1, grad, D, ent, padding_idx, scale,
-                                                          scale_mode, valid, out, counts, short_list, long_list, parts);
+            sum_runs<FEW, DENSE ? kDirectDense : kDirect>(p0, run_block, step, step == steps - 1, grad, D, ent, padding_idx,
+                                                          scale, scale_mode, valid, out, counts, short_list, long_list,
+                                                          parts);
         return;
     }
     // Row of workgroup b (run_waves is a multiple of 8: workgroup b runs on XCD b mod 8): each XCD takes kSpan consecutive
